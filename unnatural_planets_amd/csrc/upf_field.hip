@@ -12,6 +12,7 @@
 #include "upf_device_grad.hpp"
 #include "upf_device_row.hpp"
 #include "upf_device_row_grad.hpp"
+#include "upf_device_tilex.hpp"
 #include "upf_internal.hpp"
 
 namespace upf {
@@ -103,6 +104,50 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
 #pragma unroll
     for (int r = 0; r < R; r++)
       if (r < rows) write_signs(S, g, blockIdx.x, j + r, k, valid, v[r], iso);
+  }
+}
+
+// The elevation modes and the further shapes, in the exact form (upf_device_tilex.hpp): a
+// workgroup covers 64 x nodes of kTY rows and kTZ planes, its four waves 16 nodes each.
+// A wave's 16 bits of each row's sign word are stored by themselves.
+//
+// VALU-bound.  500^3 lakes field, VALU instructions per 64 nodes and time of the land mesh
+// call: per lane 2,198, 5.75 ms; 64 x 2 nodes a wave with x columns 1,150, 3.77 ms; tiles of
+// 16 x 4 x 2 1,000, 3.23 ms; of 16 x 4 x 4 867, 2.95 ms at six waves per SIMD and 2.87 ms at
+// seven (72 VGPRs from 80; the few spilled are around the rare per-lane calls).
+template <int R, bool PRIM, bool HILLS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PRIM ? 7 : 4))) void k_eval_grid_tilex(const DSpec s, const DGrid g, float* __restrict__ out,
+                                                         uint16_t* __restrict__ S, float iso) {
+  __shared__ float4 s_lds[4][kTLds];
+  __shared__ float4 s_gtab[16];
+  if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i0 = blockIdx.x * 64 + wv * kTX, k0 = blockIdx.z * R;
+  const int i = i0 + (lane & (kTX - 1)), j = blockIdx.y * kTY + lane / kTX;
+  float v[R] = {};
+  if (i0 < g.n[0]) {  // lanes past the end of a row or plane stand in for the last node
+    const float x = node_coord(g.o[0], g.s[0], min(i, g.n[0] - 1));
+    const float y = node_coord(g.o[1], g.s[1], min(j, g.n[1] - 1));
+    float z[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) z[r] = node_coord(g.o[2], g.s[2], min(k0 + r, g.n[2] - 1));
+    const TileCtx c = {s_lds[wv], s_gtab, lane};
+    tile_field<R, PRIM, HILLS>(c, s, x, y, z, v);
+  }
+  const bool valid = i < g.n[0] && j < g.n[1];
+  const int gpr = (g.n[0] + 63) / 64;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (k0 + r >= g.n[2]) break;
+    const int64_t row = (int64_t)(k0 + r) * g.n[1] + j;
+    if (valid) out[row * g.n[0] + i] = v[r];
+    if (S) {
+      const uint64_t m = __ballot(valid && v[r] < iso);
+      if ((lane & (kTX - 1)) == 0 && j < g.n[1])
+        S[(row * gpr + blockIdx.x) * 4 + wv] = (uint16_t)(m >> lane);
+    }
   }
 }
 
@@ -235,17 +280,43 @@ int adjoint_blocks(int64_t n) {
 }
 }  // namespace
 
+void lanes_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, float iso, hipStream_t stream) {
+  const dim3 blocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + kGridBY - 1) / kGridBY, g.n[2]);
+  const auto kernel = spec_ext(s) ? k_eval_grid<true> : k_eval_grid<false>;
+  hipLaunchKernelGGL(kernel, blocks, dim3(kGridBX, kGridBY, 1), 0, stream, s, g, d_field, S, iso);
+}
+
+template <int R>
+void tilex_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, float iso, hipStream_t stream) {
+  const dim3 blocks((g.n[0] + 63) / 64, (g.n[1] + kTY - 1) / kTY, (g.n[2] + R - 1) / R);
+  const bool prim = s.shape < UPF_SHAPE_H3O && !spec_composed(s);
+  const bool hills = s.mode == UPF_ELEV_LAKES || s.mode == UPF_ELEV_ISLANDS;
+  const auto kernel = prim ? (hills ? k_eval_grid_tilex<R, true, true> : k_eval_grid_tilex<R, true, false>)
+                           : (hills ? k_eval_grid_tilex<R, false, true> : k_eval_grid_tilex<R, false, false>);
+  hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, stream, s, g, d_field, reinterpret_cast<uint16_t*>(S), iso);
+}
+
+// The exact form's kernel by the number of nodes.  From 128^3 nodes four planes a wave share
+// its lattice work (400^3: lakes 2,805 us per lane, 1,185 in tiles; craters 11,142 and 1,523;
+// legacy 1,483 and 1,043).  Below, four planes leave too few waves (48^3 lakes: 14.8 us per
+// lane, 28 with four planes, 15.2 with one): one plane a wave, but per lane for the legacy
+// mode and the layer stack, most of whose layers the tiles evaluate per lane anyway (110^3
+// legacy: 39.4 us per lane, 43.7 in one-plane tiles).
+constexpr int64_t kTileNodes = (int64_t)1 << 21;
+
+void exact_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, float iso, hipStream_t stream) {
+  if ((int64_t)g.n[0] * g.n[1] * g.n[2] >= kTileNodes) tilex_launch<4>(s, g, d_field, S, iso, stream);
+  else if (s.mode == UPF_ELEV_LEGACY || s.mode == UPF_ELEV_LAYERS) lanes_launch(s, g, d_field, S, iso, stream);
+  else tilex_launch<1>(s, g, d_field, S, iso, stream);
+}
+
 int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int variant, uint64_t* S, float iso,
                       hipStream_t stream) {
   if (variant < 0 || variant > UPF_EVAL_PER_LANE) return UPF_ERR_BAD_SPEC;
-  const bool ext = spec_ext(s);
-  if (ext) variant = UPF_EVAL_PER_LANE;  // the row form covers the layer stack and the common shapes
-  const dim3 blocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + kGridBY - 1) / kGridBY, g.n[2]);
   if (variant == UPF_EVAL_PER_LANE) {
-    if (ext)
-      hipLaunchKernelGGL(k_eval_grid<true>, blocks, dim3(kGridBX, kGridBY, 1), 0, stream, s, g, d_field, S, iso);
-    else
-      hipLaunchKernelGGL(k_eval_grid<false>, blocks, dim3(kGridBX, kGridBY, 1), 0, stream, s, g, d_field, S, iso);
+    lanes_launch(s, g, d_field, S, iso, stream);
+  } else if (spec_ext(s)) {  // the row form covers the layer stack and the common shapes
+    exact_launch(s, g, d_field, S, iso, stream);
   } else {
     constexpr int rows_per_block = kRowsPerWave * kRowWaves;
     const dim3 rblocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + rows_per_block - 1) / rows_per_block, g.n[2]);

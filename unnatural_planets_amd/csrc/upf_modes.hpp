@@ -148,6 +148,14 @@ template <class T> UPF_HD bool mode_after(int mode, int l, T v, T zero, ModeStat
   return false;
 }
 
+// The lakes' and islands' masks of the ridges and the terraces, from the second layer.
+template <class T> UPF_HD T mode_ridge_mask(const ModeState<T>& st, T zero) {
+  return smoothstep1(sat_v(st.v1 * 7.0f - 0.3f, zero));
+}
+template <class T> UPF_HD T mode_terrace_mask(const ModeState<T>& st, T zero) {
+  return smoothstep1(sat_v(st.v1 * -7.0f - 1.5f, zero));
+}
+
 // Elevation (metres) of mode `mode` (not UPF_ELEV_LAYERS) from the recorded layer values.
 template <class T> UPF_HD T mode_finish(int mode, const ModeState<T>& st, T x, T y, T z, T zero) {
   switch (mode) {
@@ -167,9 +175,8 @@ template <class T> UPF_HD T mode_finish(int mode, const ModeState<T>& st, T x, T
     case UPF_ELEV_LAKES:
     case UPF_ELEV_ISLANDS: {  // commonElevationMountains, :102-122
       if (st.flat) return st.land;
-      const T mask = st.v1;
-      const T rm = smoothstep1(sat_v(mask * 7.0f - 0.3f, zero));
-      const T tm = smoothstep1(sat_v(mask * -7.0f - 1.5f, zero));
+      const T rm = mode_ridge_mask(st, zero);
+      const T tm = mode_terrace_mask(st, zero);
       T ridge = st.v2;
       ridge = max_v(ridge - 0.1f, zero);
       ridge = pow_v(ridge, 1.6f);

@@ -68,10 +68,15 @@ UPF_HD Grad sq_root(Grad a) {
 UPF_HD float sq_root(float a) { return sqrt_f(a); }
 // transcendental functions of the scalar type (the C library's for float, except pow:
 // the library's own, upf_math.hpp; forward-mode derivatives for Grad)
+#if defined(__HIP_DEVICE_COMPILE__)
+// out of line on the device: ~250 instructions, inlined at a dozen places of a mode kernel
+__device__ __noinline__ float pow_v(float a, float e) { return upf_math::powf_(a, e); }
+#else
 UPF_HD float pow_v(float a, float e) { return upf_math::powf_(a, e); }
+#endif
 UPF_HD Grad pow_v(const Grad& a, float e) {
-  const float v = upf_math::powf_(a.v, e);
-  const float d = a.v != 0.0f ? e * upf_math::powf_(a.v, e - 1.0f) : 0.0f;  // d/da a^e, 0 at a = 0
+  const float v = pow_v(a.v, e);
+  const float d = a.v != 0.0f ? e * pow_v(a.v, e - 1.0f) : 0.0f;  // d/da a^e, 0 at a = 0
   return {v, d * a.dx, d * a.dy, d * a.dz};
 }
 UPF_HD float floor_v(float a) { return floorf(a); }
