@@ -1,6 +1,7 @@
 // upf_math.hpp -- pow and atan for the library's FP32 paths, computed in double
-// arithmetic from IEEE basic operations only (+, -, *, /, comparisons, bit moves), so
-// that every compiler and target that honours IEEE double rounding gives the same bits.
+// arithmetic from IEEE basic operations only (+, -, *, /, fused multiply-add, rounding to an
+// integer, comparisons, bit moves), so that every compiler and target that honours IEEE
+// double rounding gives the same bits.
 //
 // The elevation modes (sources/elevationModes.cpp: pow), the material stack
 // (sources/coloringModes.cpp: pow, atan) and the further shapes use these in place of the
@@ -10,9 +11,10 @@
 //
 // Methods (textbook):
 //   ln:   x = m 2^k with m in [sqrt(1/2), sqrt(2)), s = (m - 1) / (m + 1), |s| <= 0.1716,
-//         ln m = 2 atanh s = 2 (s + s^3/3 + ... + s^21/21)  (next term < 2^-60 relative)
-//   exp:  y = n ln2 + r with n = round(y / ln2), |r| <= 0.347, e^r by its Taylor series
-//         to r^16/16!  (next term < 2^-56), times 2^n assembled from bits
+//         ln m = 2 atanh s = 2 (s + s^3/3 + ... + s^19/19)  (next term < 2^-55 relative)
+//   exp:  y = n ln2 + r with n = round(y / ln2), |r| <= 0.347, n ln2 exact in the fused
+//         operation, e^r by its Taylor series to r^13/13!  (next term < 2^-57), times 2^n
+//         assembled from bits
 //   atan: |x| > 1 through pi/2 - atan(1/|x|); then table-driven reduction (Muller,
 //         "Elementary Functions", ch. 6): c = round(8a)/8, atan a = atan c + atan t with
 //         t = (a - c) / (1 + a c), |t| <= 1/16, atan t by its series to t^15/15; atan(i/8)
@@ -33,6 +35,16 @@ constexpr double kLn2 = 0.6931471805599453;
 constexpr double kInvLn2 = 1.4426950408889634;
 constexpr double kHalfPi = 1.5707963267948966;
 
+// a * b + c rounded once, c a constant.  On the device it is kept in scalar registers: as an
+// addend in vector registers each constant costs two moves beside its one multiply-add
+// (60 of a pow's 115 executed vector instructions).
+UPF_MATH_FN double fma_(double a, double b, double c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+s"(c));
+#endif
+  return __builtin_fma(a, b, c);
+}
+
 // ln x for finite x > 0 (a normal double: every float > 0 is one)
 UPF_MATH_FN double ln_pos(double x) {
   const uint64_t b = __builtin_bit_cast(uint64_t, x);
@@ -44,43 +56,38 @@ UPF_MATH_FN double ln_pos(double x) {
   }
   const double s = (m - 1.0) / (m + 1.0);
   const double s2 = s * s;
-  double p = 1.0 / 21.0;
-  p = p * s2 + 1.0 / 19.0;
-  p = p * s2 + 1.0 / 17.0;
-  p = p * s2 + 1.0 / 15.0;
-  p = p * s2 + 1.0 / 13.0;
-  p = p * s2 + 1.0 / 11.0;
-  p = p * s2 + 1.0 / 9.0;
-  p = p * s2 + 1.0 / 7.0;
-  p = p * s2 + 1.0 / 5.0;
-  p = p * s2 + 1.0 / 3.0;
-  p = p * s2 + 1.0;
-  return (double)k * kLn2 + 2.0 * s * p;
+  double p = 1.0 / 19.0;
+  p = fma_(p, s2, 1.0 / 17.0);
+  p = fma_(p, s2, 1.0 / 15.0);
+  p = fma_(p, s2, 1.0 / 13.0);
+  p = fma_(p, s2, 1.0 / 11.0);
+  p = fma_(p, s2, 1.0 / 9.0);
+  p = fma_(p, s2, 1.0 / 7.0);
+  p = fma_(p, s2, 1.0 / 5.0);
+  p = fma_(p, s2, 1.0 / 3.0);
+  p = fma_(p, s2, 1.0);
+  return __builtin_fma((double)k, kLn2, 2.0 * s * p);
 }
 
 // e^y for |y| <= 700
 UPF_MATH_FN double exp_small(double y) {
-  const double nf = y * kInvLn2 + 0.5;
-  int n = (int)nf;
-  if ((double)n > nf) n = n - 1;  // floor
-  const double r = y - (double)n * kLn2;
-  double p = 1.0 / 20922789888000.0;  // 1/16!
-  p = p * r + 1.0 / 1307674368000.0;
-  p = p * r + 1.0 / 87178291200.0;
-  p = p * r + 1.0 / 6227020800.0;
-  p = p * r + 1.0 / 479001600.0;
-  p = p * r + 1.0 / 39916800.0;
-  p = p * r + 1.0 / 3628800.0;
-  p = p * r + 1.0 / 362880.0;
-  p = p * r + 1.0 / 40320.0;
-  p = p * r + 1.0 / 5040.0;
-  p = p * r + 1.0 / 720.0;
-  p = p * r + 1.0 / 120.0;
-  p = p * r + 1.0 / 24.0;
-  p = p * r + 1.0 / 6.0;
-  p = p * r + 0.5;
-  p = p * r + 1.0;
-  p = p * r + 1.0;
+  const double nf = __builtin_rint(y * kInvLn2);
+  const int n = (int)nf;
+  const double r = __builtin_fma(-nf, kLn2, y);
+  double p = 1.0 / 6227020800.0;  // 1/13!
+  p = fma_(p, r, 1.0 / 479001600.0);
+  p = fma_(p, r, 1.0 / 39916800.0);
+  p = fma_(p, r, 1.0 / 3628800.0);
+  p = fma_(p, r, 1.0 / 362880.0);
+  p = fma_(p, r, 1.0 / 40320.0);
+  p = fma_(p, r, 1.0 / 5040.0);
+  p = fma_(p, r, 1.0 / 720.0);
+  p = fma_(p, r, 1.0 / 120.0);
+  p = fma_(p, r, 1.0 / 24.0);
+  p = fma_(p, r, 1.0 / 6.0);
+  p = fma_(p, r, 0.5);
+  p = fma_(p, r, 1.0);
+  p = fma_(p, r, 1.0);
   const double two_n = __builtin_bit_cast(double, (uint64_t)(n + 1023) << 52);
   return p * two_n;
 }
@@ -121,16 +128,16 @@ UPF_MATH_FN float atanf_(float x) {
   if (inv) a = 1.0 / a;  // a = inf gives 0: atan = pi/2
   const int i = (int)(a * 8.0 + 0.5);
   const double c = (double)i * 0.125;
-  const double t = (a - c) / (1.0 + a * c);
+  const double t = (a - c) / fma_(a, c, 1.0);
   const double t2 = t * t;
   double p = -1.0 / 15.0;
-  p = p * t2 + 1.0 / 13.0;
-  p = p * t2 - 1.0 / 11.0;
-  p = p * t2 + 1.0 / 9.0;
-  p = p * t2 - 1.0 / 7.0;
-  p = p * t2 + 1.0 / 5.0;
-  p = p * t2 - 1.0 / 3.0;
-  p = p * t2 + 1.0;
+  p = fma_(p, t2, 1.0 / 13.0);
+  p = fma_(p, t2, -1.0 / 11.0);
+  p = fma_(p, t2, 1.0 / 9.0);
+  p = fma_(p, t2, -1.0 / 7.0);
+  p = fma_(p, t2, 1.0 / 5.0);
+  p = fma_(p, t2, -1.0 / 3.0);
+  p = fma_(p, t2, 1.0);
   // atan(i / 8), i = 0 .. 8, as double constants (a select chain: no array in memory)
   const double ac = i == 0 ? 0.0
                   : i == 1 ? 0.12435499454676144
@@ -141,7 +148,7 @@ UPF_MATH_FN float atanf_(float x) {
                   : i == 6 ? 0.6435011087932844
                   : i == 7 ? 0.7188299996216245
                            : 0.7853981633974483;
-  double r = ac + t * p;
+  double r = __builtin_fma(t, p, ac);
   if (inv) r = kHalfPi - r;
   return (float)(neg ? -r : r);
 }
