@@ -153,8 +153,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 7
 // the sign words; lanes of one wave may belong to two chunks.  One group per thread: the
 // batch's small chunks have several times the 512^3 grid's mixed cells per group, and
 // their classification passes need the occupancy (four or eight groups per thread with
-// the next group's words loaded ahead and the tile sums written, as the single-grid
-// kernel does, took 67 and 82 us against 50 + 5.6 us for this kernel and the separate
+// the next group's words loaded ahead and the tile sums written took 67 and 82 us against 50 + 5.6 us for this kernel and the separate
 // tile pass).
 __global__ __launch_bounds__(256) void k_batch_classify(const BChunk* __restrict__ ch, int n_chunks, int64_t groups,
                                                         const uint64_t* __restrict__ S,

@@ -4,12 +4,10 @@
 //
 // Layout.  Nodes are cut into "groups" of 64 consecutive x nodes of one row (a row of
 // nx nodes has gpr = ceil(nx/64) groups); a wavefront handles a group, lane = x offset.
-//  classify  a workgroup owns one 64-wide column of 4 rows and sweeps a z range,
-//            keeping the current z plane in registers (each step loads only the next
-//            plane: rows j and j+1 at x and x+1).  Per group it ballots the inside bits
-//            into a 64-bit sign mask S[g] and packs the counts of the crossing edges
+//  classify  from the groups' sign words S[g] (written by the field kernel, or by a pass
+//            over a stored field), one group per thread: the counts of the crossing edges
 //            the group's nodes own (+x, +y, +z) and of the triangles of the cells whose
-//            min corner it holds into one word;
+//            min corner it holds, packed into one word;
 //  scan      exclusive prefix of (vertices, triangles, active groups); writes the dense
 //            per-group vertex offset and the compacted list of active groups;
 //  emit      one wave per active group writes each owned vertex at voff[g] + rank
@@ -94,42 +92,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
                       s_pass[wave], pos, nrm, idx, cap_v, cap_t);
 }
 
-// Packed counts of every group, and the sums of the scan tiles the workgroup covers
-// (the scan's first pass): thread t takes groups t + 256 u, so tile q of the workgroup
-// is u in [q * kScanTile / 256, (q + 1) * kScanTile / 256).
-__global__ __launch_bounds__(256) void k_mc_classify_signs(const uint64_t* __restrict__ S, const McDims d,
-                                                           uint32_t* __restrict__ counts,
-                                                           uint4* __restrict__ tile_sums) {
-  constexpr int kTiles = 256 * kClassifyGroups / kScanTile, kPerTile = kScanTile / 256;
+// Packed counts of every group, one group per thread, and the sum of the scan tile that the
+// workgroup's kScanTile groups are (the scan's first pass).
+__global__ __launch_bounds__(kScanTile) void k_mc_classify_signs(const uint64_t* __restrict__ S, const McDims d,
+                                                                 uint32_t* __restrict__ counts,
+                                                                 uint4* __restrict__ tile_sums) {
   __shared__ uint8_t s_ntris[256];
-  __shared__ SignPass s_pass[4];
-  s_ntris[threadIdx.x] = upf_mc_ntris[threadIdx.x];
+  __shared__ SignPass s_pass[kScanTile / 64];
+  if (threadIdx.x < 256) s_ntris[threadIdx.x] = upf_mc_ntris[threadIdx.x];
   __syncthreads();
-  // the next group's words are loaded before the current group is classified
-  const int64_t g0 = (int64_t)blockIdx.x * (256 * kClassifyGroups) + threadIdx.x;
-  uint4 sum[kTiles];
-#pragma unroll
-  for (int q = 0; q < kTiles; q++) sum[q] = make_uint4(0, 0, 0, 0);
-  GroupWords w = load_group_words(S, d, g0, g0 < d.groups);
-#pragma unroll
-  for (int u = 0; u < kClassifyGroups; u++) {
-    const int64_t g = g0 + 256 * u;
-    const bool in = g < d.groups;
-    GroupWords next = w;
-    if (u + 1 < kClassifyGroups) next = load_group_words(S, d, g + 256, g + 256 < d.groups);
-    const uint32_t c = classify_group_words(w, d.nx, in, s_ntris, s_pass[threadIdx.x >> 6]);
-    if (in) counts[g] = c;
-    sum[u / kPerTile] = add4(sum[u / kPerTile], unpack_counts<kScanMc>(in ? c : 0u));
-    w = next;
-  }
-  const int64_t ntiles = (d.groups + kScanTile - 1) / kScanTile;
-#pragma unroll
-  for (int q = 0; q < kTiles; q++) {
-    uint4 total;
-    (void)block_exclusive_scan(sum[q], &total);
-    const int64_t tile = (int64_t)blockIdx.x * kTiles + q;
-    if (threadIdx.x == 0 && tile < ntiles) tile_sums[tile] = total;
-  }
+  const int64_t g = (int64_t)blockIdx.x * kScanTile + threadIdx.x;
+  const bool in = g < d.groups;
+  const uint32_t c = classify_group_words(load_group_words(S, d, g, in), d.nx, in, s_ntris, s_pass[threadIdx.x >> 6]);
+  if (in) counts[g] = c;
+  const uint4 total = tile_sum(unpack_counts<kScanMc>(in ? c : 0u));
+  if (threadIdx.x == 0) tile_sums[blockIdx.x] = total;
 }
 
 // ------------------------------------------------------------------ scan
@@ -309,9 +286,7 @@ int mc_classify_signs_scan(const DGrid& g, void* d_ws, size_t ws_bytes, hipStrea
   const McLayout L = mc_layout(g);
   if (!d_ws || ws_bytes < L.bytes) return UPF_ERR_WORKSPACE;
   const McPtrs P = mc_ptrs(L, d_ws);
-  const int64_t per_block = 256 * kClassifyGroups;
-  hipLaunchKernelGGL(k_mc_classify_signs, dim3((unsigned)((L.d.groups + per_block - 1) / per_block)), dim3(256), 0, s,
-                     P.S, L.d, P.counts, P.tiles);
+  hipLaunchKernelGGL(k_mc_classify_signs, dim3((unsigned)L.tiles), dim3(kScanTile), 0, s, P.S, L.d, P.counts, P.tiles);
   UPF_LAUNCH_CHECK();
   return mc_scan_launch(P.counts, L.d.groups, P.tiles, P.total, P.voff, P.act, nullptr, s, kScanMc, true);
 }

@@ -123,7 +123,26 @@ __device__ __forceinline__ uint4 block_exclusive_scan(uint4 v, uint4* total) {
   return make_uint4(before.x + inc.x - v.x, before.y + inc.y - v.y, before.z + inc.z - v.z, 0);
 }
 
+// Sum over a workgroup of kScanTile threads (valid in thread 0): a scan tile's.
+__device__ __forceinline__ uint4 tile_sum(uint4 v) {
+  constexpr int kWaves = kScanTile / 64;
+  __shared__ uint4 wsum[kWaves];
+  const uint4 inc = make_uint4((unsigned)wave_inclusive_sum((int)v.x), (unsigned)wave_inclusive_sum((int)v.y),
+                               (unsigned)wave_inclusive_sum((int)v.z), 0u);
+  if ((threadIdx.x & 63) == 63) wsum[threadIdx.x >> 6] = inc;
+  __syncthreads();
+  uint4 all = wsum[0];
+  for (int w = 1; w < kWaves; w++) all = add4(all, wsum[w]);
+  return all;
+}
+
 // ------------------------------------------------------------------ classify
+// One workgroup classifies a scan tile of kScanTile groups, a group per thread.  With 256
+// threads of eight groups each (the next group's words loaded ahead) the chip was idle at
+// all but the largest grids and the kernel no faster there: marching cubes of a stored
+// field took 51 us at 48^3, 74 at 110^3, 91 at 256^3 and 197 at 512^3; 25, 38, 69 and 193 so.
+// (The batched kernel keeps 256 threads and a separate tile pass: its workgroups' 1024 groups
+// would cross chunks, and it measured 0.6% slower per batch.)
 // Packed counts of a group from the sign words alone (written by the field kernel or
 // k_mc_signs), one lane per group.  Crossing masks come from S of the group, of its +x
 // neighbour group and of the +y / +z rows (8 words, load_group_words), so vertex counts
@@ -134,11 +153,6 @@ __device__ __forceinline__ uint4 block_exclusive_scan(uint4 v, uint4* total) {
 // LDS) and adds the code's triangle count to the group's LDS counter.  A wave with ~6 active groups of ~7 mixed cells each needs
 // one pass, instead of one wave-wide step per active group.  Lanes may belong to
 // different grids (batched chunks): everything but the pass bookkeeping is per lane.
-
-// groups per thread of the classification kernels (thread t of a workgroup takes groups
-// t + 256 u), a whole number of scan tiles per workgroup so that they write the tile sums
-constexpr int kClassifyGroups = 8;
-static_assert((256 * kClassifyGroups) % kScanTile == 0 && kScanTile % 256 == 0, "whole scan tiles per workgroup");
 
 struct SignPass {  // one wave's LDS
   uint64_t w[8][64];  // word q of lane (group) t at w[q][t]: consecutive lanes, no bank conflicts
