@@ -655,6 +655,21 @@ int upf_image_dilate(float* d_img, float* d_scratch, int32_t width, int32_t heig
 /* U8 conversion: out = NaN ? 0 : (uint8)(saturate(v) * 255 + 0.5), n values. */
 int upf_image_to_u8(const float* d_img, int64_t n_values, uint8_t* d_out, void* stream);
 
+/* Both steps of several images at once, without changing them: d_out [height][width]
+ * [out_channels] gets the U8 conversion of d_in [height][width][channels] dilated by
+ * `rounds` (at most UPF_POST_MAX_ROUNDS; more: UPF_ERR_INVALID_VALUE), the bytes that
+ * upf_image_dilate and upf_image_to_u8 give.  channels is 1..4; the channels from
+ * `channels` to `out_channels` (at most 4) are 0 (a special map of roughness with metallic
+ * 0).  The outputs must not overlap the inputs. */
+#define UPF_POST_MAX_ROUNDS 7
+typedef struct upf_post_image {
+  const float* d_in;
+  uint8_t* d_out;
+  int32_t width, height;
+  int32_t channels, out_channels;
+} upf_post_image;
+int upf_images_post(const upf_post_image* images, int32_t n_images, int32_t rounds, void* stream);
+
 /* The two conversions a land chunk's U8 maps get before export
  * (LandProcessor::chunkEntry, sources/generator.cpp:136-139).  cage's
  * imageConvertSpecialToGltfPbr and imageConvertHeigthToNormal are not in the reference

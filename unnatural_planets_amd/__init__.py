@@ -636,13 +636,34 @@ def texture_post(tex: Textures, rounds: int = 7, stream=None):
     special [h, w, 2] = (roughness, metallic = 0) and height [h, w], each dilated by
     `rounds` texels and converted to U8.  Returns (albedo_u8, special_u8, height_u8)."""
     torch = _torch()
-    albedo = tex.albedo.clone()
-    special = torch.stack([tex.roughness, torch.where(torch.isnan(tex.roughness), tex.roughness,
-                                                      torch.zeros_like(tex.roughness))], dim=2).contiguous()
-    height = tex.bump.clone()
-    for im in (albedo, special, height):
-        image_dilate(im, rounds, stream)
-    return image_to_u8(albedo, stream), image_to_u8(special, stream), image_to_u8(height, stream)
+    r = tex.roughness
+    if rounds > spec_mod.POST_MAX_ROUNDS or r.dim() != 2:
+        special = torch.stack([r, torch.where(torch.isnan(r), r, torch.zeros_like(r))], dim=2).contiguous()
+        return texture_post_images(tex.albedo, special, tex.bump, rounds, stream)
+    return _images_post((tex.albedo, r, tex.bump), (None, 2, None), rounds, stream)
+
+
+def _images_post(images, out_channels, rounds, stream):
+    """Dilation and U8 conversion of float images [h, w] or [h, w, c] in one launch
+    (upf_images_post); out_channels: None for the image's own, more for zeros after them."""
+    torch = _torch()
+    args = (spec_mod.PostImage * len(images))()
+    outs, keep = [], []
+    for a, im, oc in zip(args, images, out_channels):
+        if not im.is_contiguous():
+            im = im.clone()
+        _check_f32(im, "img")
+        if im.dim() not in (2, 3):
+            raise ValueError("img must be [h, w] or [h, w, c]")
+        c = 1 if im.dim() == 2 else int(im.shape[2])
+        out = torch.empty(tuple(im.shape) if oc is None else tuple(im.shape[:2]) + (oc,), dtype=torch.uint8,
+                          device=im.device)
+        a.d_in, a.d_out, a.width, a.height = im.data_ptr(), out.data_ptr(), int(im.shape[1]), int(im.shape[0])
+        a.channels, a.out_channels = c, c if oc is None else oc
+        outs.append(out)
+        keep.append(im)
+    check(lib().upf_images_post(args, len(images), rounds, _stream(stream)), "upf_images_post")
+    return tuple(outs)
 
 
 @_on_stream
@@ -740,6 +761,8 @@ def generate_textures(m: MaterialSpec, mesh: Mesh, width: int, height: int, stre
 @_on_stream
 def texture_post_images(albedo, special, height, rounds: int = 7, stream=None):
     """Dilation and U8 conversion of the three images (sources/textures.cpp:73-81)."""
+    if rounds <= spec_mod.POST_MAX_ROUNDS:
+        return _images_post((albedo, special, height), (None,) * 3, rounds, stream)
     ims = [albedo.clone(), special.clone(), height.clone()]
     for im in ims:
         image_dilate(im, rounds, stream)

@@ -384,48 +384,57 @@ constexpr int kDilS = kDilT + 2 * kDilR;    // loaded side
 constexpr uint8_t kTagOut = 254, kTagNone = 255;
 constexpr int kDilThreads = 512;  // 8 waves share a tile's rounds
 
-// only_nan: write only the texels that were NaN when loaded (the last launch of an
-// in-place dilation; k_dilate_merge then copies them back).
+// LDS of a tile: C values, a tag and a list entry per loaded texel.
+struct DilTile {
+  float* v;       // [C][kDilS * kDilS]
+  uint8_t* tag;   // [kDilS * kDilS]
+  uint16_t* nan;  // [kDilS * kDilS]: the loaded texels that are NaN (only they can change)
+  int* nnan;
+};
+
+// Loads the tile whose loaded corner is (x0, y0) and runs the rounds on it, by a workgroup
+// of kDilThreads; false (in every thread) when nothing changed, because no loaded texel or
+// none but NaN is valid.  Rounds end early once one fills nothing.
 template <int C>
-__global__ __launch_bounds__(kDilThreads) void k_dilate(const float* __restrict__ in, float* __restrict__ out, int w, int h,
-                                                int rounds, bool only_nan) {
-  __shared__ float s_v[C][kDilS * kDilS];
-  __shared__ uint8_t s_tag[kDilS * kDilS];
-  __shared__ uint16_t s_nan[kDilS * kDilS];  // the loaded texels that are NaN (only they can change)
-  __shared__ int s_nnan;
-  const int x0 = (int)blockIdx.x * kDilT - kDilR, y0 = (int)blockIdx.y * kDilT - kDilR;
-  if (threadIdx.x == 0) s_nnan = 0;
+__device__ __forceinline__ bool dilate_tile(const DilTile T, const float* __restrict__ in, int w, int h, int x0, int y0,
+                                            int rounds) {
+  constexpr int N = kDilS * kDilS;
+  if (threadIdx.x == 0) *T.nnan = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  for (int t0 = 0; t0 < kDilS * kDilS; t0 += kDilThreads) {  // uniform trip count: whole waves ballot
+  bool valid_here = false;
+  for (int t0 = 0; t0 < N; t0 += kDilThreads) {  // uniform trip count: whole waves ballot
     const int t = t0 + (int)threadIdx.x;
     bool nan_here = false;
-    if (t < kDilS * kDilS) {
+    if (t < N) {
       const int ly = t / kDilS, lx = t - ly * kDilS;
       const int x = x0 + lx, y = y0 + ly;
       uint8_t tag = kTagOut;
       if (x >= 0 && x < w && y >= 0 && y < h) {
         const int64_t o = ((int64_t)y * w + x) * C;
 #pragma unroll
-        for (int ch = 0; ch < C; ch++) s_v[ch][t] = in[o + ch];
-        nan_here = isnan(s_v[0][t]);
+        for (int ch = 0; ch < C; ch++) T.v[ch * N + t] = in[o + ch];
+        nan_here = isnan(T.v[t]);
         tag = nan_here ? kTagNone : 0;
+        valid_here = valid_here || !nan_here;
       }
-      s_tag[t] = tag;
+      T.tag[t] = tag;
     }
     const uint64_t m = __ballot(nan_here);
     int base = 0;
-    if (lane == 0 && m) base = atomicAdd(&s_nnan, __popcll(m));
+    if (lane == 0 && m) base = atomicAdd(T.nnan, __popcll(m));
     base = __shfl(base, 0, 64);
-    if (nan_here) s_nan[base + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)t;
+    if (nan_here) T.nan[base + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)t;
   }
-  __syncthreads();
-  const int nnan = s_nnan;
+  const bool any_valid = __syncthreads_or(valid_here);
+  const int nnan = *T.nnan;
+  if (!any_valid || nnan == 0) return false;
   for (int k = 1; k <= rounds; k++) {
+    bool filled = false;
     for (int e = threadIdx.x; e < nnan; e += kDilThreads) {
-      const int idx = s_nan[e];
+      const int idx = T.nan[e];
       const int ly = idx / kDilS, lx = idx - ly * kDilS;  // constant divisor
-      if (lx < k || lx >= kDilS - k || ly < k || ly >= kDilS - k || s_tag[idx] != kTagNone) continue;
+      if (lx < k || lx >= kDilS - k || ly < k || ly >= kDilS - k || T.tag[idx] != kTagNone) continue;
       float sum[C];
 #pragma unroll
       for (int ch = 0; ch < C; ch++) sum[ch] = 0.0f;
@@ -436,26 +445,41 @@ __global__ __launch_bounds__(kDilThreads) void k_dilate(const float* __restrict_
         for (int dx = -1; dx <= 1; dx++) {
           if (dx == 0 && dy == 0) continue;
           const int q = idx + dy * kDilS + dx;
-          if (s_tag[q] >= k) continue;  // NaN, outside, or filled in this round
+          if (T.tag[q] >= k) continue;  // NaN, outside, or filled in this round
 #pragma unroll
-          for (int ch = 0; ch < C; ch++) sum[ch] = sum[ch] + s_v[ch][q];
+          for (int ch = 0; ch < C; ch++) sum[ch] = sum[ch] + T.v[ch * N + q];
           cnt++;
         }
       if (cnt) {
 #pragma unroll
-        for (int ch = 0; ch < C; ch++) s_v[ch][idx] = sum[ch] / (float)cnt;
-        s_tag[idx] = (uint8_t)k;
+        for (int ch = 0; ch < C; ch++) T.v[ch * N + idx] = sum[ch] / (float)cnt;
+        T.tag[idx] = (uint8_t)k;
+        filled = true;
       }
     }
-    __syncthreads();
+    if (!__syncthreads_or(filled)) break;
   }
+  return true;
+}
+
+// only_nan: write only the texels that were NaN when loaded (the last launch of an
+// in-place dilation; k_dilate_merge then copies them back).
+template <int C>
+__global__ __launch_bounds__(kDilThreads) void k_dilate(const float* __restrict__ in, float* __restrict__ out, int w, int h,
+                                                int rounds, bool only_nan) {
+  __shared__ float s_v[C * kDilS * kDilS];
+  __shared__ uint8_t s_tag[kDilS * kDilS];
+  __shared__ uint16_t s_nan[kDilS * kDilS];
+  __shared__ int s_nnan;
+  const int x0 = (int)blockIdx.x * kDilT - kDilR, y0 = (int)blockIdx.y * kDilT - kDilR;
+  (void)dilate_tile<C>({s_v, s_tag, s_nan, &s_nnan}, in, w, h, x0, y0, rounds);
   for (int t = threadIdx.x; t < kDilT * kDilT; t += kDilThreads) {
     const int ly = kDilR + t / kDilT, lx = kDilR + t % kDilT;
     const int x = x0 + lx, y = y0 + ly;
     if (x < w && y < h && !(only_nan && s_tag[ly * kDilS + lx] == 0)) {
       const int64_t o = ((int64_t)y * w + x) * C;
 #pragma unroll
-      for (int ch = 0; ch < C; ch++) out[o + ch] = s_v[ch][ly * kDilS + lx];
+      for (int ch = 0; ch < C; ch++) out[o + ch] = s_v[ch * kDilS * kDilS + ly * kDilS + lx];
     }
   }
 }
@@ -607,6 +631,107 @@ __global__ __launch_bounds__(256) void k_to_u8_x4(const float4* __restrict__ in,
   if (i >= n4) return;
   const float4 v = in[i];
   out[i] = to_u8(v.x) | (to_u8(v.y) << 8) | (to_u8(v.z) << 16) | (to_u8(v.w) << 24);
+}
+
+// ------------------------------------------------------------------ dilation to U8
+// The images after the bake: dilation by up to kDilR rounds and U8 conversion in one pass,
+// several images in one launch (blockIdx.z).  A workgroup streams its kDilT x kDilT texels
+// (float4 reads, 4-byte writes where the rows allow them) and only a tile that holds a NaN
+// loads its halo and runs the rounds in LDS, then overwrites the bytes of the texels it
+// filled: no copy of the image, no float result, no merge.  HBM-bound where most tiles
+// are covered: 24 B read and 6 B written per texel of a chunk's three images.  The U8
+// values are image_to_u8's of image_dilate's result, bit for bit.  Three images (3 + 2 + 1
+// channels), copies + dilations + merges + conversions against one pass: 4096^2 covered 500
+// and 104 us (4.8 TB/s), 30% uncovered in 8 x 8 blocks 966 and 745, three quarters covered
+// 746 and 146; 500^2 90 and 21 us.  Measured and not kept: four tiles per workgroup, all
+// streamed before the first one's rounds (89, 880 and 204 us at 4096^2); a streaming kernel
+// and one that fills the tiles its flags name (101, 982 and 132: the second reads the tiles
+// again); leaving the tiles of nothing but NaN to a second launch (135, 768 and 163).
+constexpr int kPostImages = 4;
+struct PostArgs {
+  upf_post_image im[kPostImages];
+};
+
+template <int C>
+__device__ __forceinline__ void post_tile(const upf_post_image& im, int rounds, char* lds, int* nnan) {
+  const float* __restrict__ in = im.d_in;
+  uint8_t* __restrict__ out = im.d_out;
+  const int w = im.width, h = im.height, oc = im.out_channels;
+  const int x0 = (int)blockIdx.x * kDilT, y0 = (int)blockIdx.y * kDilT;
+  if (x0 >= w || y0 >= h) return;  // the grid covers the largest image
+  bool nan_here = false, valid_here = false;
+  const int row_f = min(kDilT, w - x0) * C, rows = min(kDilT, h - y0);  // floats per tile row
+  const bool vec = ((int64_t)w * C) % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0 &&
+                   (oc == C ? reinterpret_cast<uintptr_t>(out) % 4 == 0
+                            : C == 1 && oc == 2 && reinterpret_cast<uintptr_t>(out) % 8 == 0);
+  if (vec) {
+    constexpr int kRowV = kDilT * C / 4, kV = kDilT * kRowV;
+#pragma unroll
+    for (int v0 = 0; v0 < kV; v0 += kDilThreads) {
+      const int v = v0 + (int)threadIdx.x;
+      const int r = v / kRowV, e = 4 * (v - r * kRowV);
+      if (v >= kV || r >= rows || e >= row_f) continue;
+      const int64_t o = ((int64_t)(y0 + r) * w + x0) * C + e;
+      const float4 f = *reinterpret_cast<const float4*>(in + o);
+      const float a[4] = {f.x, f.y, f.z, f.w};
+      uint32_t b[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        b[j] = to_u8(a[j]);
+        if ((e + j) % C == 0) (isnan(a[j]) ? nan_here : valid_here) = true;
+      }
+      if (oc == C) *reinterpret_cast<uint32_t*>(out + o) = b[0] | (b[1] << 8) | (b[2] << 16) | (b[3] << 24);
+      else *reinterpret_cast<uint2*>(out + 2 * o) = make_uint2(b[0] | (b[1] << 16), b[2] | (b[3] << 16));
+    }
+  } else {
+    for (int t = threadIdx.x; t < kDilT * kDilT; t += kDilThreads) {
+      const int x = x0 + t % kDilT, y = y0 + t / kDilT;
+      if (x >= w || y >= h) continue;
+      const int64_t p = (int64_t)y * w + x;
+#pragma unroll
+      for (int ch = 0; ch < C; ch++) {
+        const float f = in[p * C + ch];
+        out[p * oc + ch] = (uint8_t)to_u8(f);
+        if (ch == 0) (isnan(f) ? nan_here : valid_here) = true;
+      }
+      for (int ch = C; ch < oc; ch++) out[p * oc + ch] = 0;
+    }
+  }
+  if (!__syncthreads_or(nan_here) || rounds == 0) return;
+  constexpr int N = kDilS * kDilS;
+  if (!__syncthreads_or(valid_here)) {  // nothing but NaN: done unless the halo has a valid texel
+    bool near = false;
+#pragma unroll
+    for (int t0 = 0; t0 < N; t0 += kDilThreads) {
+      const int t = t0 + (int)threadIdx.x, x = x0 - kDilR + t % kDilS, y = y0 - kDilR + t / kDilS;
+      const bool inner = x >= x0 && x < x0 + kDilT && y >= y0 && y < y0 + kDilT;
+      if (t < N && !inner && x >= 0 && x < w && y >= 0 && y < h) near = near || !isnan(in[((int64_t)y * w + x) * C]);
+    }
+    if (!__syncthreads_or(near)) return;
+  }
+  float* v = reinterpret_cast<float*>(lds);
+  uint16_t* list = reinterpret_cast<uint16_t*>(v + C * N);
+  uint8_t* tag = reinterpret_cast<uint8_t*>(list + N);
+  if (!dilate_tile<C>({v, tag, list, nnan}, in, w, h, x0 - kDilR, y0 - kDilR, rounds)) return;
+  for (int t = threadIdx.x; t < kDilT * kDilT; t += kDilThreads) {
+    const int q = (kDilR + t / kDilT) * kDilS + kDilR + t % kDilT;
+    if (tag[q] == 0 || tag[q] > kDilR) continue;  // valid from the start, still NaN, or outside
+    const int64_t p = (int64_t)(y0 + t / kDilT) * w + x0 + t % kDilT;
+#pragma unroll
+    for (int ch = 0; ch < C; ch++) out[p * oc + ch] = (uint8_t)to_u8(v[ch * N + q]);
+  }
+}
+
+__global__ __launch_bounds__(kDilThreads) void k_images_post(const PostArgs a, int rounds) {
+  extern __shared__ __attribute__((aligned(16))) char s_post[];
+  __shared__ int s_nnan;
+  const upf_post_image& im = a.im[blockIdx.z];
+  switch (im.channels) {
+    case 1: post_tile<1>(im, rounds, s_post, &s_nnan); break;
+    case 2: post_tile<2>(im, rounds, s_post, &s_nnan); break;
+    case 3: post_tile<3>(im, rounds, s_post, &s_nnan); break;
+    default: post_tile<4>(im, rounds, s_post, &s_nnan); break;
+  }
 }
 
 int atlas_side(int64_t n, int w, int h) {
@@ -769,6 +894,36 @@ int upf_image_dilate(float* d_img, float* d_scratch, int32_t w, int32_t h, int32
     float* t = a;
     a = b;
     b = t;
+  }
+  UPF_LAUNCH_CHECK();
+  return UPF_OK;
+}
+
+int upf_images_post(const upf_post_image* images, int32_t n, int32_t rounds, void* stream) {
+  if (n < 0 || rounds < 0) return UPF_ERR_BAD_GRID;
+  if (rounds > kDilR) return UPF_ERR_INVALID_VALUE;
+  if (n == 0) return UPF_OK;
+  if (!images) return UPF_ERR_NULL;
+  for (int i = 0; i < n; i++) {
+    const upf_post_image& im = images[i];
+    if (im.width < 1 || im.height < 1) return UPF_ERR_BAD_GRID;
+    if (im.channels < 1 || im.channels > 4 || im.out_channels < im.channels || im.out_channels > 4)
+      return UPF_ERR_INVALID_VALUE;
+    if (!im.d_in || !im.d_out) return UPF_ERR_NULL;
+  }
+  for (int first = 0; first < n; first += kPostImages) {
+    PostArgs a{};
+    const int count = std::min(n - first, kPostImages);
+    int w = 0, h = 0, c = 0;
+    for (int i = 0; i < count; i++) {
+      a.im[i] = images[first + i];
+      w = std::max(w, a.im[i].width);
+      h = std::max(h, a.im[i].height);
+      c = std::max(c, a.im[i].channels);
+    }
+    const dim3 grid((unsigned)((w + kDilT - 1) / kDilT), (unsigned)((h + kDilT - 1) / kDilT), (unsigned)count);
+    const size_t lds = (size_t)kDilS * kDilS * (4 * c + 3);
+    hipLaunchKernelGGL(k_images_post, grid, dim3(kDilThreads), lds, as_stream(stream), a, rounds);
   }
   UPF_LAUNCH_CHECK();
   return UPF_OK;

@@ -350,6 +350,18 @@ def bake_spec(field: FieldSpec, detail: Layer | None = None, bands=(-0.01, 0.005
     return b
 
 
+# ---------------------------------------------------------------------------- texture post
+POST_MAX_ROUNDS = 7
+
+
+class PostImage(ctypes.Structure):
+    _fields_ = [("d_in", ctypes.c_void_p), ("d_out", ctypes.c_void_p), ("width", ctypes.c_int32),
+                ("height", ctypes.c_int32), ("channels", ctypes.c_int32), ("out_channels", ctypes.c_int32)]
+
+
+assert ctypes.sizeof(PostImage) == 32
+
+
 # ---------------------------------------------------------------------------- material stack
 COLORING = {"default": 0, "barren": 1, "debug": 2}
 PURPOSE = {"land": 1, "water": 2, "navigation": 3}
