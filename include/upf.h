@@ -494,6 +494,13 @@ size_t upf_nb_workspace_bytes(const upf_grid* fine, int64_t max_active_blocks);
 int upf_nb_extract(const upf_field_spec* spec, const upf_grid* fine, float iso, float band,
                    upf_mesh_buffers* out, uint64_t* d_vertex_keys, void* d_workspace,
                    size_t workspace_bytes, upf_nb_stats* stats, void* stream);
+/* The mesh of the last upf_nb_extract on this workspace, which returned UPF_ERR_CAPACITY
+ * (the same spec, grid, iso, workspace and its stats; nothing else may have used the
+ * workspace since): emitted from the blocks it evaluated, without evaluating them again.
+ * Errors as upf_nb_extract's; does not synchronise. */
+int upf_nb_emit(const upf_field_spec* spec, const upf_grid* fine, float iso, upf_mesh_buffers* out,
+                uint64_t* d_vertex_keys, void* d_ws, size_t ws_bytes, const upf_nb_stats* stats, void* stream);
+
 
 /* ---- texel bake ---------------------------------------------------------------------
  * Replaces meshGenerateTexture(mesh, {w, h, generator = Generator::pixel})

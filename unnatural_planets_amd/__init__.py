@@ -487,37 +487,39 @@ class NbWorkspace:
 @_on_stream
 def nb_extract(s: FieldSpec, g: Grid, band: float, iso: float = 0.0, normals: bool = True, keys: bool = False,
                workspace: NbWorkspace | None = None, device=None, stream=None):
-    """Narrow-band marching cubes of the fine grid g (upf_nb_extract).  Grows the
-    workspace and the mesh buffers as the library reports (each retry reruns the
-    extraction).  Returns (Mesh, keys or None, NbStats)."""
+    """Narrow-band marching cubes of the fine grid g (upf_nb_extract, upf_nb_emit).  Grows
+    the workspace as the library reports (each retry reruns the extraction); the mesh is
+    emitted once its size is known, from the blocks already evaluated.  Returns (Mesh, keys
+    or None, NbStats)."""
     torch = _torch()
     dev = _dev(device)
     ws = workspace or NbWorkspace(g, 1024, dev)
     stats = spec_mod.NbStats()
-    cap_v = cap_t = 0
     st = _stream(stream)
+    L = lib()
     for _ in range(4):
-        pos = torch.empty((cap_v, 3), dtype=torch.float32, device=dev)
-        nrm = torch.empty((cap_v, 3), dtype=torch.float32, device=dev) if normals else None
-        idx = torch.empty((cap_t, 3), dtype=torch.int32, device=dev)
-        kk = torch.empty((cap_v,), dtype=torch.int64, device=dev) if keys else None
         mb = MeshBuffers()
-        mb.positions = pos.data_ptr() if cap_v else None
-        mb.normals = nrm.data_ptr() if (normals and cap_v) else None
-        mb.indices = idx.data_ptr() if cap_t else None
-        mb.cap_vertices, mb.cap_triangles = cap_v, cap_t
-        r = lib().upf_nb_extract(ctypes.byref(s), ctypes.byref(g), iso, band, ctypes.byref(mb),
-                                 _ptr(kk) if (keys and cap_v) else None, _ptr(ws.buf), ws.bytes,
-                                 ctypes.byref(stats), st)
+        r = L.upf_nb_extract(ctypes.byref(s), ctypes.byref(g), iso, band, ctypes.byref(mb), None, _ptr(ws.buf),
+                             ws.bytes, ctypes.byref(stats), st)
         if r == spec_mod.ERR_WORKSPACE and stats.active_blocks > ws.max_active:
             ws = NbWorkspace(g, stats.active_blocks, dev)
             continue
-        if r == spec_mod.ERR_CAPACITY:
-            cap_v, cap_t = int(stats.n_vertices), int(stats.n_triangles)
-            continue
-        check(r, "upf_nb_extract")
         n_v, n_t = int(stats.n_vertices), int(stats.n_triangles)
-        return Mesh(pos[:n_v], nrm[:n_v] if normals else None, idx[:n_t]), (kk[:n_v] if keys else None), stats
+        if r not in (0, spec_mod.ERR_CAPACITY):
+            check(r, "upf_nb_extract")
+        pos = torch.empty((n_v, 3), dtype=torch.float32, device=dev)
+        nrm = torch.empty((n_v, 3), dtype=torch.float32, device=dev) if normals else None
+        idx = torch.empty((n_t, 3), dtype=torch.int32, device=dev)
+        kk = torch.empty((n_v,), dtype=torch.int64, device=dev) if keys else None
+        if r == spec_mod.ERR_CAPACITY:
+            mb.positions = pos.data_ptr() if n_v else None
+            mb.normals = nrm.data_ptr() if (normals and n_v) else None
+            mb.indices = idx.data_ptr() if n_t else None
+            mb.cap_vertices, mb.cap_triangles = n_v, n_t
+            check(L.upf_nb_emit(ctypes.byref(s), ctypes.byref(g), iso, ctypes.byref(mb),
+                                _ptr(kk) if (keys and n_v) else None, _ptr(ws.buf), ws.bytes, ctypes.byref(stats),
+                                st), "upf_nb_emit")
+        return Mesh(pos, nrm, idx), kk, stats
     raise UpfError(spec_mod.ERR_CAPACITY, "upf_nb_extract did not converge")
 
 

@@ -86,6 +86,9 @@ SIGNATURES = {
     "upf_nb_extract": (ctypes.c_int, [ctypes.POINTER(FieldSpec), ctypes.POINTER(Grid), ctypes.c_float, ctypes.c_float,
                                       ctypes.POINTER(MeshBuffers), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
                                       ctypes.POINTER(NbStats), ctypes.c_void_p]),
+    "upf_nb_emit": (ctypes.c_int, [ctypes.POINTER(FieldSpec), ctypes.POINTER(Grid), ctypes.c_float,
+                                   ctypes.POINTER(MeshBuffers), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
+                                   ctypes.POINTER(NbStats), ctypes.c_void_p]),
     "upf_image_dilate": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
                                         ctypes.c_int32, ctypes.c_void_p]),
     "upf_images_post": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]),

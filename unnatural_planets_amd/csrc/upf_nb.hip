@@ -445,6 +445,64 @@ int nb_dims(const DGrid& g, NbDims* d) {
   return UPF_OK;
 }
 
+// The workspace of a call: its layout for the largest active-block capacity it holds.
+struct NbWs {
+  int64_t cap;
+  float* coarse;
+  uint32_t* counts;
+  uint4 *tiles, *total_a;
+  uint2* act;
+  int32_t* map;
+  float* bricks;
+  uint16_t* tabs;
+  uint32_t *bcounts, *voff, *toff;
+  uint4* total_b;
+  int64_t n_coarse;
+};
+
+int nb_workspace(const NbDims& d, void* d_ws, size_t ws_bytes, NbWs* o) {
+  const NbLayout L0 = nb_layout(d, 0);
+  if (!d_ws || ws_bytes < L0.bytes) return UPF_ERR_WORKSPACE;
+  const size_t per = 6 * (size_t)kBrick + 12;
+  int64_t cap = std::min<int64_t>(d.blocks, (int64_t)((ws_bytes - L0.bytes) / per));
+  while (cap > 0 && nb_layout(d, cap).bytes > ws_bytes) cap--;
+  const NbLayout L = nb_layout(d, cap);
+  char* w = static_cast<char*>(d_ws);
+  o->cap = cap;
+  o->n_coarse = L.coarse;
+  o->coarse = reinterpret_cast<float*>(w + L.off_coarse);
+  o->counts = reinterpret_cast<uint32_t*>(w + L.off_counts);
+  o->tiles = reinterpret_cast<uint4*>(w + L.off_tiles);
+  o->total_a = reinterpret_cast<uint4*>(w + L.off_total_a);
+  o->act = reinterpret_cast<uint2*>(w + L.off_act);
+  o->map = reinterpret_cast<int32_t*>(w + L.off_map);
+  o->bricks = reinterpret_cast<float*>(w + L.off_bricks);
+  o->tabs = reinterpret_cast<uint16_t*>(w + L.off_tabs);
+  o->bcounts = reinterpret_cast<uint32_t*>(w + L.off_bcounts);
+  o->voff = reinterpret_cast<uint32_t*>(w + L.off_voff);
+  o->toff = reinterpret_cast<uint32_t*>(w + L.off_toff);
+  o->total_b = reinterpret_cast<uint4*>(w + L.off_total_b);
+  return UPF_OK;
+}
+
+// The mesh from the workspace's evaluated blocks (nact of them, out->n_* their counts).
+int nb_emit(const DSpec& s, const DGrid& g, const NbDims& d, const NbWs& W, float iso, int64_t nact,
+            upf_mesh_buffers* out, uint64_t* d_keys, hipStream_t hs) {
+  if (out->n_vertices > out->cap_vertices || out->n_triangles > out->cap_triangles) return UPF_ERR_CAPACITY;
+  if (out->n_vertices == 0 && out->n_triangles == 0) return UPF_OK;
+  if (!out->positions || !out->indices) return UPF_ERR_NULL;
+  hipLaunchKernelGGL(k_nb_emit, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, W.act, W.map, W.bricks,
+                     W.tabs, W.voff, W.toff, out->positions, out->normals, out->indices, d_keys, out->cap_vertices,
+                     out->cap_triangles);
+  if (out->normals && out->n_vertices) {
+    const dim3 blocks((unsigned)((out->n_vertices + 255) / 256));
+    const auto kernel = spec_ext(s) ? k_nb_normals<true> : k_nb_normals<false>;
+    hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, hs, s, out->positions, out->n_vertices, out->normals);
+  }
+  UPF_LAUNCH_CHECK();
+  return UPF_OK;
+}
+
 }  // namespace upf
 
 using namespace upf;
@@ -469,51 +527,33 @@ int upf_nb_extract(const upf_field_spec* spec, const upf_grid* grid, float iso, 
   if (st || (st = to_device(grid, &g)) || (st = nb_dims(g, &d))) return st;
   *stats = upf_nb_stats{};
   stats->blocks = d.blocks;
-  // the largest active-block capacity this workspace holds
-  const NbLayout L0 = nb_layout(d, 0);
-  if (!d_ws || ws_bytes < L0.bytes) return UPF_ERR_WORKSPACE;
-  const size_t per = 6 * (size_t)kBrick + 12;
-  int64_t cap = std::min<int64_t>(d.blocks, (int64_t)((ws_bytes - L0.bytes) / per));
-  while (cap > 0 && nb_layout(d, cap).bytes > ws_bytes) cap--;
-  const NbLayout L = nb_layout(d, cap);
-  char* w = static_cast<char*>(d_ws);
-  float* coarse = reinterpret_cast<float*>(w + L.off_coarse);
-  uint32_t* counts = reinterpret_cast<uint32_t*>(w + L.off_counts);
-  uint4* tiles = reinterpret_cast<uint4*>(w + L.off_tiles);
-  uint4* total_a = reinterpret_cast<uint4*>(w + L.off_total_a);
-  uint2* act = reinterpret_cast<uint2*>(w + L.off_act);
-  int32_t* map = reinterpret_cast<int32_t*>(w + L.off_map);
-  float* bricks = reinterpret_cast<float*>(w + L.off_bricks);
-  uint16_t* tabs = reinterpret_cast<uint16_t*>(w + L.off_tabs);
-  uint32_t* bcounts = reinterpret_cast<uint32_t*>(w + L.off_bcounts);
-  uint32_t* voff = reinterpret_cast<uint32_t*>(w + L.off_voff);
-  uint32_t* toff = reinterpret_cast<uint32_t*>(w + L.off_toff);
-  uint4* total_b = reinterpret_cast<uint4*>(w + L.off_total_b);
+  NbWs W;
+  if ((st = nb_workspace(d, d_ws, ws_bytes, &W))) return st;
   hipStream_t hs = as_stream(stream);
 
   const auto nblk = [](int64_t n) { return dim3((unsigned)((n + 255) / 256)); };
   const bool modes = spec_ext(s);
-  if (modes) hipLaunchKernelGGL(k_nb_coarse<true>, nblk(L.coarse), dim3(256), 0, hs, s, g, d, coarse);
-  else hipLaunchKernelGGL(k_nb_coarse<false>, nblk(L.coarse), dim3(256), 0, hs, s, g, d, coarse);
-  hipLaunchKernelGGL(k_nb_activity, nblk(d.blocks), dim3(256), 0, hs, coarse, d, iso, band, counts);
+  if (modes) hipLaunchKernelGGL(k_nb_coarse<true>, nblk(W.n_coarse), dim3(256), 0, hs, s, g, d, W.coarse);
+  else hipLaunchKernelGGL(k_nb_coarse<false>, nblk(W.n_coarse), dim3(256), 0, hs, s, g, d, W.coarse);
+  hipLaunchKernelGGL(k_nb_activity, nblk(d.blocks), dim3(256), 0, hs, W.coarse, d, iso, band, W.counts);
   UPF_LAUNCH_CHECK();
-  if ((st = mc_scan_launch(counts, d.blocks, tiles, total_a, nullptr, act, nullptr, hs, kScanMc))) return st;
-  hipLaunchKernelGGL(k_nb_fill_i32, nblk(d.blocks), dim3(256), 0, hs, map, d.blocks, -1);
-  hipLaunchKernelGGL(k_nb_fill_i32, dim3(1), dim3(256), 0, hs, reinterpret_cast<int32_t*>(total_b), (int64_t)8, 0);
+  if ((st = mc_scan_launch(W.counts, d.blocks, W.tiles, W.total_a, nullptr, W.act, nullptr, hs, kScanMc))) return st;
+  hipLaunchKernelGGL(k_nb_fill_i32, nblk(d.blocks), dim3(256), 0, hs, W.map, d.blocks, -1);
+  hipLaunchKernelGGL(k_nb_fill_i32, dim3(1), dim3(256), 0, hs, reinterpret_cast<int32_t*>(W.total_b), (int64_t)8, 0);
   UPF_LAUNCH_CHECK();
   uint4 ha;
-  UPF_HIP_CHECK(hipMemcpyAsync(&ha, total_a, sizeof(uint4), hipMemcpyDeviceToHost, hs));
+  UPF_HIP_CHECK(hipMemcpyAsync(&ha, W.total_a, sizeof(uint4), hipMemcpyDeviceToHost, hs));
   UPF_HIP_CHECK(hipStreamSynchronize(hs));
   const int64_t nact = ha.z;
   stats->active_blocks = nact;
-  if (nact > cap) return UPF_ERR_WORKSPACE;
+  if (nact > W.cap) return UPF_ERR_WORKSPACE;
   out->n_vertices = out->n_triangles = 0;
   if (nact == 0) return UPF_OK;
 
-  hipLaunchKernelGGL(k_nb_map, nblk(nact), dim3(256), 0, hs, act, nact, map);
+  hipLaunchKernelGGL(k_nb_map, nblk(nact), dim3(256), 0, hs, W.act, nact, W.map);
   if (modes)
-    hipLaunchKernelGGL(k_nb_fine<true>, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, act, map, bricks,
-                       tabs, bcounts, reinterpret_cast<uint32_t*>(total_b + 1), 0);
+    hipLaunchKernelGGL(k_nb_fine<true>, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, W.act, W.map, W.bricks,
+                       W.tabs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), 0);
   else {
     int oct_max = 1;  // octaves of the largest gradient / value layer (the brick rows' table)
     for (int l = 0; l < s.n_layers; l++)
@@ -521,16 +561,16 @@ int upf_nb_extract(const upf_field_spec* spec, const upf_grid* grid, float iso, 
         oct_max = std::max(oct_max, s.L[l].fractal == UPF_FRACTAL_NONE ? 1 : s.L[l].octaves);
     const size_t lds = sizeof(float4) * 4 * 2 * kBrickRows * kBrickGroups * oct_max;
     if (spec_composed(s))
-      hipLaunchKernelGGL((k_nb_fine<false, true>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, act,
-                         map, bricks, tabs, bcounts, reinterpret_cast<uint32_t*>(total_b + 1), oct_max);
+      hipLaunchKernelGGL((k_nb_fine<false, true>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, W.act,
+                         W.map, W.bricks, W.tabs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
     else
-      hipLaunchKernelGGL((k_nb_fine<false, false>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, act,
-                         map, bricks, tabs, bcounts, reinterpret_cast<uint32_t*>(total_b + 1), oct_max);
+      hipLaunchKernelGGL((k_nb_fine<false, false>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, W.act,
+                         W.map, W.bricks, W.tabs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
   }
   UPF_LAUNCH_CHECK();
-  if ((st = mc_scan_launch(bcounts, nact, tiles, total_b, voff, nullptr, toff, hs, kScanBlocks))) return st;
+  if ((st = mc_scan_launch(W.bcounts, nact, W.tiles, W.total_b, W.voff, nullptr, W.toff, hs, kScanBlocks))) return st;
   uint4 hb[2];
-  UPF_HIP_CHECK(hipMemcpyAsync(hb, total_b, 2 * sizeof(uint4), hipMemcpyDeviceToHost, hs));
+  UPF_HIP_CHECK(hipMemcpyAsync(hb, W.total_b, 2 * sizeof(uint4), hipMemcpyDeviceToHost, hs));
   UPF_HIP_CHECK(hipStreamSynchronize(hs));
   stats->n_vertices = hb[0].x;
   stats->n_triangles = hb[0].y;
@@ -538,22 +578,25 @@ int upf_nb_extract(const upf_field_spec* spec, const upf_grid* grid, float iso, 
   out->n_vertices = hb[0].x;
   out->n_triangles = hb[0].y;
   if (stats->unresolved) return UPF_ERR_BAND;
-  if (out->n_vertices > out->cap_vertices || out->n_triangles > out->cap_triangles) return UPF_ERR_CAPACITY;
-  if (out->n_vertices == 0 && out->n_triangles == 0) return UPF_OK;
-  if (!out->positions || !out->indices) return UPF_ERR_NULL;
-  hipLaunchKernelGGL(k_nb_emit, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, act, map, bricks, tabs,
-                     voff, toff, out->positions, out->normals, out->indices, d_keys, out->cap_vertices,
-                     out->cap_triangles);
-  if (out->normals && out->n_vertices) {
-    if (modes)
-      hipLaunchKernelGGL(k_nb_normals<true>, nblk(out->n_vertices), dim3(256), 0, hs, s, out->positions,
-                         out->n_vertices, out->normals);
-    else
-      hipLaunchKernelGGL(k_nb_normals<false>, nblk(out->n_vertices), dim3(256), 0, hs, s, out->positions,
-                         out->n_vertices, out->normals);
-  }
-  UPF_LAUNCH_CHECK();
-  return UPF_OK;
+  return nb_emit(s, g, d, W, iso, nact, out, d_keys, hs);
+}
+
+int upf_nb_emit(const upf_field_spec* spec, const upf_grid* grid, float iso, upf_mesh_buffers* out, uint64_t* d_keys,
+                void* d_ws, size_t ws_bytes, const upf_nb_stats* stats, void* stream) {
+  if (!out || !stats) return UPF_ERR_NULL;
+  if (!std::isfinite(iso)) return UPF_ERR_INVALID_VALUE;
+  DSpec s;
+  DGrid g;
+  NbDims d;
+  int st = to_device(spec, &s);
+  if (st || (st = to_device(grid, &g)) || (st = nb_dims(g, &d))) return st;
+  NbWs W;
+  if ((st = nb_workspace(d, d_ws, ws_bytes, &W))) return st;
+  if (stats->active_blocks < 0 || stats->active_blocks > W.cap) return UPF_ERR_WORKSPACE;
+  if (stats->unresolved) return UPF_ERR_BAND;
+  out->n_vertices = stats->n_vertices;
+  out->n_triangles = stats->n_triangles;
+  return nb_emit(s, g, d, W, iso, stats->active_blocks, out, d_keys, as_stream(stream));
 }
 
 }  // extern "C"
