@@ -1,0 +1,63 @@
+"""Grids of many rows are evaluated in bands of eight rows, smaller ones two rows at a time:
+the same values.  A large grid is compared with its planes evaluated a few at a time, over
+ragged sides, all layer kinds and blends, spacings at which a wave spans few cells, more
+columns than a band's share and more than fit at all, and bands over several cells."""
+import pytest
+
+from unnatural_planets_amd import spec as S
+
+pytestmark = pytest.mark.gpu
+
+# the fewest workgroups that take the bands, ragged rows and row ends, one short row each
+DIMS = [(64, 32, 1024), (65, 37, 300), (3, 9, 1030), (130, 2, 400), (257, 66, 90)]
+
+
+def _layers(kind):
+    if kind == "blends":
+        return [S.layer("gradient", "ridged", 6, 0.002, 2.1, -0.4, 3.0, 7), S.layer("value", "none", 1, 0.004, weight=0.5, seed=9, blend="mask"),
+                S.layer("cellular", "fbm", 3, 0.001, weight=2.0, seed=11, jitter=0.8, blend="lerp"),
+                S.layer("value", "fbm", 3, 0.003, weight=1.5, seed=13)]
+    if kind == "cells":
+        return [S.layer("cellular", "ridged", 2, 0.003, weight=2.0, seed=11), S.layer("cellular", "none", 1, 0.0625, weight=1.0, seed=12)]
+    if kind == "wide":
+        return [S.layer("gradient", "fbm", 3, 0.12, weight=2.0, seed=21), S.layer("value", "fbm", 2, 0.9, weight=1.0, seed=22)]
+    return [S.layer("simplex", "fbm", 3, 0.002, weight=1.5, seed=13)]
+
+
+def _grid(dims, spacing, k0=0, n=None):
+    """The grid, or n of its planes from plane k0 on."""
+    g = S.Grid()
+    for a in range(3):
+        g.dims[a] = dims[a]
+        g.spacing[a] = spacing * (1.0, 1.5, 0.5)[a]
+        g.origin[a] = -round(0.5 * dims[a]) * g.spacing[a] + (11.0, -896.0, 256.0)[a]
+    if n:
+        g.dims[2] = n
+        g.origin[2] += k0 * g.spacing[2]  # exact: multiples of an eighth
+    return g
+
+
+@pytest.mark.parametrize("dims", DIMS)
+@pytest.mark.parametrize("spacing", [0.5, 8.0, 9.5, 61.0])
+@pytest.mark.parametrize("kind", ["blends", "cells", "wide", "simplex"])
+@pytest.mark.parametrize("shape,params,compose", [("torus", (1200.0, 450.0), "land"), ("pipe", (), "navigation"), ("none", (), "elevation_raw"),
+                                                  ("hemispheres", (), "water"), ("sphere", (900.0,), "elevation")])
+def test_bands_are_rows(upf, shape, params, compose, kind, spacing, dims):
+    import torch
+    s = S.field_spec(shape, params, _layers(kind), compose, 0.1)
+    whole = upf.field_eval_grid(s, _grid(dims, spacing))
+    assert torch.isfinite(whole).all()
+    for k in range(0, dims[2], 30):
+        k = min(k, dims[2] - 30)
+        part = upf.field_eval_grid(s, _grid(dims, spacing, k, 30))
+        assert torch.equal(whole[k:k + 30], part)
+
+
+def test_signs_and_mesh(upf):
+    """The sign words that the band kernel writes give the mesh of the stored field."""
+    import torch
+    s, g = S.spec_torus_ridged_voronoi(8), S.grid_torus(133)
+    f, ws, nv, nt = upf.field_mesh_count(s, g)
+    a = upf.mc_emit_counted(f, g, 0.0, ws, nv, nt)
+    b = upf.mc_extract(f, g)
+    assert nv > 0 and torch.equal(a.positions, b.positions) and torch.equal(a.indices, b.indices)

@@ -13,6 +13,7 @@
 #include "upf_device_row.hpp"
 #include "upf_device_row_grad.hpp"
 #include "upf_device_tilex.hpp"
+#include "upf_device_band.hpp"
 #include "upf_internal.hpp"
 
 namespace upf {
@@ -56,9 +57,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 8
 // the last node so that all 64 lanes take part in the shared lattice work, rows past the
 // end of the plane repeat its last row, and only real nodes are stored.  A workgroup
 // covers 64 x nodes of kRowWaves row groups.
-// Two rows: four rows per wave would share more (the x part over 4 rows) but measured
-// 3.5 ms at the same workload: the fully unrolled 4-row layers spill (400-600 B of
-// scratch at 80 to 128 VGPRs).
+// Two rows, the octaves unrolled (four rows spill).  Grids with rows to spare run in bands of
+// eight, k_eval_grid_band: this form is for small ones, and decides per wave whether a layer
+// fits LDS.
 constexpr int kRowsPerWave = 2;
 constexpr int kRowWaves = 4;
 static_assert(kRowsPerWave <= kRowMaxRows, "the per-octave table holds kRowMaxRows rows");
@@ -94,6 +95,42 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
   const RowCtx c = make_row_ctx(s_slice[wv], s_gtab, s_oct[wv], lane);
   float v[R];
   row_field<R, COMPOSED>(c, s, x, y, z, v);
+  const int i = (int)blockIdx.x * kGridBX + lane_of(c);  // recomputed: not live across the layers
+  const bool valid = i < g.n[0];
+  const size_t row0 = ((size_t)k * g.n[1] + j) * g.n[0];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+    if (r < rows && valid) out[row0 + (size_t)r * g.n[0] + i] = v[r];
+  if (S) {
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if (r < rows) write_signs(S, g, blockIdx.x, j + r, k, valid, v[r], iso);
+  }
+}
+
+// Bands of kBandRows rows (upf_device_band.hpp), the same values as k_eval_grid_row.  512^3
+// torus at 7 waves a SIMD 863 us, at 6 909, at 8 (64 registers, spills) 928.
+template <bool COMPOSED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_eval_grid_band(
+    const DSpec s, const DGrid g, float* __restrict__ out, uint64_t* __restrict__ S, float iso) {
+  constexpr int R = kBandRows;
+  __shared__ float4 s_slice[kRowWaves][kRowSlice];
+  __shared__ float4 s_gtab[16];
+  if (threadIdx.y == 0 && threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+  __syncthreads();
+  const int lane = threadIdx.x;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int j = (blockIdx.y * kRowWaves + wv) * R;
+  const int k = blockIdx.z;
+  if (j >= g.n[1]) return;
+  const int rows = min(R, g.n[1] - j);  // real rows of this wave
+  const int ic = min((int)blockIdx.x * kGridBX + lane, g.n[0] - 1);
+  const float x = node_coord(g.o[0], g.s[0], ic);
+  const float yl = node_coord(g.o[1], g.s[1], j + min(lane & (R - 1), rows - 1));
+  const float z = node_coord(g.o[2], g.s[2], k);
+  const RowCtx c = make_row_ctx(s_slice[wv], s_gtab, nullptr, lane);
+  float v[R];
+  band_field<R, COMPOSED>(c, s, x, yl, z, v);
   const int i = (int)blockIdx.x * kGridBX + lane_of(c);  // recomputed: not live across the layers
   const bool valid = i < g.n[0];
   const size_t row0 = ((size_t)k * g.n[1] + j) * g.n[0];
@@ -310,6 +347,41 @@ void exact_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, f
   else tilex_launch<1>(s, g, d_field, S, iso, stream);
 }
 
+// Whether every wave of a grid evaluates every layer of the spec in LDS, as columns or cells
+// (no simplex, and the octaves' spans over 64 nodes fit).  The bound covers the rounding of
+// the nodes' coordinates, so no wave needs more; near it the two-row form decides per wave.
+bool band_fits(const DSpec& s, const DGrid& g) {
+  if (s.compose != UPF_COMPOSE_LAND && s.compose != UPF_COMPOSE_NAVIGATION && s.compose != UPF_COMPOSE_ELEVATION_RAW)
+    return true;  // no layer is read
+  const double step = fabs((double)g.s[0]);
+  const double reach = fabs((double)g.o[0]) + step * g.n[0];
+  for (int l = 0; l < s.n_layers; l++) {
+    const DLayer& L = s.L[l];
+    if (L.noise == UPF_NOISE_SIMPLEX) return false;
+    double columns = 0.0;
+    const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
+    if (L.noise == UPF_NOISE_CELLULAR && 72 * oct > kRowSlice2) return false;  // per lane in rows
+    for (int k = 0; k < oct; k++) {
+      const double f = fabs((double)L.freq[k]);
+      const double span = f * (63.0 * step + reach * 0x1p-21);  // cells from end to end
+      if (L.noise == UPF_NOISE_CELLULAR && !(span <= 3.9)) return false;
+      columns += span + 3.0;
+    }
+    if (L.noise != UPF_NOISE_CELLULAR && !(columns <= kRowSlice2)) return false;
+  }
+  return true;
+}
+
+// Bands of eight rows take a quarter of the two-row form's workgroups, which they need four
+// to a CU of: 5 octaves on a torus, two rows against eight, 64^3 (128 workgroups) 10.0 / 12.2
+// us, 96^3 14.1 / 16.8, 110^3 (880) 17.2 / 16.7, 128^3 19.5 / 15.3, 256^3 99 / 55.
+constexpr int kBandBlocks = 1024;
+
+int64_t band_blocks(const DGrid& g) {
+  constexpr int rows_per_block = kBandRows * kRowWaves;
+  return (int64_t)((g.n[0] + kGridBX - 1) / kGridBX) * ((g.n[1] + rows_per_block - 1) / rows_per_block) * g.n[2];
+}
+
 int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int variant, uint64_t* S, float iso,
                       hipStream_t stream) {
   if (variant < 0 || variant > UPF_EVAL_PER_LANE) return UPF_ERR_BAD_SPEC;
@@ -317,6 +389,11 @@ int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int varian
     lanes_launch(s, g, d_field, S, iso, stream);
   } else if (spec_ext(s)) {  // the row form covers the layer stack and the common shapes
     exact_launch(s, g, d_field, S, iso, stream);
+  } else if (band_blocks(g) >= kBandBlocks && band_fits(s, g)) {
+    constexpr int rows_per_block = kBandRows * kRowWaves;
+    const dim3 blocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + rows_per_block - 1) / rows_per_block, g.n[2]);
+    const auto kernel = spec_composed(s) ? k_eval_grid_band<true> : k_eval_grid_band<false>;
+    hipLaunchKernelGGL(kernel, blocks, dim3(kGridBX, kRowWaves, 1), 0, stream, s, g, d_field, S, iso);
   } else {
     constexpr int rows_per_block = kRowsPerWave * kRowWaves;
     const dim3 rblocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + rows_per_block - 1) / rows_per_block, g.n[2]);
