@@ -8,8 +8,8 @@ from unnatural_planets_amd import spec as S
 
 pytestmark = pytest.mark.gpu
 
-# the fewest workgroups that take the bands, ragged rows and row ends, one short row each
-DIMS = [(64, 32, 1024), (65, 37, 300), (3, 9, 1030), (130, 2, 400), (257, 66, 90)]
+# the fewest bands, ragged rows and row ends, one band a plane, too few rows for bands
+DIMS = [(64, 32, 1024), (65, 37, 300), (3, 9, 1030), (130, 5, 700), (130, 4, 700), (257, 66, 90)]
 
 
 def _layers(kind):
@@ -35,6 +35,35 @@ def _grid(dims, spacing, k0=0, n=None):
         g.dims[2] = n
         g.origin[2] += k0 * g.spacing[2]  # exact: multiples of an eighth
     return g
+
+
+@pytest.mark.parametrize("variant", ["rows", "lanes"])
+@pytest.mark.parametrize("first", ["bands", "pairs"])
+def test_batch_of_both_kinds(upf, first, variant):
+    """Chunks in bands between chunks in row pairs (too few rows, an octave too fine for the
+    spacing), small ones of several a workgroup: each as its own grid."""
+    import torch
+    from unnatural_planets_amd.batch import Batch
+    sizes = [((65, 37, 300), 8.0, "blends"), ((9, 7, 5), 8.0, "blends"), ((130, 4, 70), 8.0, "blends"), ((3, 9, 530), 8.0, "cells"),
+             ((2, 2, 2), 8.0, "blends"), ((2, 6, 2), 8.0, "wide"), ((64, 65, 66), 61.0, "wide"), ((70, 31, 90), 8.0, "simplex"),
+             ((5, 5, 5), 0.5, "cells"), ((128, 64, 250), 0.5, "wide")]
+    if first == "pairs":
+        sizes = sizes[::-1]
+    chunks = (S.Chunk * len(sizes))()
+    for c, (dims, spacing, kind) in zip(chunks, sizes):
+        c.spec = S.field_spec("torus", (1200.0, 450.0), _layers(kind), "land", 0.1)
+        c.grid = _grid(dims, spacing)
+        c.iso = 900.0
+    v = upf.EVAL_ROWS if variant == "rows" else upf.EVAL_PER_LANE
+    b = Batch(chunks, S.BatchOpts(v, 0, 0, 0))
+    b.size_outputs()
+    b.run()
+    table = b.mesh_table()
+    for i, c in enumerate(chunks):
+        f = upf.field_eval_grid(c.spec, c.grid, variant=v)
+        assert torch.equal(b.field_of(i), f), sizes[i]
+        m, bm = upf.mc_extract(f, c.grid, 900.0), b.mesh_of(i, table)
+        assert torch.equal(bm.indices, m.indices) and torch.equal(bm.positions, m.positions), sizes[i]
 
 
 @pytest.mark.parametrize("dims", DIMS)

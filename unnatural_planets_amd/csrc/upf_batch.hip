@@ -3,8 +3,8 @@
 // sources/generator.cpp:159).
 //
 // Work items, enumerated chunk after chunk:
-//   field     64 x nodes of a pair of grid rows            (chunk, xb, j / 2, k), which
-//             also stores the rows' sign words: one item per wave over all chunks' items
+//   field     64 x nodes of a band of eight grid rows or of a pair (chunk, xb, band, k),
+//             which also stores the rows' sign words: one item per wave over all chunks'
 //   classify  one marching-cubes group per lane, from the sign words alone
 //   emit      packed passes over the active groups of the concatenated scan, on a
 //             fixed grid
@@ -19,7 +19,7 @@
 #include <new>
 #include <vector>
 
-#include "upf_device_row.hpp"
+#include "upf_device_band.hpp"
 #include "upf_internal.hpp"
 #include "upf_mc.hpp"
 
@@ -35,28 +35,33 @@ struct BChunk {
   int32_t gx;          // 64-node row segments per row
   int64_t node_off;    // first field value of the chunk
   int64_t group_off;   // first marching-cubes group of the chunk
-  int64_t row_off;     // first field item (row pairs)
+  int64_t item_off[2]; // first field item of the pairs, of the bands: a chunk has one kind
 };
 
-// chunk holding item r of a list whose per-chunk starts are at member `off`
-template <int64_t BChunk::*OFF>
+// chunk holding marching-cubes group r
 __device__ __forceinline__ int find_chunk(const BChunk* __restrict__ ch, int n, int64_t r) {
   int lo = 0, hi = n - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (ch[mid].*OFF <= r) lo = mid;
+    if (ch[mid].group_off <= r) lo = mid;
     else hi = mid - 1;
   }
   return lo;
 }
 
-// One field item: nodes xb * 64 + lane of rows 2 jp and 2 jp + 1 (when it exists) of
-// layer k of chunk C, their values into the chunk's field and their sign words into S.
+// Rows of an item of either list, and its item's rows of a grid.
+constexpr int kItemRows[2] = {2, kBandRows};
+
+__host__ __device__ __forceinline__ int item_rows(const DGrid& g, int list) {
+  return (g.n[1] + kItemRows[list] - 1) / kItemRows[list];
+}
+
+// A row pair: nodes xb * 64 + lane of rows j and j + 1 (when it exists) of layer k of
+// chunk C, their values into the chunk's field and their sign words into S.
 template <int VARIANT, bool EXT, bool COMPOSED>
-__device__ __forceinline__ void batch_field_item(const RowCtx& ctx, const BChunk& C, int xb, int jp, int k,
+__device__ __forceinline__ void batch_field_pair(const RowCtx& ctx, const BChunk& C, int xb, int j, int k,
                                                  float* __restrict__ field, uint64_t* __restrict__ S) {
   const int lane = threadIdx.x & 63;
-  const int j = 2 * jp;
   const bool two = j + 1 < C.grid.n[1];
   const int ic = min(xb * 64 + lane, C.grid.n[0] - 1);
   const float x = node_coord(C.grid.o[0], C.grid.s[0], ic);
@@ -95,21 +100,80 @@ __device__ __forceinline__ void batch_field_item(const RowCtx& ctx, const BChunk
   }
 }
 
+// A band (upf_device_band.hpp): the same of kBandRows rows from row j on, as
+// k_eval_grid_band's waves.
+template <bool COMPOSED>
+__device__ __forceinline__ void batch_field_band(const RowCtx& ctx, const BChunk& C, int xb, int j, int k,
+                                                 float* __restrict__ field, uint64_t* __restrict__ S) {
+  constexpr int R = kBandRows;
+  const int lane = threadIdx.x & 63;
+  const int rows = min(R, C.grid.n[1] - j);
+  const int ic = min(xb * 64 + lane, C.grid.n[0] - 1);
+  const float x = node_coord(C.grid.o[0], C.grid.s[0], ic);
+  const float yl = node_coord(C.grid.o[1], C.grid.s[1], j + min(lane & (R - 1), rows - 1));
+  const float z = node_coord(C.grid.o[2], C.grid.s[2], k);
+  float v[R];
+  band_field<R, COMPOSED>(ctx, C.spec, x, yl, z, v);
+  const int in = xb * 64 + lane_of(ctx);  // recomputed: not live across the layers
+  const bool valid = in < C.grid.n[0];
+  const int64_t o = C.node_off + ((int64_t)k * C.grid.n[1] + j) * C.grid.n[0] + in;
+  const int64_t w = C.group_off + ((int64_t)k * C.grid.n[1] + j) * C.gx + xb;
+#pragma unroll
+  for (int r = 0; r < R; r++) {
+    if (r >= rows) break;
+    if (valid) field[o + (int64_t)r * C.grid.n[0]] = v[r];
+    const uint64_t m = ballot64(valid && v[r] < C.iso);
+    if (lane == 0) S[w + (int64_t)r * C.gx] = m;
+  }
+}
+
+// Item r of a list: its chunk, segment, row (of items) and plane.  A workgroup takes 4
+// consecutive items; st holds its first item's chunk, segment, row and plane (16 bits
+// each), from which a wave steps to its own item with carries.  An item in a later chunk
+// than the first (chunks of tiny grids hold fewer than 4 items, those of the other list
+// none) walks on to its chunk and is decoded by division (two 32-bit divisions per item
+// cost ~50 VALU instructions).
+struct BItem {
+  int c, xb, row, k;
+};
+
+template <int LIST>
+__device__ __forceinline__ BItem batch_item(const BChunk* __restrict__ ch, int n_chunks, uint64_t st, int64_t r, int wave) {
+  int c = (int)(st & 0xFFFFu);
+  int xb = (int)((st >> 16) & 0xFFFFu), row = (int)((st >> 32) & 0xFFFFu), k = (int)(st >> 48);
+  if (c + 1 < n_chunks && ch[c + 1].item_off[LIST] <= r) {
+    do c++; while (c + 1 < n_chunks && ch[c + 1].item_off[LIST] <= r);
+    c = uniform(c);
+    const BChunk& C = ch[c];
+    const uint32_t local = (uint32_t)(r - C.item_off[LIST]);  // < 2^31: a chunk's groups fit 31 bits
+    const uint32_t rows = (uint32_t)item_rows(C.grid, LIST), rest = local / (uint32_t)C.gx;
+    xb = (int)(local % (uint32_t)C.gx);
+    row = (int)(rest % rows);
+    k = (int)(rest / rows);
+  } else {
+    const BChunk& C = ch[c];
+    const int rows = item_rows(C.grid, LIST);
+    for (int w = 0; w < wave; w++)
+      if (++xb == C.gx) {
+        xb = 0;
+        if (++row == rows) {
+          row = 0;
+          k++;
+        }
+      }
+  }
+  return {uniform(c), uniform(xb), uniform(row), uniform(k)};
+}
+
 // The field pass: one field item per wave over all chunks' items, as the single-grid
-// kernels run.  A workgroup takes 4 consecutive items; blk_start[workgroup] holds its
-// first item's chunk, segment, row pair and plane (16 bits each), from which a wave
-// steps to its own item with carries.  An item in a later chunk than the first (chunks
-// of tiny grids hold fewer than 4 items, empty ones none) walks on to its chunk and is
-// decoded by division (two 32-bit divisions per item cost ~50 VALU instructions, ~9% of
-// an item of the 64-chunk batch).  A
-// persistent loop of blocks_per_cu workgroups per CU striding over spans of items ran
-// the row form at 1.06-1.08 ms on the 17 192^3 chunks of the 64-chunk batch against
-// 0.83 ms for the single-grid kernel over the same chunks one by one (20 B per lane
-// spilled in the loop); this launch takes the 64-chunk batch's row-form pass from 1.33
-// to 1.09 ms and its per-lane form from 2.52 to 2.23 ms.  Seven waves per SIMD as the
-// single-grid row kernel, six for the per-lane elevation modes and further shapes.
-template <int VARIANT, bool EXT, bool COMPOSED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 7))) void k_batch_field_items(
+// kernels run.  A persistent loop of blocks_per_cu workgroups per CU striding over spans
+// of items ran the row form at 1.06-1.08 ms on the 17 192^3 chunks of the 64-chunk batch
+// against 0.83 ms for the single-grid kernel over the same chunks one by one (20 B per
+// lane spilled in the loop).  Seven waves per SIMD as the single-grid row kernel, six for
+// the per-lane elevation modes and further shapes.  The per-lane form also takes the list
+// of bands, a row pair of each band per plane of workgroups.
+template <int VARIANT, bool EXT, bool COMPOSED, int LIST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 7))) void k_batch_field_pairs(
     const BChunk* __restrict__ ch, int n_chunks, const uint64_t* __restrict__ blk_start, int64_t n_items,
     float* __restrict__ field, uint64_t* __restrict__ S) {
   __shared__ float4 s_slice[4][kRowSlice];
@@ -120,41 +184,37 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 7
   const int wave = uniform(threadIdx.x >> 6);
   const int64_t r = (int64_t)blockIdx.x * 4 + wave;
   if (r >= n_items) return;  // whole waves
-  const uint64_t st = blk_start[blockIdx.x];
-  int c = (int)(st & 0xFFFFu);
-  int xb = (int)((st >> 16) & 0xFFFFu), jp = (int)((st >> 32) & 0xFFFFu), k = (int)(st >> 48);
-  if (c + 1 < n_chunks && ch[c + 1].row_off <= r) {
-    do c++; while (c + 1 < n_chunks && ch[c + 1].row_off <= r);
-    c = uniform(c);
-    const BChunk& C = ch[c];
-    const uint32_t local = (uint32_t)(r - C.row_off);  // < 2^31: a chunk's groups fit 31 bits
-    const uint32_t pairs = (uint32_t)(C.grid.n[1] + 1) / 2, rest = local / (uint32_t)C.gx;
-    xb = (int)(local % (uint32_t)C.gx);
-    jp = (int)(rest % pairs);
-    k = (int)(rest / pairs);
-  } else {
-    const BChunk& C = ch[c];
-    const int pairs = (C.grid.n[1] + 1) / 2;
-    for (int w = 0; w < wave; w++)
-      if (++xb == C.gx) {
-        xb = 0;
-        if (++jp == pairs) {
-          jp = 0;
-          k++;
-        }
-      }
-  }
-  c = uniform(c);
+  const BItem it = batch_item<LIST>(ch, n_chunks, blk_start[blockIdx.x], r, wave);
+  const int j = kItemRows[LIST] * it.row + 2 * (int)blockIdx.y;
+  if (j >= ch[it.c].grid.n[1]) return;
   const RowCtx ctx = make_row_ctx(s_slice[wave], s_gtab, s_oct[wave], threadIdx.x & 63);
-  batch_field_item<VARIANT, EXT, COMPOSED>(ctx, ch[c], uniform(xb), uniform(jp), uniform(k), field, S);
+  batch_field_pair<VARIANT, EXT, COMPOSED>(ctx, ch[it.c], it.xb, j, it.k, field, S);
+}
+
+// The list of bands.  64-chunk batch (32^3 to 192^3, 152 M nodes) as a whole, row pairs
+// against bands: 1.33 / 0.84 ms.
+template <bool COMPOSED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_batch_field_bands(
+    const BChunk* __restrict__ ch, int n_chunks, const uint64_t* __restrict__ blk_start, int64_t n_items,
+    float* __restrict__ field, uint64_t* __restrict__ S) {
+  __shared__ float4 s_slice[4][kRowSlice];
+  __shared__ float4 s_gtab[16];
+  if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+  __syncthreads();
+  const int wave = uniform(threadIdx.x >> 6);
+  const int64_t r = (int64_t)blockIdx.x * 4 + wave;
+  if (r >= n_items) return;  // whole waves
+  const BItem it = batch_item<1>(ch, n_chunks, blk_start[blockIdx.x], r, wave);
+  const RowCtx ctx = make_row_ctx(s_slice[wave], s_gtab, nullptr, threadIdx.x & 63);
+  batch_field_band<COMPOSED>(ctx, ch[it.c], it.xb, kBandRows * it.row, it.k, field, S);
 }
 
 // Counts of every group of every chunk (global id g: chunk, then its local group) from
 // the sign words; lanes of one wave may belong to two chunks.  One group per thread: the
 // batch's small chunks have several times the 512^3 grid's mixed cells per group, and
 // their classification passes need the occupancy (four or eight groups per thread with
-// the next group's words loaded ahead and the tile sums written took 67 and 82 us against 50 + 5.6 us for this kernel and the separate
-// tile pass).
+// the next group's words loaded ahead and the tile sums written took 67 and 82 us against
+// 50 + 5.6 us for this kernel and the separate tile pass).
 __global__ __launch_bounds__(256) void k_batch_classify(const BChunk* __restrict__ ch, int n_chunks, int64_t groups,
                                                         const uint64_t* __restrict__ S,
                                                         uint32_t* __restrict__ counts) {
@@ -166,7 +226,7 @@ __global__ __launch_bounds__(256) void k_batch_classify(const BChunk* __restrict
   const bool in = g < groups;
   // the chunk of the workgroup's first group (one search per workgroup), then a short
   // walk per lane: a workgroup's 256 groups rarely cross a chunk boundary
-  int c = uniform(find_chunk<&BChunk::group_off>(ch, n_chunks, (int64_t)blockIdx.x * 256));
+  int c = uniform(find_chunk(ch, n_chunks, (int64_t)blockIdx.x * 256));
   while (c + 1 < n_chunks && ch[c + 1].group_off <= (in ? g : groups - 1)) c++;
   const BChunk& C = ch[c];
   const GroupWords w = load_group_words(S + C.group_off, C.md, g - C.group_off, in);
@@ -204,7 +264,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
   const int64_t per = (n_active + nw - 1) / nw;
   int64_t a = ((int64_t)blockIdx.x * 4 + wave) * per;
   const int64_t a1 = min(a + per, n_active);
-  int c = a < a1 ? uniform(find_chunk<&BChunk::group_off>(ch, n_chunks, (int64_t)(uint32_t)uniform((int)act[a].x))) : 0;
+  int c = a < a1 ? uniform(find_chunk(ch, n_chunks, (int64_t)(uint32_t)uniform((int)act[a].x))) : 0;
   while (a < a1) {
     // the list is sorted, so the chunk only advances
     const int64_t g = (int64_t)(uint32_t)uniform((int)act[a].x);
@@ -230,13 +290,14 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 struct upf_batch {
   std::vector<upf::BChunk> host;
   upf::BChunk* dev = nullptr;
-  uint64_t* blk_start = nullptr;  // first field item of each workgroup of 4: chunk | xb << 16 | jp << 32 | k << 48
-  int64_t item_blocks = 0;
+  // first field item of each workgroup of 4, of the pairs, then of the bands: chunk | xb << 16 | row << 32 | k << 48
+  uint64_t* blk_start = nullptr;
+  int64_t item_blocks[2] = {0, 0};
   int device = 0;
   int n = 0;
   int cus = 256;
   int emit_blocks = 256 * 32;  // k_batch_emit's grid
-  int64_t nodes = 0, groups = 0, rows = 0;
+  int64_t nodes = 0, groups = 0, items[2] = {0, 0};
   bool any_ext = false;  // a chunk with an elevation mode or a further shape: the field runs per lane
   bool any_composed = false;  // a chunk whose shape is a composition (spec_composed)
   upf_batch_opts opts{};
@@ -267,6 +328,15 @@ int upload(upf_batch* b) {
   return UPF_OK;
 }
 
+using FieldKernel = void (*)(const BChunk*, int, const uint64_t*, int64_t, float*, uint64_t*);
+
+FieldKernel field_kernel(int list, bool lanes, bool ext, bool composed) {
+  if (ext) return k_batch_field_pairs<UPF_EVAL_PER_LANE, true, true, 0>;  // no bands then
+  if (lanes) return list ? k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, 1> : k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, 0>;
+  if (list) return composed ? k_batch_field_bands<true> : k_batch_field_bands<false>;
+  return composed ? k_batch_field_pairs<UPF_EVAL_ROWS, false, true, 0> : k_batch_field_pairs<UPF_EVAL_ROWS, false, false, 0>;
+}
+
 int run(upf_batch* b, float* field, void* ws, size_t ws_bytes, float* pos, float* nrm, uint32_t* idx, int64_t cap_v,
         int64_t cap_t, upf_chunk_mesh* meshes, hipStream_t s) {
   if (!field || !ws || !meshes || (cap_v > 0 && !pos) || (cap_t > 0 && !idx)) return UPF_ERR_NULL;
@@ -279,19 +349,14 @@ int run(upf_batch* b, float* field, void* ws, size_t ws_bytes, float* pos, float
   uint2* act = reinterpret_cast<uint2*>(w + b->off_act);
   uint4* tiles = reinterpret_cast<uint4*>(w + b->off_tiles);
   uint4* total = reinterpret_cast<uint4*>(w + b->off_total);
-  const dim3 items((unsigned)b->item_blocks);
-  if (b->any_ext)
-    hipLaunchKernelGGL((k_batch_field_items<UPF_EVAL_PER_LANE, true, true>), items, dim3(256), 0, s, b->dev, b->n,
-                       b->blk_start, b->rows, field, S);
-  else if (b->opts.field_variant == UPF_EVAL_PER_LANE)
-    hipLaunchKernelGGL((k_batch_field_items<UPF_EVAL_PER_LANE, false, true>), items, dim3(256), 0, s, b->dev, b->n,
-                       b->blk_start, b->rows, field, S);
-  else if (b->any_composed)
-    hipLaunchKernelGGL((k_batch_field_items<UPF_EVAL_ROWS, false, true>), items, dim3(256), 0, s, b->dev, b->n,
-                       b->blk_start, b->rows, field, S);
-  else
-    hipLaunchKernelGGL((k_batch_field_items<UPF_EVAL_ROWS, false, false>), items, dim3(256), 0, s, b->dev, b->n,
-                       b->blk_start, b->rows, field, S);
+  for (int list = 0; list < 2; list++) {
+    if (!b->items[list]) continue;
+    const bool lanes = b->any_ext || b->opts.field_variant == UPF_EVAL_PER_LANE;
+    const auto kernel = field_kernel(list, lanes, b->any_ext, b->any_composed);
+    const dim3 blocks((unsigned)b->item_blocks[list], lanes ? kItemRows[list] / 2 : 1);
+    hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, s, b->dev, b->n, b->blk_start + (list ? b->item_blocks[0] : 0),
+                       b->items[list], field, S);
+  }
   hipLaunchKernelGGL(k_batch_classify, dim3((unsigned)((b->groups + 255) / 256)), dim3(256), 0, s, b->dev, b->n,
                      b->groups, S, counts);
   UPF_LAUNCH_CHECK();
@@ -340,10 +405,18 @@ int upf_batch_create(const upf_chunk* chunks, int32_t n_chunks, const upf_batch_
     C.gx = (C.grid.n[0] + 63) / 64;
     C.node_off = b->nodes;
     C.group_off = b->groups;
-    C.row_off = b->rows;
     b->nodes += (int64_t)C.grid.n[0] * C.grid.n[1] * C.grid.n[2];
     b->groups += C.md.groups;
-    b->rows += (int64_t)C.gx * ((C.grid.n[1] + 1) / 2) * C.grid.n[2];
+  }
+  // bands for the chunks that fit them, if there are enough bands to fill the machine (and
+  // no chunk makes the whole batch run per lane)
+  int64_t bands = 0;
+  for (const BChunk& C : b->host)
+    if (band_fits(C.spec, C.grid)) bands += band_items(C.grid);
+  for (BChunk& C : b->host) {
+    const int list = !b->any_ext && bands >= kBandItems && band_fits(C.spec, C.grid);
+    for (int l = 0; l < 2; l++) C.item_off[l] = b->items[l];
+    b->items[list] += (int64_t)C.gx * item_rows(C.grid, list) * C.grid.n[2];
   }
   if (b->groups >= ((int64_t)1 << 31)) { delete b; return UPF_ERR_BAD_GRID; }
   size_t o = 0;
@@ -362,19 +435,21 @@ int upf_batch_create(const upf_chunk* chunks, int32_t n_chunks, const upf_batch_
     return UPF_ERR_HIP;
   }
   {
-    // each workgroup's first field item (chunk, segment, row pair, plane; all < 2^16: at
-    // most 65536 chunks of at most 65535 nodes per axis), for the field kernel
-    b->item_blocks = (b->rows + 3) / 4;
-    if (b->item_blocks >= ((int64_t)1 << 31)) { upf_batch_destroy(b); return UPF_ERR_BAD_GRID; }
-    std::vector<uint64_t> tab((size_t)b->item_blocks);
-    int c = 0;
-    for (int64_t q = 0; q < b->item_blocks; q++) {
-      while (c + 1 < n_chunks && b->host[c + 1].row_off <= 4 * q) c++;
-      const BChunk& C = b->host[c];
-      const int64_t local = 4 * q - C.row_off, pairs = (C.grid.n[1] + 1) / 2;
-      const uint64_t xb = (uint64_t)(local % C.gx), rest = (uint64_t)(local / C.gx);
-      tab[(size_t)q] = (uint64_t)c | xb << 16 | (rest % pairs) << 32 | (rest / pairs) << 48;
+    // each workgroup's first field item (chunk, segment, row, plane; all < 2^16: at most
+    // 65536 chunks of at most 65535 nodes per axis), for the field kernels
+    for (int l = 0; l < 2; l++) {
+      b->item_blocks[l] = (b->items[l] + 3) / 4;
+      if (b->item_blocks[l] >= ((int64_t)1 << 31)) { upf_batch_destroy(b); return UPF_ERR_BAD_GRID; }
     }
+    std::vector<uint64_t> tab((size_t)(b->item_blocks[0] + b->item_blocks[1]));
+    for (int l = 0, c = 0; l < 2; l++, c = 0)
+      for (int64_t q = 0; q < b->item_blocks[l]; q++) {
+        while (c + 1 < n_chunks && b->host[c + 1].item_off[l] <= 4 * q) c++;
+        const BChunk& C = b->host[c];
+        const int64_t local = 4 * q - C.item_off[l], rows = item_rows(C.grid, l);
+        const uint64_t xb = (uint64_t)(local % C.gx), rest = (uint64_t)(local / C.gx);
+        tab[(size_t)(l ? b->item_blocks[0] + q : q)] = (uint64_t)c | xb << 16 | (rest % rows) << 32 | (rest / rows) << 48;
+      }
     if (hipMalloc(&b->blk_start, sizeof(uint64_t) * tab.size()) != hipSuccess ||
         hipMemcpy(b->blk_start, tab.data(), sizeof(uint64_t) * tab.size(), hipMemcpyHostToDevice) != hipSuccess) {
       upf_batch_destroy(b);

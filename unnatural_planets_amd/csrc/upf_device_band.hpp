@@ -16,6 +16,8 @@
 // fiftieth, R = 16 by a fifteenth: spills).
 #pragma once
 
+#include <cmath>
+
 #include "upf_device_row.hpp"
 
 namespace upf {
@@ -23,6 +25,42 @@ namespace upf {
 constexpr int kBandRows = 8;
 constexpr int kBandStride = 56;  // columns per row in LDS: rows 16 banks apart
 static_assert(kBandRows * kBandStride <= kRowSlice2 && UPF_MAX_OCTAVES * kBandStride <= kRowSlice2, "the columns fit the slice");
+
+// Whether every wave of a grid evaluates every layer of the spec in LDS, as columns or cells
+// (no simplex, and the octaves' spans over 64 nodes fit).  The bound covers the rounding of
+// the nodes' coordinates, so no wave needs more; near it the two-row form decides per wave.
+// A grid of four rows or fewer has no use for eight.
+inline bool band_fits(const DSpec& s, const DGrid& g) {
+  if (g.n[1] <= kBandRows / 2) return false;
+  if (s.compose != UPF_COMPOSE_LAND && s.compose != UPF_COMPOSE_NAVIGATION && s.compose != UPF_COMPOSE_ELEVATION_RAW)
+    return true;  // no layer is read
+  const double step = std::fabs((double)g.s[0]);
+  const double reach = std::fabs((double)g.o[0]) + step * g.n[0];
+  for (int l = 0; l < s.n_layers; l++) {
+    const DLayer& L = s.L[l];
+    if (L.noise == UPF_NOISE_SIMPLEX) return false;
+    double columns = 0.0;
+    const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
+    if (L.noise == UPF_NOISE_CELLULAR && 72 * oct > kRowSlice2) return false;  // per lane in rows
+    for (int k = 0; k < oct; k++) {
+      const double f = std::fabs((double)L.freq[k]);
+      const double span = f * (63.0 * step + reach * 0x1p-21);  // cells from end to end
+      if (L.noise == UPF_NOISE_CELLULAR && !(span <= 3.9)) return false;
+      columns += span + 3.0;
+    }
+    if (L.noise != UPF_NOISE_CELLULAR && !(columns <= kRowSlice2)) return false;
+  }
+  return true;
+}
+
+// Bands of eight rows take a quarter of the two-row form's waves, and need 16 to a CU (four
+// workgroups).  5 octaves on a torus, two rows against eight: 64^3 (512 bands) 10.0 / 12.2
+// us, 96^3 14.1 / 16.8, 110^3 (3520) 17.2 / 16.7, 128^3 19.5 / 15.3, 256^3 99 / 55.
+constexpr int64_t kBandItems = 4096;
+
+inline int64_t band_items(const DGrid& g) {
+  return (int64_t)((g.n[0] + 63) / 64) * ((g.n[1] + kBandRows - 1) / kBandRows) * g.n[2];
+}
 
 // Value v of row r's lane.
 __device__ __forceinline__ float band_row(float v, int r) {

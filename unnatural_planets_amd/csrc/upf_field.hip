@@ -347,41 +347,6 @@ void exact_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, f
   else tilex_launch<1>(s, g, d_field, S, iso, stream);
 }
 
-// Whether every wave of a grid evaluates every layer of the spec in LDS, as columns or cells
-// (no simplex, and the octaves' spans over 64 nodes fit).  The bound covers the rounding of
-// the nodes' coordinates, so no wave needs more; near it the two-row form decides per wave.
-bool band_fits(const DSpec& s, const DGrid& g) {
-  if (s.compose != UPF_COMPOSE_LAND && s.compose != UPF_COMPOSE_NAVIGATION && s.compose != UPF_COMPOSE_ELEVATION_RAW)
-    return true;  // no layer is read
-  const double step = fabs((double)g.s[0]);
-  const double reach = fabs((double)g.o[0]) + step * g.n[0];
-  for (int l = 0; l < s.n_layers; l++) {
-    const DLayer& L = s.L[l];
-    if (L.noise == UPF_NOISE_SIMPLEX) return false;
-    double columns = 0.0;
-    const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
-    if (L.noise == UPF_NOISE_CELLULAR && 72 * oct > kRowSlice2) return false;  // per lane in rows
-    for (int k = 0; k < oct; k++) {
-      const double f = fabs((double)L.freq[k]);
-      const double span = f * (63.0 * step + reach * 0x1p-21);  // cells from end to end
-      if (L.noise == UPF_NOISE_CELLULAR && !(span <= 3.9)) return false;
-      columns += span + 3.0;
-    }
-    if (L.noise != UPF_NOISE_CELLULAR && !(columns <= kRowSlice2)) return false;
-  }
-  return true;
-}
-
-// Bands of eight rows take a quarter of the two-row form's workgroups, which they need four
-// to a CU of: 5 octaves on a torus, two rows against eight, 64^3 (128 workgroups) 10.0 / 12.2
-// us, 96^3 14.1 / 16.8, 110^3 (880) 17.2 / 16.7, 128^3 19.5 / 15.3, 256^3 99 / 55.
-constexpr int kBandBlocks = 1024;
-
-int64_t band_blocks(const DGrid& g) {
-  constexpr int rows_per_block = kBandRows * kRowWaves;
-  return (int64_t)((g.n[0] + kGridBX - 1) / kGridBX) * ((g.n[1] + rows_per_block - 1) / rows_per_block) * g.n[2];
-}
-
 int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int variant, uint64_t* S, float iso,
                       hipStream_t stream) {
   if (variant < 0 || variant > UPF_EVAL_PER_LANE) return UPF_ERR_BAD_SPEC;
@@ -389,7 +354,7 @@ int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int varian
     lanes_launch(s, g, d_field, S, iso, stream);
   } else if (spec_ext(s)) {  // the row form covers the layer stack and the common shapes
     exact_launch(s, g, d_field, S, iso, stream);
-  } else if (band_blocks(g) >= kBandBlocks && band_fits(s, g)) {
+  } else if (band_items(g) >= kBandItems && band_fits(s, g)) {
     constexpr int rows_per_block = kBandRows * kRowWaves;
     const dim3 blocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + rows_per_block - 1) / rows_per_block, g.n[2]);
     const auto kernel = spec_composed(s) ? k_eval_grid_band<true> : k_eval_grid_band<false>;
