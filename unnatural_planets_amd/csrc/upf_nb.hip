@@ -10,16 +10,18 @@
 //  coarse    one thread per block corner;
 //  activity  one thread per block: a count word with the active bit; the shared scan
 //            compacts the active blocks, and a dense map block -> active rank follows;
-//  fine      one workgroup per active block: its 9^3 brick of fine nodes into LDS and
-//            HBM, then per node the crossing edges it owns (a node owns its +x/+y/+z
-//            edges; nodes on the block's upper faces belong to the next block except on
-//            the grid's upper boundary) and their exclusive prefix, packed with the
-//            node's crossing bits into one uint16 per node; per block the vertex and
-//            triangle counts;
-//  scan      vertex and triangle bases per active block;
-//  emit      one workgroup per active block: vertices at base + prefix + axis rank,
-//            and triangles whose edge ids come from the owning block's node table (this
-//            block's, or a neighbour's through the dense map);
+//  fine      one workgroup per active block: its 9^3 brick of fine nodes, and from the signs
+//            of its 81 rows of 9 nodes, as bit masks, the crossing edges that each row owns
+//            (a node owns its +x/+y/+z edges; nodes on the block's upper faces belong to the
+//            next block except on the grid's upper boundary), their exclusive prefix and the
+//            block's vertex and triangle counts.  A brick that the surface crosses goes to HBM
+//            with a record per row; one of a single sign (two of three in a band that is
+//            sure to hold the surface) leaves its zero count alone;
+//  scan      vertex and triangle bases per active block, and the list of crossed blocks;
+//  emit      a workgroup per crossed block at a time: its vertices and triangles listed in LDS,
+//            then a thread per vertex (base + prefix + rank) and per triangle corner, whose
+//            edge id comes from the owning row's record (this block's, or a neighbour's
+//            through the dense map);
 //  normals   one thread per vertex: the normalized analytic gradient at the vertex.
 // Vertex positions use the same interpolation as the dense path on the same per-lane
 // node values, so the mesh equals the dense one up to order when the band holds the
@@ -41,10 +43,47 @@ namespace upf {
 constexpr int kB = UPF_NB_BLOCK;          // cells per block edge
 constexpr int kBN = kB + 1;               // nodes per brick edge
 constexpr int kBrick = kBN * kBN * kBN;   // 729 nodes
+constexpr int kRows = kBN * kBN;          // 81 rows (j + 9 k) of 9 nodes
 constexpr int kCells = kB * kB * kB;      // 512 cells
 constexpr int kNbThreads = 256;
 static_assert(kCells == 2 * kNbThreads, "fine/emit give each thread two cells");
-static_assert(kBrick <= 3 * kNbThreads, "fine/emit give each thread at most three brick nodes");
+static_assert(kRows <= kNbThreads, "fine/emit give each row a thread");
+
+// A brick row's record: x = owned vertices of the block before the row | X << 12 | M << 21,
+// y = Y | Z << 9, with M the nodes inside, X / Y / Z the nodes whose +x / +y / +z edge
+// crosses (within the brick, owned or not).
+struct BrickRow {
+  uint32_t m, x, y, z;
+};
+
+// Row t's masks, from the rows' M.
+__device__ __forceinline__ BrickRow brick_row_masks(const uint32_t* s_row, int t) {
+  BrickRow r;
+  r.m = s_row[t];
+  r.x = (r.m ^ (r.m >> 1)) & 0xFFu;
+  r.y = t % kBN < kB ? r.m ^ s_row[t + 1] : 0u;
+  r.z = t < kB * kBN ? r.m ^ s_row[t + kBN] : 0u;
+  return r;
+}
+
+// The nodes of row t that the block owns.
+__device__ __forceinline__ uint32_t owned_nodes(int t, bool lx, bool ly, bool lz) {
+  return (t % kBN < kB || ly) && (t < kB * kBN || lz) ? (lx ? 0x1FFu : 0xFFu) : 0u;
+}
+
+// The block's vertex of node i's edge along axis, from its (owned) row's record.
+__device__ __forceinline__ uint32_t row_vertex(uint2 rec, int i, int axis) {
+  const uint32_t below = (1u << i) - 1u;
+  const uint32_t rank = ((rec.x >> (12 + i)) & (uint32_t)(axis > 0)) + ((rec.y >> i) & (uint32_t)(axis > 1));
+  return (rec.x & 0xFFFu) + (uint32_t)__popc(rec.x & (below << 12)) + (uint32_t)__popc(rec.y & (below | below << 9)) + rank;
+}
+
+// Case code of the cell at the rows' masks shifted to its first node: rows (j, k),
+// (j + 1, k), (j, k + 1), (j + 1, k + 1).
+__device__ __forceinline__ int cell_code(uint32_t m00, uint32_t m10, uint32_t m01, uint32_t m11) {
+  const auto swap = [](uint32_t m) { return ((m & 1u) << 1) | ((m >> 1) & 1u); };
+  return (int)((m00 & 3u) | swap(m10) << 2 | (m01 & 3u) << 4 | swap(m11) << 6);
+}
 
 struct NbDims {
   int bx, by, bz;  // blocks per axis
@@ -127,7 +166,7 @@ template <bool EXT, bool COMPOSED = true>
 __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGrid g, const NbDims d, float iso,
                                                         const uint2* __restrict__ act,
                                                         const int32_t* __restrict__ map, float* __restrict__ bricks,
-                                                        uint16_t* __restrict__ tabs, uint32_t* __restrict__ bcounts,
+                                                        uint2* __restrict__ recs, uint32_t* __restrict__ bcounts,
                                                         uint32_t* __restrict__ unresolved, int oct_max) {
   __shared__ float s_fe[EXT ? kBrick : 1];
   __shared__ float4 s_slice[4][EXT ? 1 : kRowSlice];
@@ -135,8 +174,12 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
   // the (row, octave) tables of the 4 waves, 2 * kBrickRows * kBrickGroups * oct_max float4
   // each (launch-sized: the spec's largest octave count sets the LDS, hence the occupancy)
   extern __shared__ float4 s_oct[];
+  __shared__ uint64_t s_bits[EXT ? 1 : 4 * kBrickGroups];  // signs of the groups of rows
+  __shared__ uint32_t s_row[kRows];                        // and of each row
+  __shared__ int s_crossed;
   __shared__ uint8_t s_ntris[256];  // triangles per case code
   s_ntris[threadIdx.x] = upf_mc_ntris[threadIdx.x];  // read after the barriers below
+  if (threadIdx.x == 0) s_crossed = 0;
   const int64_t a = blockIdx.x;
   const uint32_t b = act[a].x;
   int bx, by, bz;
@@ -144,19 +187,21 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
   const int gi0 = bx * kB, gj0 = by * kB, gk0 = bz * kB;
   const bool lx = bx == d.bx - 1, ly = by == d.by - 1, lz = bz == d.bz - 1;
   float* __restrict__ brick = bricks + a * kBrick;
-  // the brick's values in LDS; the row path stores them over its slices once every wave
-  // has finished with its slice (LDS sets the occupancy here)
-  float* s_f = EXT ? s_fe : reinterpret_cast<float*>(&s_slice[0][0]);
-  static_assert(sizeof(float) * kBrick <= sizeof(float4) * 4 * kRowSlice, "the brick fits the slices");
+  float v[kBrickGroups];  // this lane's nodes (rows)
+  const int t = threadIdx.x;
+  uint32_t mask = 0;  // thread t < kRows: row t's nodes inside
+  bool first;         // whether node 0 is
   if (EXT) {  // elevation modes and further shapes: per node
     for (int n = threadIdx.x; n < kBrick; n += kNbThreads) {
       const int k = n / (kBN * kBN), r = n - k * kBN * kBN;
       const int j = r / kBN, i = r - j * kBN;
-      const float v = field_eval<EXT>(s, node_coord(g.o[0], g.s[0], gi0 + i), node_coord(g.o[1], g.s[1], gj0 + j),
-                                      node_coord(g.o[2], g.s[2], gk0 + k));
-      s_f[n] = v;
-      brick[n] = v;
+      s_fe[n] = field_eval<EXT>(s, node_coord(g.o[0], g.s[0], gi0 + i), node_coord(g.o[1], g.s[1], gj0 + j),
+                                node_coord(g.o[2], g.s[2], gk0 + k));
     }
+    __syncthreads();
+    if (t < kRows)
+      for (int i = 0; i < kBN; i++) mask |= (uint32_t)(s_fe[t * kBN + i] < iso) << i;
+    first = s_fe[0] < iso;
   } else {
     // the brick's 81 rows of 9 nodes (row = j + 9 k) in 12 groups of kBrickRows; wave w
     // takes groups w, w + 4, w + 8 (kBrickGroups of them), its row rho = 7 m + r being
@@ -181,203 +226,186 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
       yy = node_coord(g.o[1], g.s[1], gj0 + jj);
       zz = node_coord(g.o[2], g.s[2], gk0 + kk);
     };
-    float y[kBrickGroups], z[kBrickGroups], v[kBrickGroups];
+    float y[kBrickGroups], z[kBrickGroups];
 #pragma unroll
     for (int m = 0; m < kBrickGroups; m++) yz(kBrickRows * m + rl, y[m], z[m]);
     brick_field<kBrickGroups, COMPOSED>(ctx, s, rl, yz, x, y, z, v);
-    __syncthreads();  // every wave done with its slice
 #pragma unroll
     for (int m = 0; m < kBrickGroups; m++) {
-      const int br = kBrickRows * (wave + 4 * m) + rl;
-      if (node_lane && br < kBN * kBN) {
-        const int n = br * kBN + i;
-        s_f[n] = v[m];
-        brick[n] = v[m];
-      }
+      const bool real = node_lane && kBrickRows * (wave + 4 * m) + rl < kRows;
+      const uint64_t w = ballot64(real && v[m] < iso);
+      if (lane == 0) s_bits[wave + 4 * m] = w;
     }
+    __syncthreads();
+    if (t < kRows) mask = (uint32_t)(s_bits[t / kBrickRows] >> (kBN * (t % kBrickRows))) & 0x1FFu;
+    first = s_bits[0] & 1u;
+  }
+  if (t < kRows) {
+    s_row[t] = mask;
+    if (mask != (first ? 0x1FFu : 0u)) s_crossed = 1;
   }
   __syncthreads();
-
-  // nodes 3t .. 3t+2: crossing bits, owned vertex counts
-  int cnt[3], cross[3], tot = 0;
+  if (!s_crossed) {
+    if (t == 0) bcounts[a] = 0;
+    return;
+  }
+  if (EXT) {
+    for (int n = t; n < kBrick; n += kNbThreads) brick[n] = s_fe[n];
+  } else {
+    const int wave = t >> 6, lane = t & 63;
 #pragma unroll
-  for (int q = 0; q < 3; q++) {
-    const int n = 3 * threadIdx.x + q;
-    cnt[q] = cross[q] = 0;
-    if (n >= kBrick) continue;
-    const int k = n / (kBN * kBN), r = n - k * kBN * kBN;
-    const int j = r / kBN, i = r - j * kBN;
-    const bool in0 = s_f[n] < iso;
-    int c = 0;
-    if (i < kB && (s_f[n + 1] < iso) != in0) c |= 1;
-    if (j < kB && (s_f[n + kBN] < iso) != in0) c |= 2;
-    if (k < kB && (s_f[n + kBN * kBN] < iso) != in0) c |= 4;
-    const int ox = (i == kB && !lx), oy = (j == kB && !ly), oz = (k == kB && !lz);
-    cross[q] = c;
-    if (!(ox | oy | oz)) {
-      cnt[q] = __popc(c);
-    } else if (c) {
-      const int64_t nb = (int64_t)b + ox + (int64_t)oy * d.bx + (int64_t)oz * d.bx * d.by;
-      if (map[nb] < 0) atomicAdd(unresolved, 1u);
+    for (int m = 0; m < kBrickGroups; m++) {
+      const int n = kBrickRows * kBN * (wave + 4 * m) + lane;
+      if (lane < kBrickRows * kBN && n < kBrick) brick[n] = v[m];
     }
-    tot += cnt[q];
-  }
-  int nv;
-  int pre = wg_exclusive_sum(tot, &nv);
-  uint16_t* __restrict__ tab = tabs + a * kBrick;
-#pragma unroll
-  for (int q = 0; q < 3; q++) {
-    const int n = 3 * threadIdx.x + q;
-    if (n < kBrick) tab[n] = (uint16_t)(pre | (cross[q] << 12));
-    pre += cnt[q];
   }
 
-  // cells 2t, 2t+1
-  int nt = 0;
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int c = 2 * threadIdx.x + q;
-    const int i = c & 7, j = (c >> 3) & 7, k = c >> 6;
-    const int n = (k * kBN + j) * kBN + i;
-    const int code = (s_f[n] < iso) | ((s_f[n + 1] < iso) << 1) | ((s_f[n + kBN + 1] < iso) << 2) |
-                     ((s_f[n + kBN] < iso) << 3) | ((s_f[n + kBN * kBN] < iso) << 4) |
-                     ((s_f[n + kBN * kBN + 1] < iso) << 5) | ((s_f[n + kBN * kBN + kBN + 1] < iso) << 6) |
-                     ((s_f[n + kBN * kBN + kBN] < iso) << 7);
-    nt += s_ntris[code];
+  // thread t < 81: row t's crossing edges; all: cells 2t, 2t + 1
+  BrickRow r{0, 0, 0, 0};
+  uint32_t own = 0;
+  if (t < kRows) {
+    r = brick_row_masks(s_row, t);
+    own = owned_nodes(t, lx, ly, lz);
+    if (const uint32_t rest = (r.x | r.y | r.z) & ~own) {  // crossings of other blocks' nodes
+      const int oy = t % kBN == kB && !ly, oz = t >= kB * kBN && !lz;
+      const int64_t nb = (int64_t)b + (int64_t)oy * d.bx + (int64_t)oz * d.bx * d.by;
+      const uint32_t last = lx ? 0u : rest & 0x100u, here = rest & ~last;
+      if (here && map[nb] < 0) atomicAdd(unresolved, (uint32_t)__popc(here));
+      if (last && map[nb + 1] < 0) atomicAdd(unresolved, 1u);
+    }
   }
-  int ntot;
-  (void)wg_exclusive_sum(nt, &ntot);
-  if (threadIdx.x == 0) bcounts[a] = (uint32_t)nv | ((uint32_t)ntot << 12) | (1u << 24);
+  const int cr = (t >> 5) * kBN + ((t >> 2) & 7), ci = 2 * (t & 3);
+  const uint32_t m00 = s_row[cr] >> ci, m10 = s_row[cr + 1] >> ci;
+  const uint32_t m01 = s_row[cr + kBN] >> ci, m11 = s_row[cr + kBN + 1] >> ci;
+  const int nt = s_ntris[cell_code(m00, m10, m01, m11)] + s_ntris[cell_code(m00 >> 1, m10 >> 1, m01 >> 1, m11 >> 1)];
+  const int nv = __popc(r.x & own) + __popc(r.y & own) + __popc(r.z & own);
+  int total;  // both counts in one sum: at most 2187 vertices, 2560 triangles
+  const uint32_t pre = (uint32_t)wg_exclusive_sum(nv | nt << 16, &total) & 0xFFFFu;
+  if (t < kRows) recs[a * kRows + t] = make_uint2(pre | r.x << 12 | r.m << 21, r.y | r.z << 9);
+  if (t == 0) bcounts[a] = (uint32_t)(total & 0xFFFF) | ((uint32_t)(total >> 16) << 12) | (1u << 24);
 }
 
-__global__ __launch_bounds__(kNbThreads) void k_nb_emit(const DSpec s, const DGrid g, const NbDims d, float iso,
-                                                        const uint2* __restrict__ act,
-                                                        const int32_t* __restrict__ map,
-                                                        const float* __restrict__ bricks,
-                                                        const uint16_t* __restrict__ tabs,
+// list: the crossed blocks (active rank, first triangle), total->z of them; a workgroup
+// takes every gridDim.x-th.  Bound by vector instructions; with the lists a lane has a vertex
+// or a corner at a time, where a thread per three nodes and two cells left most of a wave idle.
+// 1025^3 rounded cube (129,032 active blocks, a third crossed): 384 -> 143 us.
+__global__ __launch_bounds__(kNbThreads) void k_nb_emit(const DGrid g, const NbDims d, float iso,
+                                                        const uint2* __restrict__ act, const int32_t* __restrict__ map,
+                                                        const float* __restrict__ bricks, const uint2* __restrict__ recs,
+                                                        const uint32_t* __restrict__ bcounts,
                                                         const uint32_t* __restrict__ voff,
-                                                        const uint32_t* __restrict__ toff, float* __restrict__ pos,
-                                                        float* __restrict__ nrm, uint32_t* __restrict__ idx,
+                                                        const uint2* __restrict__ list, const uint4* __restrict__ total,
+                                                        float* __restrict__ pos, uint32_t* __restrict__ idx,
                                                         uint64_t* __restrict__ keys, int64_t cap_v, int64_t cap_t) {
   __shared__ float s_f[kBrick];
-  __shared__ uint16_t s_tab[kBrick];
-  __shared__ uint8_t s_ntris[256];  // triangles per case code (per-lane table reads stay in LDS)
-  __shared__ int32_t s_nrow[8];     // upper neighbour (dx | dy << 1 | dz << 2): its active row, or -1
-  __shared__ uint32_t s_nvoff[8];   // and its first vertex id
-  const int64_t a = blockIdx.x;
-  const uint32_t b = act[a].x;
-  int bx, by, bz;
-  block_coords(d, b, bx, by, bz);
-  const int gi0 = bx * kB, gj0 = by * kB, gk0 = bz * kB;
-  const bool lx = bx == d.bx - 1, ly = by == d.by - 1, lz = bz == d.bz - 1;
+  __shared__ uint2 s_rec[kRows];
+  __shared__ uint32_t s_row[kRows];
+  // the block's vertices (node << 2 | axis), then its triangles (cell | triangle << 9 | code << 12)
+  __shared__ uint32_t s_list[UPF_MC_MAX_TRIS * kCells];
+  static_assert(3 * kBrick <= 2 * UPF_MC_MAX_TRIS * kCells, "a block's vertices fit the list");
+  uint16_t* s_vert = reinterpret_cast<uint16_t*>(s_list);
+  __shared__ uint8_t s_ntris[256];         // triangles per case code
+  __shared__ uint4 s_tris[256];            // and their edges (c_tris16)
+  __shared__ int32_t s_nrow[8];            // upper neighbour (dx | dy << 1 | dz << 2): its active row, -1: none, -2: not crossed
+  __shared__ uint32_t s_nvoff[8];          // and its first vertex id
   static_assert(kNbThreads == 256, "one case code per thread");
-  s_ntris[threadIdx.x] = upf_mc_ntris[threadIdx.x];
-  // threads 1..7 look up the upper neighbours that own the vertices of the brick's upper
-  // faces: the rank read overlaps the brick's reads, the neighbour's first vertex id the
-  // vertex section; both are published before the triangle section's barrier
-  const int no = (int)threadIdx.x;
-  const bool nlook = no >= 1 && no < 8 && !((no & 1) && lx) && !((no & 2) && ly) && !((no & 4) && lz);
-  const int32_t nrow =
-      nlook ? map[(int64_t)b + (no & 1) + (int64_t)((no >> 1) & 1) * d.bx + (int64_t)(no >> 2) * d.bx * d.by] : -1;
-  for (int n = threadIdx.x; n < kBrick; n += kNbThreads) {
-    s_f[n] = bricks[a * kBrick + n];
-    s_tab[n] = tabs[a * kBrick + n];
-  }
-  __syncthreads();
-  const uint32_t vb = voff[a];
-  const uint32_t nvoff = nrow >= 0 ? voff[nrow] : 0u;
-
-  // ---- vertices of the owned nodes 3t .. 3t+2 (normals follow in k_nb_normals)
-  for (int q = 0; q < 3; q++) {
-    const int n = 3 * threadIdx.x + q;
-    if (n >= kBrick) break;
-    const int k = n / (kBN * kBN), r = n - k * kBN * kBN;
-    const int j = r / kBN, i = r - j * kBN;
-    const bool owned = (i < kB || lx) && (j < kB || ly) && (k < kB || lz);
-    const int entry = s_tab[n];
-    const int c = entry >> 12;
-    if (!owned || !c) continue;
-    uint32_t vid = vb + (uint32_t)(entry & 0xFFF);
-    const int gi[3] = {gi0 + i, gj0 + j, gk0 + k};
-    const float p0[3] = {node_coord(g.o[0], g.s[0], gi[0]), node_coord(g.o[1], g.s[1], gi[1]),
-                         node_coord(g.o[2], g.s[2], gi[2])};
-    const float f0 = s_f[n];
-    const int step[3] = {1, kBN, kBN * kBN};
-    const int64_t node = ((int64_t)gi[2] * g.n[1] + gi[1]) * g.n[0] + gi[0];
-    for (int ax = 0; ax < 3; ax++) {
-      if (!((c >> ax) & 1)) continue;
-      const float f1 = s_f[n + step[ax]];
-      const float t = (iso - f0) / (f1 - f0);
-      const float p1a = node_coord(g.o[ax], g.s[ax], gi[ax] + 1);
-      float p[3] = {p0[0], p0[1], p0[2]};
-      p[ax] = p0[ax] + t * (p1a - p0[ax]);
-      if ((int64_t)vid < cap_v) {
-        pos[3 * (size_t)vid + 0] = p[0];
-        pos[3 * (size_t)vid + 1] = p[1];
-        pos[3 * (size_t)vid + 2] = p[2];
-        if (keys) keys[vid] = (uint64_t)node * 3u + (uint64_t)ax;
-      }
-      vid++;
+  const int t = threadIdx.x;
+  s_ntris[t] = upf_mc_ntris[t];
+  s_tris[t] = *reinterpret_cast<const uint4*>(&c_tris16.v[t][0]);
+  const uint8_t* tris = reinterpret_cast<const uint8_t*>(s_tris);
+  const int64_t n_list = (int64_t)total->z;
+  for (int64_t q = blockIdx.x; q < n_list; q += gridDim.x) {
+    const int64_t a = (int64_t)uniform((int)list[q].x);
+    const uint32_t b = act[a].x;
+    int bx, by, bz;
+    block_coords(d, b, bx, by, bz);
+    const bool lx = bx == d.bx - 1, ly = by == d.by - 1, lz = bz == d.bz - 1;
+    const uint32_t vb = voff[a];
+    const int nv = (int)(bcounts[a] & 0xFFFu);
+    __syncthreads();  // the last block's lists are read
+    // threads 1..7 look up the upper neighbours that own the vertices of the brick's upper
+    // faces; a neighbour of one sign owns none of them (its record would count none)
+    if (t >= 1 && t < 8) {
+      const bool there = !((t & 1) && lx) && !((t & 2) && ly) && !((t & 4) && lz);
+      const int32_t row = there ? map[(int64_t)b + (t & 1) + (int64_t)((t >> 1) & 1) * d.bx + (int64_t)(t >> 2) * d.bx * d.by] : -1;
+      s_nrow[t] = row >= 0 && bcounts[row] == 0 ? -2 : row;
+      s_nvoff[t] = row >= 0 ? voff[row] : 0u;
     }
-  }
-
-  if (no >= 1 && no < 8) {
-    s_nrow[no] = nrow;
-    s_nvoff[no] = nvoff;
-  }
-
-  // ---- triangles of cells 2t, 2t+1 (wg_exclusive_sum's barrier publishes s_nrow)
-  int code[2], nt = 0;
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const int cc = 2 * threadIdx.x + q;
-    const int i = cc & 7, j = (cc >> 3) & 7, k = cc >> 6;
-    const int n = (k * kBN + j) * kBN + i;
-    code[q] = (s_f[n] < iso) | ((s_f[n + 1] < iso) << 1) | ((s_f[n + kBN + 1] < iso) << 2) |
-              ((s_f[n + kBN] < iso) << 3) | ((s_f[n + kBN * kBN] < iso) << 4) |
-              ((s_f[n + kBN * kBN + 1] < iso) << 5) | ((s_f[n + kBN * kBN + kBN + 1] < iso) << 6) |
-              ((s_f[n + kBN * kBN + kBN] < iso) << 7);
-    nt += s_ntris[code[q]];
-  }
-  int ntot;
-  uint32_t tid = toff[a] + (uint32_t)wg_exclusive_sum(nt, &ntot);
-  // the triangles' corners: the case's triangulation row in one 16-byte load, the edge
-  // owners from a 64-bit immediate (per-element reads of the constant tables at per-lane
-  // indices were a chain of dependent memory reads per triangle corner: 528 -> 213 us
-  // for this kernel without the whole section)
-  for (int q = 0; q < 2; q++) {
-    const int cc = 2 * threadIdx.x + q;
-    const int i = cc & 7, j = (cc >> 3) & 7, k = cc >> 6;
-    const int ntc = s_ntris[code[q]];
-    if (!ntc) continue;
-    const int4 row = *reinterpret_cast<const int4*>(&c_tris16.v[code[q]][0]);
-    const uint32_t rw[4] = {(uint32_t)row.x, (uint32_t)row.y, (uint32_t)row.z, (uint32_t)row.w};
-#pragma unroll
-    for (int tr = 0; tr < UPF_MC_MAX_TRIS; tr++, tid++) {
-      if (tr >= ntc) break;
-#pragma unroll
-      for (int v = 0; v < 3; v++) {
-        const int qq = 3 * tr + v;
-        const int e = (int)((rw[qq >> 2] >> (8 * (qq & 3))) & 0xFu);  // 0..11 on a triangle row
-        const int own = (int)((kEdgeOwner >> (5 * e)) & 31u);
-        const int li = i + (own & 1), lj = j + ((own >> 1) & 1), lk = k + ((own >> 2) & 1);
-        const int axis = own >> 3;
-        const int ox = (li == kB && !lx), oy = (lj == kB && !ly), oz = (lk == kB && !lz);
-        const int nn = ((lk - kB * oz) * kBN + (lj - kB * oy)) * kBN + (li - kB * ox);
-        uint32_t id = 0xFFFFFFFFu;
-        if (!(ox | oy | oz)) {
-          const int entry = s_tab[nn];
-          id = vb + (uint32_t)(entry & 0xFFF) + (uint32_t)__popc((entry >> 12) & ((1 << axis) - 1));
-        } else {
-          const int o = ox | (oy << 1) | (oz << 2);
-          const int32_t rnb = s_nrow[o];
-          if (rnb >= 0) {
-            const int entry = tabs[(int64_t)rnb * kBrick + nn];
-            id = s_nvoff[o] + (uint32_t)(entry & 0xFFF) + (uint32_t)__popc((entry >> 12) & ((1 << axis) - 1));
-          }
-        }
-        if ((int64_t)tid < cap_t) idx[3 * (size_t)tid + v] = id;
+    for (int n = t; n < kBrick; n += kNbThreads) s_f[n] = bricks[a * kBrick + n];
+    if (t < kRows) {  // the row's owned crossings, node after node
+      const uint2 rec = recs[a * kRows + t];
+      s_rec[t] = rec;
+      s_row[t] = (rec.x >> 21) & 0x1FFu;
+      const uint32_t own = owned_nodes(t, lx, ly, lz);
+      const uint32_t x = (rec.x >> 12) & own, y = rec.y & own, z = (rec.y >> 9) & own;
+      uint16_t* at = s_vert + (rec.x & 0xFFFu);
+      for (uint32_t left = x | y | z; left; left &= left - 1u) {
+        const int i = __ffs(left) - 1;
+        const int node = 4 * (kBN * t + i);
+        if ((x >> i) & 1u) *at++ = (uint16_t)node;
+        if ((y >> i) & 1u) *at++ = (uint16_t)(node + 1);
+        if ((z >> i) & 1u) *at++ = (uint16_t)(node + 2);
       }
+    }
+    __syncthreads();
+
+    // ---- vertices (normals follow in k_nb_normals)
+    for (int e = t; e < nv; e += kNbThreads) {
+      const int n = s_vert[e] >> 2, ax = s_vert[e] & 3;
+      const int k = n / kRows, j = (n - k * kRows) / kBN, i = n - k * kRows - j * kBN;
+      const int gi[3] = {bx * kB + i, by * kB + j, bz * kB + k};
+      const float p0[3] = {node_coord(g.o[0], g.s[0], gi[0]), node_coord(g.o[1], g.s[1], gi[1]),
+                           node_coord(g.o[2], g.s[2], gi[2])};
+      const float f0 = s_f[n], f1 = s_f[n + (ax == 0 ? 1 : (ax == 1 ? kBN : kRows))];
+      const float u = (iso - f0) / (f1 - f0);
+      const uint32_t vid = vb + (uint32_t)e;
+      if ((int64_t)vid < cap_v) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+          const float p1 = node_coord(g.o[c], g.s[c], gi[c] + 1);
+          pos[3 * (size_t)vid + c] = ax == c ? p0[c] + u * (p1 - p0[c]) : p0[c];
+        }
+        if (keys) {
+          const int64_t node = ((int64_t)gi[2] * g.n[1] + gi[1]) * g.n[0] + gi[0];
+          keys[vid] = (uint64_t)node * 3u + (uint64_t)ax;
+        }
+      }
+    }
+
+    // ---- triangles of cells 2t, 2t + 1 into the list (the sum's barriers end the vertices' part)
+    const int cr = (t >> 5) * kBN + ((t >> 2) & 7), ci = 2 * (t & 3);
+    const uint32_t m00 = s_row[cr] >> ci, m10 = s_row[cr + 1] >> ci;
+    const uint32_t m01 = s_row[cr + kBN] >> ci, m11 = s_row[cr + kBN + 1] >> ci;
+    const int code[2] = {cell_code(m00, m10, m01, m11), cell_code(m00 >> 1, m10 >> 1, m01 >> 1, m11 >> 1)};
+    const int nt[2] = {s_ntris[code[0]], s_ntris[code[1]]};
+    int ntot;
+    int at = wg_exclusive_sum(nt[0] + nt[1], &ntot);
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+      for (int tr = 0; tr < nt[h]; tr++) s_list[at++] = (uint32_t)(2 * t + h) | (uint32_t)tr << 9 | (uint32_t)code[h] << 12;
+    __syncthreads();
+
+    // ---- their corners
+    const int64_t first = (int64_t)list[q].y;
+    for (int c = t; c < 3 * ntot; c += kNbThreads) {
+      const int tri = c / 3;
+      const uint32_t entry = s_list[tri];
+      const int cell = (int)(entry & 511u);
+      const int e = tris[(entry >> 12) * 16 + 3 * ((entry >> 9) & 7u) + (uint32_t)(c - 3 * tri)] & 15;  // 0..11
+      const int own = (int)((kEdgeOwner >> (5 * e)) & 31u);
+      const int li = (cell & 7) + (own & 1), lj = ((cell >> 3) & 7) + ((own >> 1) & 1), lk = (cell >> 6) + ((own >> 2) & 1);
+      const int axis = own >> 3;
+      const int ox = (li == kB && !lx), oy = (lj == kB && !ly), oz = (lk == kB && !lz);
+      const int o = ox | (oy << 1) | (oz << 2);
+      uint32_t id;
+      if (!o) {
+        id = vb + row_vertex(s_rec[lk * kBN + lj], li, axis);
+      } else {
+        const int32_t rnb = s_nrow[o];
+        const uint2 rec = rnb >= 0 ? recs[(int64_t)rnb * kRows + (lk - kB * oz) * kBN + (lj - kB * oy)] : make_uint2(0, 0);
+        id = rnb == -1 ? 0xFFFFFFFFu : s_nvoff[o] + row_vertex(rec, li - kB * ox, axis);
+      }
+      if (first + tri < cap_t) idx[3 * (size_t)first + c] = id;
     }
   }
 }
@@ -404,8 +432,8 @@ __global__ __launch_bounds__(256) void k_nb_normals(const DSpec s, const float* 
 struct NbLayout {
   NbDims d;
   int64_t coarse, max_active;
-  size_t off_coarse, off_counts, off_tiles, off_total_a, off_act, off_map, off_bricks, off_tabs, off_bcounts,
-      off_voff, off_toff, off_total_b, bytes;
+  size_t off_coarse, off_counts, off_tiles, off_total_a, off_act, off_map, off_bricks, off_recs, off_list,
+      off_bcounts, off_voff, off_total_b, bytes;
 };
 
 inline size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -424,10 +452,10 @@ NbLayout nb_layout(const NbDims& d, int64_t max_active) {
   L.off_act = o; o = al256(o + sizeof(uint2) * (size_t)d.blocks);
   L.off_map = o; o = al256(o + 4 * (size_t)d.blocks);
   L.off_bricks = o; o = al256(o + 4 * (size_t)kBrick * max_active);
-  L.off_tabs = o; o = al256(o + 2 * (size_t)kBrick * max_active);
+  L.off_recs = o; o = al256(o + sizeof(uint2) * (size_t)kRows * max_active);
+  L.off_list = o; o = al256(o + sizeof(uint2) * (size_t)max_active);
   L.off_bcounts = o; o = al256(o + 4 * (size_t)max_active);
   L.off_voff = o; o = al256(o + 4 * (size_t)max_active);
-  L.off_toff = o; o = al256(o + 4 * (size_t)max_active);
   L.off_total_b = o; o = al256(o + 2 * sizeof(uint4));  // totals + unresolved counter
   L.bytes = o;
   return L;
@@ -454,8 +482,8 @@ struct NbWs {
   uint2* act;
   int32_t* map;
   float* bricks;
-  uint16_t* tabs;
-  uint32_t *bcounts, *voff, *toff;
+  uint2 *recs, *list;
+  uint32_t *bcounts, *voff;
   uint4* total_b;
   int64_t n_coarse;
 };
@@ -463,7 +491,7 @@ struct NbWs {
 int nb_workspace(const NbDims& d, void* d_ws, size_t ws_bytes, NbWs* o) {
   const NbLayout L0 = nb_layout(d, 0);
   if (!d_ws || ws_bytes < L0.bytes) return UPF_ERR_WORKSPACE;
-  const size_t per = 6 * (size_t)kBrick + 12;
+  const size_t per = 4 * (size_t)kBrick + sizeof(uint2) * (kRows + 1) + 8;
   int64_t cap = std::min<int64_t>(d.blocks, (int64_t)((ws_bytes - L0.bytes) / per));
   while (cap > 0 && nb_layout(d, cap).bytes > ws_bytes) cap--;
   const NbLayout L = nb_layout(d, cap);
@@ -477,10 +505,10 @@ int nb_workspace(const NbDims& d, void* d_ws, size_t ws_bytes, NbWs* o) {
   o->act = reinterpret_cast<uint2*>(w + L.off_act);
   o->map = reinterpret_cast<int32_t*>(w + L.off_map);
   o->bricks = reinterpret_cast<float*>(w + L.off_bricks);
-  o->tabs = reinterpret_cast<uint16_t*>(w + L.off_tabs);
+  o->recs = reinterpret_cast<uint2*>(w + L.off_recs);
+  o->list = reinterpret_cast<uint2*>(w + L.off_list);
   o->bcounts = reinterpret_cast<uint32_t*>(w + L.off_bcounts);
   o->voff = reinterpret_cast<uint32_t*>(w + L.off_voff);
-  o->toff = reinterpret_cast<uint32_t*>(w + L.off_toff);
   o->total_b = reinterpret_cast<uint4*>(w + L.off_total_b);
   return UPF_OK;
 }
@@ -491,9 +519,11 @@ int nb_emit(const DSpec& s, const DGrid& g, const NbDims& d, const NbWs& W, floa
   if (out->n_vertices > out->cap_vertices || out->n_triangles > out->cap_triangles) return UPF_ERR_CAPACITY;
   if (out->n_vertices == 0 && out->n_triangles == 0) return UPF_OK;
   if (!out->positions || !out->indices) return UPF_ERR_NULL;
-  hipLaunchKernelGGL(k_nb_emit, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, W.act, W.map, W.bricks,
-                     W.tabs, W.voff, W.toff, out->positions, out->normals, out->indices, d_keys, out->cap_vertices,
-                     out->cap_triangles);
+  // the crossed blocks' number stays on the device: as many workgroups as four rounds of the
+  // machine's, or as there are blocks
+  hipLaunchKernelGGL(k_nb_emit, dim3((unsigned)std::min<int64_t>(nact, 8192)), dim3(kNbThreads), 0, hs, g, d, iso,
+                     W.act, W.map, W.bricks, W.recs, W.bcounts, W.voff, W.list, W.total_b, out->positions, out->indices,
+                     d_keys, out->cap_vertices, out->cap_triangles);
   if (out->normals && out->n_vertices) {
     const dim3 blocks((unsigned)((out->n_vertices + 255) / 256));
     const auto kernel = spec_ext(s) ? k_nb_normals<true> : k_nb_normals<false>;
@@ -553,7 +583,7 @@ int upf_nb_extract(const upf_field_spec* spec, const upf_grid* grid, float iso, 
   hipLaunchKernelGGL(k_nb_map, nblk(nact), dim3(256), 0, hs, W.act, nact, W.map);
   if (modes)
     hipLaunchKernelGGL(k_nb_fine<true>, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, W.act, W.map, W.bricks,
-                       W.tabs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), 0);
+                       W.recs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), 0);
   else {
     int oct_max = 1;  // octaves of the largest gradient / value layer (the brick rows' table)
     for (int l = 0; l < s.n_layers; l++)
@@ -562,13 +592,13 @@ int upf_nb_extract(const upf_field_spec* spec, const upf_grid* grid, float iso, 
     const size_t lds = sizeof(float4) * 4 * 2 * kBrickRows * kBrickGroups * oct_max;
     if (spec_composed(s))
       hipLaunchKernelGGL((k_nb_fine<false, true>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, W.act,
-                         W.map, W.bricks, W.tabs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
+                         W.map, W.bricks, W.recs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
     else
       hipLaunchKernelGGL((k_nb_fine<false, false>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, W.act,
-                         W.map, W.bricks, W.tabs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
+                         W.map, W.bricks, W.recs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
   }
   UPF_LAUNCH_CHECK();
-  if ((st = mc_scan_launch(W.bcounts, nact, W.tiles, W.total_b, W.voff, nullptr, W.toff, hs, kScanBlocks))) return st;
+  if ((st = mc_scan_launch(W.bcounts, nact, W.tiles, W.total_b, W.voff, W.list, nullptr, hs, kScanBlocks))) return st;
   uint4 hb[2];
   UPF_HIP_CHECK(hipMemcpyAsync(hb, W.total_b, 2 * sizeof(uint4), hipMemcpyDeviceToHost, hs));
   UPF_HIP_CHECK(hipStreamSynchronize(hs));
