@@ -486,98 +486,125 @@ __device__ __forceinline__ void row_field(const RowCtx& c, const DSpec& s, float
 // 9 nodes of a narrow-band brick): M groups of kBrickRows rows, row rho = kBrickRows m + r,
 // lane r * nxr + i holding node i of row r of every group (the lanes past kBrickRows *
 // nxr stand in for the last node of row kBrickRows - 1, so that lanes 0 and 63 hold the
-// extreme x).  The collapsed columns of every (row, octave) go into the wave's slice, row
-// rho's regions at rho * total, and each lane reads its M rows with one x part.  The
-// lattice and the column folds and reads are those of the row kernels, so brick values
-// equal the row kernels' at the same nodes bit for bit (while neither falls back to the
-// per-lane functions).  Simplex layers, and layers whose regions do not fit the slice,
-// run per lane.
+// extreme x).  One octave at a time: the collapsed columns of its rows go into the wave's
+// slice, a lane per row and column (63 lanes: 21 rows, three columns a round, an octave's
+// span over 9 nodes being two or three), with the row's octave constants in that lane's
+// registers, and each lane reads its M rows with one x part.  The lattice and the column
+// folds and reads are those of the row kernels, so brick values equal the row kernels' at
+// the same nodes bit for bit (while neither falls back to the per-lane functions).  Simplex
+// layers, and layers whose columns over all octaves would not fit the slice, run per lane.
+// All octaves at once, from a table of (row, octave) constants, with each column's row and
+// octave looked up, took 1,088 vector instructions a wave against 888 for 5 octaves of a
+// 9^3 brick (129,032 bricks of a 1025^3 rounded cube: 841 -> 630 us).
 constexpr int kBrickRows = 7;
 constexpr int kBrickGroups = 3;  // M: groups of rows per wave
 
-// Quotient a / b of small non-negative integers (a < 4096, 1 <= b <= 512; here a task or
-// lane index and a region size) with the divisor given as rb = 1 / b in float32:
-// (a + 1/2) / b lies at least 1 / (2 b) >= 2^-10 away from an integer, and the roundings
-// of rb and of the product move it by less than 4096 * 2^-23 = 2^-11, so truncation
-// gives the exact quotient (an integer division by a variable is a long correction
-// sequence).
-__device__ __forceinline__ int small_div(int a, float rb) { return (int)(((float)a + 0.5f) * rb); }
+// One octave per lane, out of line: the layers that do not run in the slice.  (Inlined, the
+// four noises over unrolled octaves and nodes were 16,000 instructions of the kernel and
+// set its registers.)
+__device__ __noinline__ float lane_noise(int noise, uint32_t seed, float x, float y, float z, float js, float j0) {
+  if (noise == UPF_NOISE_GRADIENT) return noise_gradient(seed, x, y, z);
+  if (noise == UPF_NOISE_VALUE) return noise_value(seed, x, y, z);
+  if (noise == UPF_NOISE_SIMPLEX) return noise_simplex(seed, x, y, z);
+  return noise_cellular(seed, x, y, z, js, j0);
+}
+
+__device__ __forceinline__ float lane_layer(const DLayer& L, float x, float y, float z) {
+  const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
+  float acc = 0.0f;
+  for (int k = 0; k < oct; k++) {
+    const float f = L.freq[k];
+    acc = fractal_acc(L, k, lane_noise(L.noise, L.seed + (uint32_t)k, x * f, y * f, z * f, L.js, L.j0), acc);
+  }
+  return acc;
+}
+
+// The row whose columns this lane folds (rho = 7 m + r), its first column, and the row's
+// y and z.
+struct BrickLane {
+  int rho, col;
+  float y, z;
+};
+
+// Whether a layer's columns over all octaves, times the rows of M groups, exceed the slice.
+template <int M>
+__device__ __forceinline__ bool brick_per_lane(const DLayer& L, int oct, float x) {
+  constexpr int most = kRowSlice2 / (kBrickRows * M);
+  // columns <= 3 + |x span| f, roundings included, unless the spans are huge
+  float sum = 0.0f;
+  for (int k = 0; k < oct; k++) sum = sum + fabsf(L.freq[k]);
+  const float x0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 0));
+  const float x1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+  if (4.0f * (float)oct + 1.01f * fabsf(x1 - x0) * sum <= (float)most) return false;
+  int total = 0;
+  for (int k = 0; k < oct; k++) {
+    int lo, hi;
+    lane_range((int)floorf(x * L.freq[k]), lo, hi);
+    total += hi - lo + 2;
+  }
+  return total > most;
+}
 
 // One gradient / value layer at this lane's M nodes (x, y[m], z[m]) of rows
-// rho = kBrickRows m + rl; yz(rho, y, z) gives row rho's coordinates.  The (row, octave)
-// table has two float4 per entry (ty, tz, uy, uz; the combo seeds), entry rho * oct + k.
-template <int NOISE, int M, class YZ>
-__device__ __forceinline__ void brick_layer_m(const RowCtx& c, const DLayer& L, int rl, YZ yz, float x,
+// rho = kBrickRows m + rl.
+template <int NOISE, int M>
+__device__ __forceinline__ void brick_layer_m(const RowCtx& c, const DLayer& L, int rl, const BrickLane& own, float x,
                                               const float* y, const float* z, float* out) {
   constexpr int NR = kBrickRows * M;
+  constexpr int round = 64 / NR;  // columns a round
   const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
   float2* slice = reinterpret_cast<float2*>(c.slice);
-  int lo[UPF_MAX_OCTAVES], base[UPF_MAX_OCTAVES];
-  int total = 0;
+  if (__builtin_amdgcn_readfirstlane(brick_per_lane<M>(L, oct, x))) {
 #pragma unroll
-  for (int k = 0; k < UPF_MAX_OCTAVES; k++) {
-    if (k < oct) {
-      int hi;
-      lane_range((int)floorf(x * L.freq[k]), lo[k], hi);
-      base[k] = total;
-      total += hi - lo[k] + 2;
-    }
-  }
-  if (NR * total > kRowSlice2) {
-#pragma unroll
-    for (int m = 0; m < M; m++) out[m] = layer_value(L, x, y[m], z[m]);
+    for (int m = 0; m < M; m++) out[m] = lane_layer(L, x, y[m], z[m]);
     return;
   }
-  const float roct = 1.0f / (float)oct;
-  const int lane = lane_of(c);
-  for (int e = lane; e < NR * oct; e += 64) {
-    const int rho = small_div(e, roct);
-    const int k = e - rho * oct;
-    float f = L.freq[0];
 #pragma unroll
-    for (int j = 1; j < UPF_MAX_OCTAVES; j++)
-      if (j < oct && k == j) f = L.freq[j];
-    float yr, zr;
-    yz(rho, yr, zr);
-    const float qy = yr * f, qz = zr * f;
+  for (int m = 0; m < M; m++) out[m] = 0.0f;
+  for (int k = 0; k < oct; k++) {
+    const float f = L.freq[k], amp = L.amp[k];
+    const uint32_t sk = L.seed + (uint32_t)k;
+    const float qx = x * f;
+    const float fx = floorf(qx);
+    int lo, hi;
+    lane_range((int)fx, lo, hi);
+    const int cols = hi - lo + 2;
+    const int stride = min(cols | 1, kRowSlice2 / NR);
+    const float qy = own.y * f, qz = own.z * f;
     const float fy = floorf(qy), fz = floorf(qz);
     const float ty = qy - fy, tz = qz - fz;
     const uint32_t y0 = (uint32_t)(int)fy * kPY, z0 = (uint32_t)(int)fz * kPZ;
-    const uint32_t sk = L.seed + (uint32_t)k;
-    c.oct[2 * e] = make_float4(ty, tz, fade(ty), fade(tz));
-    c.oct[2 * e + 1] = make_float4(__uint_as_float(sk ^ y0 ^ z0), __uint_as_float(sk ^ (y0 + kPY) ^ z0),
-                                   __uint_as_float(sk ^ y0 ^ (z0 + kPZ)), __uint_as_float(sk ^ (y0 + kPY) ^ (z0 + kPZ)));
-  }
-  wave_sync();
-  const float rtotal = 1.0f / (float)total;
-  for (int rd = 0; rd * 64 < NR * total; rd++) {
-    const int t = 64 * rd + lane;
-    const int rho = min(small_div(t, rtotal), NR - 1);
-    const int tt = t - rho * total;
-    int k = 0, off = lo[0] - base[0];  // column X = tt + off of octave k
+    const float4 p0 = make_float4(ty, tz, fade(ty), fade(tz));
+    const float4 p1 = make_float4(__uint_as_float(sk ^ y0 ^ z0), __uint_as_float(sk ^ (y0 + kPY) ^ z0),
+                                  __uint_as_float(sk ^ y0 ^ (z0 + kPZ)), __uint_as_float(sk ^ (y0 + kPY) ^ (z0 + kPZ)));
+    for (int b = 0; b < cols; b += round) {
+      const int col = b + own.col;
+      const float2 v = fold_column<NOISE>(c, p0, p1, (uint32_t)(lo + col));
+      if (col < cols && own.col < round) slice[own.rho * stride + col] = v;
+    }
+    const float tx = qx - fx, ux = fade(tx);
+    const float2* e = slice + rl * stride + ((int)fx - lo);
+    float n[M];
+    wave_sync();
 #pragma unroll
-    for (int j = 1; j < UPF_MAX_OCTAVES; j++)
-      if (j < oct && tt >= base[j]) { k = j; off = lo[j] - base[j]; }
-    const int e = rho * oct + k;
-    const float2 v = fold_column<NOISE>(c, c.oct[2 * e], c.oct[2 * e + 1], (uint32_t)(tt + off));
-    if (t < NR * total) slice[t] = v;
-  }
-  wave_sync();
-  float acc[M];
+    for (int m = 0; m < M; m++) {
+      const float2 e0 = e[m * kBrickRows * stride], e1 = e[m * kBrickRows * stride + 1];
+      if (NOISE == UPF_NOISE_VALUE) n[m] = lerpf(e0.x, e1.x, ux);
+      else n[m] = lerpf(fmaf(e0.x, tx, e0.y), fmaf(e1.x, tx - 1.0f, e1.y), ux);
+    }
+    wave_sync();
+    if (L.fractal == UPF_FRACTAL_RIDGED) {
 #pragma unroll
-  for (int m = 0; m < M; m++) acc[m] = 0.0f;
+      for (int m = 0; m < M; m++) n[m] = fmaf(-2.0f, fabsf(n[m]), 1.0f);
+    }
+    if (L.fractal == UPF_FRACTAL_NONE) {
 #pragma unroll
-  for (int k = 0; k < UPF_MAX_OCTAVES; k++) {
-    if (k < oct) {
-      float n[M];
-      col_read<NOISE, M>(x * L.freq[k], lo[k], slice + base[k] + rl * total, kBrickRows * total, n);
+      for (int m = 0; m < M; m++) out[m] = n[m];
+    } else {
 #pragma unroll
-      for (int m = 0; m < M; m++) acc[m] = fractal_acc(L, k, n[m], acc[m]);
+      for (int m = 0; m < M; m++) out[m] = fmaf(amp, n[m], out[m]);
     }
   }
-  wave_sync();
-#pragma unroll
-  for (int m = 0; m < M; m++) out[m] = acc[m];
 }
 
 // One cellular layer at this lane's node of row rl of a group of kBrickRows rows
@@ -602,7 +629,7 @@ __device__ __forceinline__ float brick_cell_layer(const RowCtx& c, const DLayer&
       fits = fits && hi - lo[k] + 3 <= 7;
     }
   }
-  if (!fits || R * total > kRowSlice2) return layer_value(L, x, y, z);
+  if (!fits || R * total > kRowSlice2) return lane_layer(L, x, y, z);
   for (int r = 0; r < R; r++) {
     float yr, zr;
     yz(r, yr, zr);
@@ -637,6 +664,9 @@ __device__ __forceinline__ void brick_field(const RowCtx& c, const DSpec& s, int
 #pragma unroll
   for (int m = 0; m < M; m++) elev[m] = 0.0f;
   if (need_elev) {
+    const int lane = lane_of(c);
+    BrickLane own{lane % (kBrickRows * M), lane / (kBrickRows * M), 0.0f, 0.0f};
+    yz(own.rho, own.y, own.z);
     float acc[M], msk[M];
 #pragma unroll
     for (int m = 0; m < M; m++) acc[m] = msk[m] = 0.0f;
@@ -644,9 +674,9 @@ __device__ __forceinline__ void brick_field(const RowCtx& c, const DSpec& s, int
       const DLayer& L = s.L[l];
       float raw[M];
       if (L.noise == UPF_NOISE_GRADIENT) {
-        brick_layer_m<UPF_NOISE_GRADIENT, M>(c, L, rl, yz, x, y, z, raw);
+        brick_layer_m<UPF_NOISE_GRADIENT, M>(c, L, rl, own, x, y, z, raw);
       } else if (L.noise == UPF_NOISE_VALUE) {
-        brick_layer_m<UPF_NOISE_VALUE, M>(c, L, rl, yz, x, y, z, raw);
+        brick_layer_m<UPF_NOISE_VALUE, M>(c, L, rl, own, x, y, z, raw);
       } else if (L.noise == UPF_NOISE_CELLULAR) {
 #pragma unroll
         for (int m = 0; m < M; m++) {
@@ -655,7 +685,7 @@ __device__ __forceinline__ void brick_field(const RowCtx& c, const DSpec& s, int
         }
       } else {
 #pragma unroll
-        for (int m = 0; m < M; m++) raw[m] = layer_value(L, x, y[m], z[m]);
+        for (int m = 0; m < M; m++) raw[m] = lane_layer(L, x, y[m], z[m]);
       }
 #pragma unroll
       for (int m = 0; m < M; m++) {

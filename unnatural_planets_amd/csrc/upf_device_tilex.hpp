@@ -25,6 +25,14 @@
 
 namespace upf {
 
+// Quotient a / b of small non-negative integers (a < 4096, 1 <= b <= 512; here a task or
+// lane index and a region size) with the divisor given as rb = 1 / b in float32:
+// (a + 1/2) / b lies at least 1 / (2 b) >= 2^-10 away from an integer, and the roundings
+// of rb and of the product move it by less than 4096 * 2^-23 = 2^-11, so truncation
+// gives the exact quotient (an integer division by a variable is a long correction
+// sequence).
+__device__ __forceinline__ int small_div(int a, float rb) { return (int)(((float)a + 0.5f) * rb); }
+
 constexpr int kTX = 16, kTY = 4;   // nodes of a wave's tile in a plane
 constexpr int kTLds = 256;         // float4 entries of LDS per wave
 static_assert(kTX * kTY == 64, "a lane per node");

@@ -157,9 +157,16 @@ __global__ void k_nb_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t v) {
   if (i < n) p[i] = v;
 }
 
-__global__ void k_nb_map(const uint2* __restrict__ act, int64_t nact, int32_t* __restrict__ map) {
+// The dense map, and in place of each active block's index its coordinates (z, x | y << 16):
+// decoded once here instead of by two integer divisions (40 vector instructions) per wave.
+__global__ void k_nb_map(uint2* __restrict__ act, int64_t nact, const NbDims d, int32_t* __restrict__ map) {
   const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (r < nact) map[act[r].x] = (int32_t)r;
+  if (r >= nact) return;
+  const uint32_t b = act[r].x;
+  map[b] = (int32_t)r;
+  int bx, by, bz;
+  block_coords(d, b, bx, by, bz);
+  act[r] = make_uint2((uint32_t)bz, (uint32_t)bx | (uint32_t)by << 16);
 }
 
 template <bool EXT, bool COMPOSED = true>
@@ -167,13 +174,10 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
                                                         const uint2* __restrict__ act,
                                                         const int32_t* __restrict__ map, float* __restrict__ bricks,
                                                         uint2* __restrict__ recs, uint32_t* __restrict__ bcounts,
-                                                        uint32_t* __restrict__ unresolved, int oct_max) {
+                                                        uint32_t* __restrict__ unresolved) {
   __shared__ float s_fe[EXT ? kBrick : 1];
   __shared__ float4 s_slice[4][EXT ? 1 : kRowSlice];
   __shared__ float4 s_gtab[16];
-  // the (row, octave) tables of the 4 waves, 2 * kBrickRows * kBrickGroups * oct_max float4
-  // each (launch-sized: the spec's largest octave count sets the LDS, hence the occupancy)
-  extern __shared__ float4 s_oct[];
   __shared__ uint64_t s_bits[EXT ? 1 : 4 * kBrickGroups];  // signs of the groups of rows
   __shared__ uint32_t s_row[kRows];                        // and of each row
   __shared__ int s_crossed;
@@ -181,9 +185,9 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
   s_ntris[threadIdx.x] = upf_mc_ntris[threadIdx.x];  // read after the barriers below
   if (threadIdx.x == 0) s_crossed = 0;
   const int64_t a = blockIdx.x;
-  const uint32_t b = act[a].x;
-  int bx, by, bz;
-  block_coords(d, b, bx, by, bz);
+  const uint2 at = act[a];
+  const int bx = (int)(at.y & 0xFFFFu), by = (int)(at.y >> 16), bz = (int)at.x;
+  const int64_t b = ((int64_t)bz * d.by + by) * d.bx + bx;
   const int gi0 = bx * kB, gj0 = by * kB, gk0 = bz * kB;
   const bool lx = bx == d.bx - 1, ly = by == d.by - 1, lz = bz == d.bz - 1;
   float* __restrict__ brick = bricks + a * kBrick;
@@ -211,8 +215,7 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
     if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
     __syncthreads();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const RowCtx ctx = make_row_ctx(s_slice[wave], s_gtab, s_oct + wave * (2 * kBrickRows * kBrickGroups * oct_max),
-                                    lane);
+    const RowCtx ctx = make_row_ctx(s_slice[wave], s_gtab, nullptr, lane);
     const bool node_lane = lane < kBrickRows * kBN;
     const int rl = node_lane ? lane / kBN : kBrickRows - 1;
     const int i = node_lane ? lane - rl * kBN : kBN - 1;
@@ -268,7 +271,7 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
     own = owned_nodes(t, lx, ly, lz);
     if (const uint32_t rest = (r.x | r.y | r.z) & ~own) {  // crossings of other blocks' nodes
       const int oy = t % kBN == kB && !ly, oz = t >= kB * kBN && !lz;
-      const int64_t nb = (int64_t)b + (int64_t)oy * d.bx + (int64_t)oz * d.bx * d.by;
+      const int64_t nb = b + (int64_t)oy * d.bx + (int64_t)oz * d.bx * d.by;
       const uint32_t last = lx ? 0u : rest & 0x100u, here = rest & ~last;
       if (here && map[nb] < 0) atomicAdd(unresolved, (uint32_t)__popc(here));
       if (last && map[nb + 1] < 0) atomicAdd(unresolved, 1u);
@@ -288,8 +291,10 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
 // list: the crossed blocks (active rank, first triangle), total->z of them; a workgroup
 // takes every gridDim.x-th.  Bound by vector instructions; with the lists a lane has a vertex
 // or a corner at a time, where a thread per three nodes and two cells left most of a wave idle.
-// 1025^3 rounded cube (129,032 active blocks, a third crossed): 384 -> 143 us.
-__global__ __launch_bounds__(kNbThreads) void k_nb_emit(const DGrid g, const NbDims d, float iso,
+// 1025^3 rounded cube (129,032 active blocks, a third crossed): 384 -> 120 us (143 at seven
+// waves a SIMD: a block is a chain of dependent reads; one workgroup per block 25 us more,
+// 2048 in all 35 us more).
+__global__ __launch_bounds__(kNbThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_nb_emit(const DGrid g, const NbDims d, float iso,
                                                         const uint2* __restrict__ act, const int32_t* __restrict__ map,
                                                         const float* __restrict__ bricks, const uint2* __restrict__ recs,
                                                         const uint32_t* __restrict__ bcounts,
@@ -316,21 +321,17 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_emit(const DGrid g, const NbD
   const int64_t n_list = (int64_t)total->z;
   for (int64_t q = blockIdx.x; q < n_list; q += gridDim.x) {
     const int64_t a = (int64_t)uniform((int)list[q].x);
-    const uint32_t b = act[a].x;
-    int bx, by, bz;
-    block_coords(d, b, bx, by, bz);
+    const uint2 where = act[a];
+    const int bx = (int)(where.y & 0xFFFFu), by = (int)(where.y >> 16), bz = (int)where.x;
+    const int64_t b = ((int64_t)bz * d.by + by) * d.bx + bx;
     const bool lx = bx == d.bx - 1, ly = by == d.by - 1, lz = bz == d.bz - 1;
     const uint32_t vb = voff[a];
     const int nv = (int)(bcounts[a] & 0xFFFu);
     __syncthreads();  // the last block's lists are read
     // threads 1..7 look up the upper neighbours that own the vertices of the brick's upper
-    // faces; a neighbour of one sign owns none of them (its record would count none)
-    if (t >= 1 && t < 8) {
-      const bool there = !((t & 1) && lx) && !((t & 2) && ly) && !((t & 4) && lz);
-      const int32_t row = there ? map[(int64_t)b + (t & 1) + (int64_t)((t >> 1) & 1) * d.bx + (int64_t)(t >> 2) * d.bx * d.by] : -1;
-      s_nrow[t] = row >= 0 && bcounts[row] == 0 ? -2 : row;
-      s_nvoff[t] = row >= 0 ? voff[row] : 0u;
-    }
+    // faces, published after the vertices' part
+    const bool there = t >= 1 && t < 8 && !((t & 1) && lx) && !((t & 2) && ly) && !((t & 4) && lz);
+    const int32_t row = there ? map[b + (t & 1) + (int64_t)((t >> 1) & 1) * d.bx + (int64_t)(t >> 2) * d.bx * d.by] : -1;
     for (int n = t; n < kBrick; n += kNbThreads) s_f[n] = bricks[a * kBrick + n];
     if (t < kRows) {  // the row's owned crossings, node after node
       const uint2 rec = recs[a * kRows + t];
@@ -370,6 +371,12 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_emit(const DGrid g, const NbD
           keys[vid] = (uint64_t)node * 3u + (uint64_t)ax;
         }
       }
+    }
+
+    // a neighbour of one sign owns none of the vertices (its record would count none)
+    if (t >= 1 && t < 8) {
+      s_nrow[t] = row >= 0 && bcounts[row] == 0 ? -2 : row;
+      s_nvoff[t] = row >= 0 ? voff[row] : 0u;
     }
 
     // ---- triangles of cells 2t, 2t + 1 into the list (the sum's barriers end the vertices' part)
@@ -580,23 +587,10 @@ int upf_nb_extract(const upf_field_spec* spec, const upf_grid* grid, float iso, 
   out->n_vertices = out->n_triangles = 0;
   if (nact == 0) return UPF_OK;
 
-  hipLaunchKernelGGL(k_nb_map, nblk(nact), dim3(256), 0, hs, W.act, nact, W.map);
-  if (modes)
-    hipLaunchKernelGGL(k_nb_fine<true>, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, W.act, W.map, W.bricks,
-                       W.recs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), 0);
-  else {
-    int oct_max = 1;  // octaves of the largest gradient / value layer (the brick rows' table)
-    for (int l = 0; l < s.n_layers; l++)
-      if (s.L[l].noise == UPF_NOISE_GRADIENT || s.L[l].noise == UPF_NOISE_VALUE)
-        oct_max = std::max(oct_max, s.L[l].fractal == UPF_FRACTAL_NONE ? 1 : s.L[l].octaves);
-    const size_t lds = sizeof(float4) * 4 * 2 * kBrickRows * kBrickGroups * oct_max;
-    if (spec_composed(s))
-      hipLaunchKernelGGL((k_nb_fine<false, true>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, W.act,
-                         W.map, W.bricks, W.recs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
-    else
-      hipLaunchKernelGGL((k_nb_fine<false, false>), dim3((unsigned)nact), dim3(kNbThreads), lds, hs, s, g, d, iso, W.act,
-                         W.map, W.bricks, W.recs, W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1), oct_max);
-  }
+  hipLaunchKernelGGL(k_nb_map, nblk(nact), dim3(256), 0, hs, W.act, nact, d, W.map);
+  const auto fine = modes ? k_nb_fine<true> : (spec_composed(s) ? k_nb_fine<false, true> : k_nb_fine<false, false>);
+  hipLaunchKernelGGL(fine, dim3((unsigned)nact), dim3(kNbThreads), 0, hs, s, g, d, iso, W.act, W.map, W.bricks, W.recs,
+                     W.bcounts, reinterpret_cast<uint32_t*>(W.total_b + 1));
   UPF_LAUNCH_CHECK();
   if ((st = mc_scan_launch(W.bcounts, nact, W.tiles, W.total_b, W.voff, W.list, nullptr, hs, kScanBlocks))) return st;
   uint4 hb[2];
