@@ -1,7 +1,8 @@
 """Grids of many rows are evaluated in bands of eight rows, smaller ones two rows at a time:
 the same values.  A large grid is compared with its planes evaluated a few at a time, over
 ragged sides, all layer kinds and blends, spacings at which a wave spans few cells, more
-columns than a band's share and more than fit at all, and bands over several cells."""
+columns than a band's share and more than fit at all, bands over several cells and cells
+past the pairs' reach.  The adjoint's bands of four rows likewise."""
 import pytest
 
 from unnatural_planets_amd import spec as S
@@ -19,6 +20,8 @@ def _layers(kind):
                 S.layer("value", "fbm", 3, 0.003, weight=1.5, seed=13)]
     if kind == "cells":
         return [S.layer("cellular", "ridged", 2, 0.003, weight=2.0, seed=11), S.layer("cellular", "none", 1, 0.0625, weight=1.0, seed=12)]
+    if kind == "cells8":  # more octaves than the pairs hold
+        return [S.layer("cellular", "fbm", 8, 0.0005, weight=2.0, seed=11)]
     if kind == "wide":
         return [S.layer("gradient", "fbm", 3, 0.12, weight=2.0, seed=21), S.layer("value", "fbm", 2, 0.9, weight=1.0, seed=22)]
     return [S.layer("simplex", "fbm", 3, 0.002, weight=1.5, seed=13)]
@@ -68,7 +71,7 @@ def test_batch_of_both_kinds(upf, first, variant):
 
 @pytest.mark.parametrize("dims", DIMS)
 @pytest.mark.parametrize("spacing", [0.5, 8.0, 9.5, 61.0])
-@pytest.mark.parametrize("kind", ["blends", "cells", "wide", "simplex"])
+@pytest.mark.parametrize("kind", ["blends", "cells", "cells8", "wide", "simplex"])
 @pytest.mark.parametrize("shape,params,compose", [("torus", (1200.0, 450.0), "land"), ("pipe", (), "navigation"), ("none", (), "elevation_raw"),
                                                   ("hemispheres", (), "water"), ("sphere", (900.0,), "elevation")])
 def test_bands_are_rows(upf, shape, params, compose, kind, spacing, dims):
@@ -90,3 +93,41 @@ def test_signs_and_mesh(upf):
     a = upf.mc_emit_counted(f, g, 0.0, ws, nv, nt)
     b = upf.mc_extract(f, g)
     assert nv > 0 and torch.equal(a.positions, b.positions) and torch.equal(a.indices, b.indices)
+
+
+# the fewest bands of four rows, ragged, one band a plane, more rows than planes
+GRAD_DIMS = [(64, 16, 1024), (65, 37, 210), (130, 3, 1400), (257, 201, 34)]
+
+
+@pytest.mark.parametrize("dims", GRAD_DIMS)
+@pytest.mark.parametrize("spacing", [0.5, 8.0, 61.0])
+@pytest.mark.parametrize("kind", ["sum", "cells", "cells8", "wide"])
+@pytest.mark.parametrize("shape,params,compose", [("torus", (1200.0, 450.0), "land"), ("none", (), "elevation_raw"), ("box", (700.0, 500.0, 300.0, 90.0), "water"),
+                                                  ("capsule", (900.0, 300.0), "elevation")])
+@pytest.mark.parametrize("theta", [True, False])
+def test_adjoint_bands_are_rows(upf, theta, shape, params, compose, kind, spacing, dims):
+    """f and df/dp of a large grid equal those of its planes taken a few at a time (rows), and
+    dL/dtheta their sum within 1e-4 of its scale, as the grid adjoint is held to elsewhere."""
+    import torch
+    layers = _layers(kind) if kind != "sum" else [S.layer("gradient", "ridged", 4, 0.002, 2.1, -0.4, 3.0, 7),
+                                                  S.layer("value", "fbm", 3, 0.003, weight=1.5, seed=13),
+                                                  S.layer("cellular", "none", 1, 0.004, weight=2.0, seed=11, jitter=0.8)]
+    s = S.field_spec(shape, params, layers, compose, 0.1)
+    w = torch.randn(dims[::-1], device="cuda", generator=torch.Generator("cuda").manual_seed(5)) if theta else None
+    f, dfdx, th = upf.field_adjoint_grid(s, _grid(dims, spacing), w)
+    assert torch.isfinite(f).all() and torch.isfinite(dfdx).all()
+    total = 0.0
+    for k in range(0, dims[2], 34):
+        n = min(34, dims[2] - k)
+        if n < 2:
+            k, n = k - 1, 2
+        pf, pd, pt = upf.field_adjoint_grid(s, _grid(dims, spacing, k, n), w[k:k + n].contiguous() if theta else None)
+        assert torch.equal(f[k:k + n], pf) and torch.equal(dfdx[k:k + n], pd)
+        if theta:
+            if (k % 34) and n == 2:  # the plane before is counted already
+                zero = w[k:k + n].clone()
+                zero[0] = 0
+                pt = upf.field_adjoint_grid(s, _grid(dims, spacing, k, n), zero)[2]
+            total = total + pt.double()
+    if theta:
+        assert float((th.double() - total).abs().max()) <= 1e-4 * max(float(total.abs().max()), 1e-6)

@@ -102,7 +102,7 @@ __device__ __forceinline__ void batch_field_pair(const RowCtx& ctx, const BChunk
 
 // A band (upf_device_band.hpp): the same of kBandRows rows from row j on, as
 // k_eval_grid_band's waves.
-template <bool COMPOSED>
+template <bool COMPOSED, bool WIDE>
 __device__ __forceinline__ void batch_field_band(const RowCtx& ctx, const BChunk& C, int xb, int j, int k,
                                                  float* __restrict__ field, uint64_t* __restrict__ S) {
   constexpr int R = kBandRows;
@@ -113,7 +113,7 @@ __device__ __forceinline__ void batch_field_band(const RowCtx& ctx, const BChunk
   const float yl = node_coord(C.grid.o[1], C.grid.s[1], j + min(lane & (R - 1), rows - 1));
   const float z = node_coord(C.grid.o[2], C.grid.s[2], k);
   float v[R];
-  band_field<R, COMPOSED>(ctx, C.spec, x, yl, z, v);
+  band_field<R, COMPOSED, WIDE>(ctx, C.spec, x, yl, z, v);
   const int in = xb * 64 + lane_of(ctx);  // recomputed: not live across the layers
   const bool valid = in < C.grid.n[0];
   const int64_t o = C.node_off + ((int64_t)k * C.grid.n[1] + j) * C.grid.n[0] + in;
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 7
 
 // The list of bands.  64-chunk batch (32^3 to 192^3, 152 M nodes) as a whole, row pairs
 // against bands: 1.33 / 0.84 ms.
-template <bool COMPOSED>
+template <bool COMPOSED, bool WIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_batch_field_bands(
     const BChunk* __restrict__ ch, int n_chunks, const uint64_t* __restrict__ blk_start, int64_t n_items,
     float* __restrict__ field, uint64_t* __restrict__ S) {
@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
   if (r >= n_items) return;  // whole waves
   const BItem it = batch_item<1>(ch, n_chunks, blk_start[blockIdx.x], r, wave);
   const RowCtx ctx = make_row_ctx(s_slice[wave], s_gtab, nullptr, threadIdx.x & 63);
-  batch_field_band<COMPOSED>(ctx, ch[it.c], it.xb, kBandRows * it.row, it.k, field, S);
+  batch_field_band<COMPOSED, WIDE>(ctx, ch[it.c], it.xb, kBandRows * it.row, it.k, field, S);
 }
 
 // Counts of every group of every chunk (global id g: chunk, then its local group) from
@@ -300,6 +300,7 @@ struct upf_batch {
   int64_t nodes = 0, groups = 0, items[2] = {0, 0};
   bool any_ext = false;  // a chunk with an elevation mode or a further shape: the field runs per lane
   bool any_composed = false;  // a chunk whose shape is a composition (spec_composed)
+  bool any_wide = false;  // a chunk in bands with a cellular layer past the pairs' reach (band_wide)
   upf_batch_opts opts{};
   size_t off_S = 0, off_counts = 0, off_voff = 0, off_toff = 0, off_act = 0, off_tiles = 0, off_total = 0,
          ws_bytes = 0;
@@ -330,10 +331,11 @@ int upload(upf_batch* b) {
 
 using FieldKernel = void (*)(const BChunk*, int, const uint64_t*, int64_t, float*, uint64_t*);
 
-FieldKernel field_kernel(int list, bool lanes, bool ext, bool composed) {
+FieldKernel field_kernel(int list, bool lanes, bool ext, bool composed, bool wide) {
   if (ext) return k_batch_field_pairs<UPF_EVAL_PER_LANE, true, true, 0>;  // no bands then
   if (lanes) return list ? k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, 1> : k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, 0>;
-  if (list) return composed ? k_batch_field_bands<true> : k_batch_field_bands<false>;
+  if (list && wide) return composed ? k_batch_field_bands<true, true> : k_batch_field_bands<false, true>;
+  if (list) return composed ? k_batch_field_bands<true, false> : k_batch_field_bands<false, false>;
   return composed ? k_batch_field_pairs<UPF_EVAL_ROWS, false, true, 0> : k_batch_field_pairs<UPF_EVAL_ROWS, false, false, 0>;
 }
 
@@ -352,7 +354,7 @@ int run(upf_batch* b, float* field, void* ws, size_t ws_bytes, float* pos, float
   for (int list = 0; list < 2; list++) {
     if (!b->items[list]) continue;
     const bool lanes = b->any_ext || b->opts.field_variant == UPF_EVAL_PER_LANE;
-    const auto kernel = field_kernel(list, lanes, b->any_ext, b->any_composed);
+    const auto kernel = field_kernel(list, lanes, b->any_ext, b->any_composed, b->any_wide);
     const dim3 blocks((unsigned)b->item_blocks[list], lanes ? kItemRows[list] / 2 : 1);
     hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, s, b->dev, b->n, b->blk_start + (list ? b->item_blocks[0] : 0),
                        b->items[list], field, S);
@@ -415,6 +417,7 @@ int upf_batch_create(const upf_chunk* chunks, int32_t n_chunks, const upf_batch_
     if (band_fits(C.spec, C.grid)) bands += band_items(C.grid);
   for (BChunk& C : b->host) {
     const int list = !b->any_ext && bands >= kBandItems && band_fits(C.spec, C.grid);
+    if (list && band_wide(C.spec, C.grid, kRowSlice2)) b->any_wide = true;
     for (int l = 0; l < 2; l++) C.item_off[l] = b->items[l];
     b->items[list] += (int64_t)C.gx * item_rows(C.grid, list) * C.grid.n[2];
   }

@@ -26,6 +26,9 @@ constexpr int kBandRows = 8;
 constexpr int kBandStride = 56;  // columns per row in LDS: rows 16 banks apart
 static_assert(kBandRows * kBandStride <= kRowSlice2 && UPF_MAX_OCTAVES * kBandStride <= kRowSlice2, "the columns fit the slice");
 
+constexpr int kWidePoints = 4 * kRowSlice / 3;  // feature points in the slice: x, y, z
+constexpr int kWideCells = kWidePoints / 9;     // cells that 64 nodes may reach along x
+
 // Whether every wave of a grid evaluates every layer of the spec in LDS, as columns or cells
 // (no simplex, and the octaves' spans over 64 nodes fit).  The bound covers the rounding of
 // the nodes' coordinates, so no wave needs more; near it the two-row form decides per wave.
@@ -41,16 +44,32 @@ inline bool band_fits(const DSpec& s, const DGrid& g) {
     if (L.noise == UPF_NOISE_SIMPLEX) return false;
     double columns = 0.0;
     const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
-    if (L.noise == UPF_NOISE_CELLULAR && 72 * oct > kRowSlice2) return false;  // per lane in rows
     for (int k = 0; k < oct; k++) {
       const double f = std::fabs((double)L.freq[k]);
       const double span = f * (63.0 * step + reach * 0x1p-21);  // cells from end to end
-      if (L.noise == UPF_NOISE_CELLULAR && !(span <= 3.9)) return false;
+      if (L.noise == UPF_NOISE_CELLULAR && !(span <= kWideCells - 3.1)) return false;
       columns += span + 3.0;
     }
     if (L.noise != UPF_NOISE_CELLULAR && !(columns <= kRowSlice2)) return false;
   }
   return true;
+}
+
+// Whether some wave may need band_cellular_wide: a cellular layer past the two-row form's
+// reach (cells_in_slice).  The kernels that have it are instantiations of their own: its
+// registers cost the others 12 %.
+inline bool band_wide(const DSpec& s, const DGrid& g, int slice) {
+  const double step = std::fabs((double)g.s[0]);
+  const double reach = std::fabs((double)g.o[0]) + step * g.n[0];
+  for (int l = 0; l < s.n_layers; l++) {
+    const DLayer& L = s.L[l];
+    if (L.noise != UPF_NOISE_CELLULAR) continue;
+    const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
+    if (72 * oct > slice) return true;
+    for (int k = 0; k < oct; k++)
+      if (!(std::fabs((double)L.freq[k]) * (63.0 * step + reach * 0x1p-21) <= 3.9)) return true;
+  }
+  return false;
 }
 
 // Bands of eight rows take a quarter of the two-row form's waves, and need 16 to a CU (four
@@ -173,10 +192,86 @@ __device__ __forceinline__ void band_cellular(const RowCtx& c, const DLayer& L, 
   }
 }
 
-// One layer at this lane's node of R rows.
+// The feature points (x, y, z - q_z) of the cells that a wave's nodes reach in one row of
+// cells cy, as entry lx + stride * (dy + 3 dz) of three arrays: as many cells as fit.
+__device__ __forceinline__ void wide_points(const RowCtx& c, const DLayer& L, uint32_t sk, int lo, int n, int cy, int cz,
+                                            float qz) {
+  float* px = reinterpret_cast<float*>(c.slice);
+  const CellLane cl = cell_lane(c.lane);
+  const int ky = cy - 1 + cl.dy, kz = cz - 1 + cl.dz;
+  for (int b = cl.lx; b < n; b += 7) {
+    const int kx = lo - 1 + b;
+    const uint32_t h = (sk ^ ((uint32_t)kx * kPX) ^ ((uint32_t)ky * kPY) ^ ((uint32_t)kz * kPZ)) * kHM;
+    const uint32_t m = h ^ (h >> 15);
+    if (cl.c9 < 9) {
+      const int at = b + n * cl.c9;
+      px[at] = fmaf((float)(m & 1023u), L.js, (float)kx - L.j0);
+      px[kWidePoints + at] = fmaf((float)((m >> 10) & 1023u), L.js, (float)ky - L.j0);
+      px[2 * kWidePoints + at] = fmaf((float)((m >> 20) & 1023u), L.js, (float)kz - L.j0) - qz;
+    }
+  }
+}
+
+// One octave of a cellular layer whose lanes span more cells than the two-row form takes:
+// the distances in the order of the per-lane form, which that form then runs, the points
+// hashed once a wave.  Torus with six octaves and a cellular layer at 6 per unit, 240^3: 269
+// us with the layer per lane, 149 here.
 template <int R>
+__device__ __forceinline__ void band_cellular_wide(const RowCtx& c, const DLayer& L, float f, uint32_t sk, float x, float yl,
+                                                   float z, float* n) {
+  const float* px = reinterpret_cast<const float*>(c.slice);
+  const float qx = x * f, qz = z * f;
+  const int ix = (int)rintf(qx);
+  int lo, hi;
+  lane_range(ix, lo, hi);
+  const int cells = hi - lo + 3;
+  const int cyl = (int)rintf(yl * f), cz = __builtin_amdgcn_readfirstlane((int)rintf(qz));
+  for (int r0 = 0; r0 < R;) {
+    const int cy = __builtin_amdgcn_readlane(cyl, r0);
+    const uint32_t rows = (uint32_t)__ballot(cyl == cy) & ((1u << R) - 1u);  // lane r holds row r
+    wide_points(c, L, sk, lo, cells, cy, cz, qz);
+    wave_sync();
+    float best[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) best[r] = __builtin_inff();
+    for (int c9 = 0; c9 < 9; c9++) {
+      const float* p = px + (ix - lo) + cells * c9;
+#pragma unroll
+      for (int q = 0; q < 3; q++) {
+        const float dx = p[q] - qx, py = p[kWidePoints + q], dz = p[2 * kWidePoints + q];
+        const float dxx = dx * dx;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+          const float dy = py - band_row(yl, r) * f;
+          best[r] = fminf(best[r], fmaf(dz, dz, fmaf(dy, dy, dxx)));
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++)
+      if ((rows >> r) & 1u) n[r] = sqrt_hw(best[r]);
+    wave_sync();
+    r0 += __popc(rows);
+  }
+}
+
+// Whether the two-row form evaluates a cellular layer in LDS: at most 5 cells spanned, all
+// octaves in the slice.
+__device__ __forceinline__ bool cells_in_slice(const DLayer& L, int oct, float x, int slice) {
+  bool fits = 72 * oct <= slice;
+  for (int k = 0; k < oct; k++) {
+    int lo, hi;
+    lane_range((int)rintf(x * L.freq[k]), lo, hi);
+    fits = fits && hi - lo <= 4;
+  }
+  return __builtin_amdgcn_readfirstlane(fits);
+}
+
+// One layer at this lane's node of R rows.
+template <int R, bool WIDE>
 __device__ __forceinline__ void band_layer(const RowCtx& c, const DLayer& L, float x, float yl, float z, float* out) {
   const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
+  const bool wide = WIDE && L.noise == UPF_NOISE_CELLULAR && !cells_in_slice(L, oct, x, kRowSlice2);
 #pragma unroll
   for (int r = 0; r < R; r++) out[r] = 0.0f;
   for (int k = 0; k < oct; k++) {
@@ -187,6 +282,8 @@ __device__ __forceinline__ void band_layer(const RowCtx& c, const DLayer& L, flo
       band_lattice<UPF_NOISE_GRADIENT, R>(c, f, sk, x, yl, z, n);
     } else if (L.noise == UPF_NOISE_VALUE) {
       band_lattice<UPF_NOISE_VALUE, R>(c, f, sk, x, yl, z, n);
+    } else if (wide) {
+      band_cellular_wide<R>(c, L, f, sk, x, yl, z, n);
     } else {
       band_cellular<R>(c, L, f, sk, x, yl, z, n);
     }
@@ -205,7 +302,7 @@ __device__ __forceinline__ void band_layer(const RowCtx& c, const DLayer& L, flo
 }
 
 // f at this lane's node of R rows (row_field's values).
-template <int R, bool COMPOSED>
+template <int R, bool COMPOSED, bool WIDE>
 __device__ __forceinline__ void band_field(const RowCtx& c, const DSpec& s, float x, float yl, float z, float* out) {
   const bool need_elev = s.compose == UPF_COMPOSE_LAND || s.compose == UPF_COMPOSE_NAVIGATION ||
                          s.compose == UPF_COMPOSE_ELEVATION_RAW;
@@ -215,7 +312,7 @@ __device__ __forceinline__ void band_field(const RowCtx& c, const DSpec& s, floa
   for (int l = 0; need_elev && l < s.n_layers; l++) {
     const DLayer& L = s.L[l];
     float v[R];
-    band_layer<R>(c, L, x, yl, z, v);
+    band_layer<R, WIDE>(c, L, x, yl, z, v);
 #pragma unroll
     for (int r = 0; r < R; r++) v[r] = L.weight * v[r];
     if (L.blend == UPF_BLEND_ADD) {

@@ -151,7 +151,7 @@ __device__ __noinline__ Grad shape_more_d(int shape, float p0, float p1, float p
 }
 
 // Returns shape(p); writes d shape/dp and d shape/d params[0..3].
-template <bool EXT = true>
+template <bool EXT, bool COMPOSED = true>
 __device__ __forceinline__ float shape_eval_d(const DSpec& s, float x, float y, float z, float g[3],
                                               float dp[4]) {
   g[0] = g[1] = g[2] = 0.0f;
@@ -209,6 +209,7 @@ __device__ __forceinline__ float shape_eval_d(const DSpec& s, float x, float y, 
     case UPF_SHAPE_NONE:
       return 0.0f;
     default: {  // extended shapes: forward-mode position gradient, no parameter gradient
+      if (!COMPOSED) return 0.0f;
       const Grad r = EXT && s.shape >= UPF_SHAPE_H3O ? shape_more_d(s.shape, s.sp[0], s.sp[1], s.sp[2], s.sp[3], s.w, x, y, z)
                                               : shape_ext<Grad>(s.shape, s.sp, gvar(x, 0), gvar(y, 1), gvar(z, 2),
                                                                 gc(0.0f));

@@ -26,6 +26,39 @@
 
 namespace upf {
 
+// Column X of an octave with its derivatives: planes v = (A, B), vy, vz.
+template <int NOISE>
+__device__ __forceinline__ void fold_column_d(const RowCtx& c, const float4 p0, const float4 p1, float duy, float duz,
+                                              uint32_t X, float2& v, float2& vy, float2& vz) {
+  const uint32_t hx = X * kPX;
+  const uint32_t h0 = (__float_as_uint(p1.x) ^ hx) * kHM, h1 = (__float_as_uint(p1.y) ^ hx) * kHM;
+  const uint32_t h2 = (__float_as_uint(p1.z) ^ hx) * kHM, h3 = (__float_as_uint(p1.w) ^ hx) * kHM;
+  const float ty = p0.x, tz = p0.y, uy = p0.z, uz = p0.w;
+  float a0, a1, a2, a3, b0 = 0.0f, b1 = 0.0f, b2 = 0.0f, b3 = 0.0f;
+  float gy = 0.0f, gz = 0.0f;  // fold(g_y), fold(g_z)
+  if (NOISE == UPF_NOISE_GRADIENT) {
+    const float4 g0 = c.gtab[h0 >> 28], g1 = c.gtab[h1 >> 28], g2 = c.gtab[h2 >> 28], g3 = c.gtab[h3 >> 28];
+    const float ty1 = ty - 1.0f, tz1 = tz - 1.0f;
+    a0 = g0.x; a1 = g1.x; a2 = g2.x; a3 = g3.x;
+    b0 = fmaf(g0.z, tz, g0.y * ty); b1 = fmaf(g1.z, tz, g1.y * ty1);
+    b2 = fmaf(g2.z, tz1, g2.y * ty); b3 = fmaf(g3.z, tz1, g3.y * ty1);
+    gy = lerpf(lerpf(g0.y, g1.y, uy), lerpf(g2.y, g3.y, uy), uz);
+    gz = lerpf(lerpf(g0.z, g1.z, uy), lerpf(g2.z, g3.z, uy), uz);
+  } else {
+    a0 = lattice_value(h0); a1 = lattice_value(h1); a2 = lattice_value(h2); a3 = lattice_value(h3);
+  }
+  const float ay0 = lerpf(a0, a1, uy), ay1 = lerpf(a2, a3, uy);
+  const float by0 = lerpf(b0, b1, uy), by1 = lerpf(b2, b3, uy);
+  const float A = lerpf(ay0, ay1, uz), B = lerpf(by0, by1, uz);
+  const float Ay = duy * lerpf(a1 - a0, a3 - a2, uz);
+  const float By = fmaf(duy, lerpf(b1 - b0, b3 - b2, uz), gy);
+  const float Az = duz * (ay1 - ay0);
+  const float Bz = fmaf(duz, by1 - by0, gz);
+  v = make_float2(A, B);
+  vy = make_float2(Ay, By);
+  vz = make_float2(Az, Bz);
+}
+
 template <int NOISE>
 __device__ __forceinline__ void col_write_d(const RowCtx& c, const DLayer& L, int oct, float y, float z,
                                             const int* lo, const int* base, int total, float2* slice) {
@@ -55,49 +88,24 @@ __device__ __forceinline__ void col_write_d(const RowCtx& c, const DLayer& L, in
     for (int j = 1; j < UPF_MAX_OCTAVES; j++)
       if (j < oct) k += t >= base[j];
     const float4 p0 = c.oct[3 * k], p1 = c.oct[3 * k + 1], p2 = c.oct[3 * k + 2];
-    const uint32_t hx = (uint32_t)(t + __float_as_int(p2.x)) * kPX;
-    const uint32_t h0 = (__float_as_uint(p1.x) ^ hx) * kHM, h1 = (__float_as_uint(p1.y) ^ hx) * kHM;
-    const uint32_t h2 = (__float_as_uint(p1.z) ^ hx) * kHM, h3 = (__float_as_uint(p1.w) ^ hx) * kHM;
-    const float ty = p0.x, tz = p0.y, uy = p0.z, uz = p0.w, duy = p2.y, duz = p2.z;
-    float a0, a1, a2, a3, b0 = 0.0f, b1 = 0.0f, b2 = 0.0f, b3 = 0.0f;
-    float gy = 0.0f, gz = 0.0f;  // fold(g_y), fold(g_z)
-    if (NOISE == UPF_NOISE_GRADIENT) {
-      const float4 g0 = c.gtab[h0 >> 28], g1 = c.gtab[h1 >> 28], g2 = c.gtab[h2 >> 28], g3 = c.gtab[h3 >> 28];
-      const float ty1 = ty - 1.0f, tz1 = tz - 1.0f;
-      a0 = g0.x; a1 = g1.x; a2 = g2.x; a3 = g3.x;
-      b0 = fmaf(g0.z, tz, g0.y * ty); b1 = fmaf(g1.z, tz, g1.y * ty1);
-      b2 = fmaf(g2.z, tz1, g2.y * ty); b3 = fmaf(g3.z, tz1, g3.y * ty1);
-      gy = lerpf(lerpf(g0.y, g1.y, uy), lerpf(g2.y, g3.y, uy), uz);
-      gz = lerpf(lerpf(g0.z, g1.z, uy), lerpf(g2.z, g3.z, uy), uz);
-    } else {
-      a0 = lattice_value(h0); a1 = lattice_value(h1); a2 = lattice_value(h2); a3 = lattice_value(h3);
-    }
-    const float ay0 = lerpf(a0, a1, uy), ay1 = lerpf(a2, a3, uy);
-    const float by0 = lerpf(b0, b1, uy), by1 = lerpf(b2, b3, uy);
-    const float A = lerpf(ay0, ay1, uz), B = lerpf(by0, by1, uz);
-    const float Ay = duy * lerpf(a1 - a0, a3 - a2, uz);
-    const float By = fmaf(duy, lerpf(b1 - b0, b3 - b2, uz), gy);
-    const float Az = duz * (ay1 - ay0);
-    const float Bz = fmaf(duz, by1 - by0, gz);
+    float2 v, vy, vz;
+    fold_column_d<NOISE>(c, p0, p1, p2.y, p2.z, (uint32_t)(t + __float_as_int(p2.x)), v, vy, vz);
     if (t < total) {
-      slice[t] = make_float2(A, B);
-      slice[total + t] = make_float2(Ay, By);
-      slice[2 * total + t] = make_float2(Az, Bz);
+      slice[t] = v;
+      slice[total + t] = vy;
+      slice[2 * total + t] = vz;
     }
   }
 }
 
-// n and dn/dq of one octave from the three planes (`total` entries apart).
+// n and dn/dq of one octave from the node's entry of the three planes (`plane` entries apart).
 template <int NOISE>
-__device__ __forceinline__ float col_read_d(float qx, int lo, const float2* region, int total, float& dx, float& dy,
-                                            float& dz) {
-  const float fx = floorf(qx);
-  const float tx = qx - fx, sx = tx - 1.0f;
-  const float ux = fade(tx), dux = dfade(tx);
-  const int o = (int)fx - lo;
-  const float2 e0 = region[o], e1 = region[o + 1];
-  const float2 y0 = region[total + o], y1 = region[total + o + 1];
-  const float2 z0 = region[2 * total + o], z1 = region[2 * total + o + 1];
+__device__ __forceinline__ float col_value_d(float tx, float ux, float dux, const float2* e, int plane, float& dx, float& dy,
+                                             float& dz) {
+  const float sx = tx - 1.0f;
+  const float2 e0 = e[0], e1 = e[1];
+  const float2 y0 = e[plane], y1 = e[plane + 1];
+  const float2 z0 = e[2 * plane], z1 = e[2 * plane + 1];
   if (NOISE == UPF_NOISE_VALUE) {
     dx = dux * (e1.x - e0.x);
     dy = lerpf(y0.x, y1.x, ux);
@@ -109,6 +117,14 @@ __device__ __forceinline__ float col_read_d(float qx, int lo, const float2* regi
   dy = lerpf(fmaf(y0.x, tx, y0.y), fmaf(y1.x, sx, y1.y), ux);
   dz = lerpf(fmaf(z0.x, tx, z0.y), fmaf(z1.x, sx, z1.y), ux);
   return lerpf(a0, a1, ux);
+}
+
+template <int NOISE>
+__device__ __forceinline__ float col_read_d(float qx, int lo, const float2* region, int total, float& dx, float& dy,
+                                            float& dz) {
+  const float fx = floorf(qx);
+  const float tx = qx - fx;
+  return col_value_d<NOISE>(tx, fade(tx), dfade(tx), region + ((int)fx - lo), total, dx, dy, dz);
 }
 
 // Cellular with derivatives: 63 lanes write one feature point each as float4.

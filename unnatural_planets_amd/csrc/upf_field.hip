@@ -14,6 +14,7 @@
 #include "upf_device_row_grad.hpp"
 #include "upf_device_tilex.hpp"
 #include "upf_device_band.hpp"
+#include "upf_device_band_grad.hpp"
 #include "upf_internal.hpp"
 
 namespace upf {
@@ -110,7 +111,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
 
 // Bands of kBandRows rows (upf_device_band.hpp), the same values as k_eval_grid_row.  512^3
 // torus at 7 waves a SIMD 863 us, at 6 909, at 8 (64 registers, spills) 928.
-template <bool COMPOSED>
+template <bool COMPOSED, bool WIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_eval_grid_band(
     const DSpec s, const DGrid g, float* __restrict__ out, uint64_t* __restrict__ S, float iso) {
   constexpr int R = kBandRows;
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
   const float z = node_coord(g.o[2], g.s[2], k);
   const RowCtx c = make_row_ctx(s_slice[wv], s_gtab, nullptr, lane);
   float v[R];
-  band_field<R, COMPOSED>(c, s, x, yl, z, v);
+  band_field<R, COMPOSED, WIDE>(c, s, x, yl, z, v);
   const int i = (int)blockIdx.x * kGridBX + lane_of(c);  // recomputed: not live across the layers
   const bool valid = i < g.n[0];
   const size_t row0 = ((size_t)k * g.n[1] + j) * g.n[0];
@@ -308,6 +309,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
   }
 }
 
+// The same over bands of kBandGradRows rows (upf_device_band_grad.hpp), for the specs that
+// band_grad_fits accepts.  Sixteen waves a workgroup, one workgroup a CU: the sums meet
+// dLdtheta in 256 float additions at most, whose rounding is most of a sum's error (256^3,
+// relative: 5.0e-7 of the row kernel's 1,536 workgroups, 7.0e-7 of 1,280 with four waves at
+// five a SIMD, 1.8e-7 so; that form ran 230 us against 243).
+constexpr int kBandGradWaves = 16;
+
+template <bool THETA, bool WIDE>
+__global__ __launch_bounds__(64 * kBandGradWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_adjoint_bands(const DSpec s, const DGrid g, int64_t items,
+                                                      const float* __restrict__ dLdf, float* __restrict__ fout,
+                                                      float* __restrict__ dfdx, float* __restrict__ dLdtheta) {
+  constexpr int R = kBandGradRows;
+  __shared__ float4 s_slice[kBandGradWaves][kRowSlice];
+  __shared__ float4 s_gtab[16];
+  __shared__ float th[kBandGradWaves][UPF_THETA_COUNT];
+  if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+  if (THETA)
+    for (int t = threadIdx.x; t < kBandGradWaves * UPF_THETA_COUNT; t += 64 * kBandGradWaves) (&th[0][0])[t] = 0.0f;
+  __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const RowCtx c = make_row_ctx(s_slice[wave], s_gtab, nullptr, threadIdx.x & 63);
+  ThetaAcc acc{th[wave]};
+  const int gpr = (g.n[0] + 63) / 64, bands = (g.n[1] + R - 1) / R;
+  const int64_t stride = (int64_t)gridDim.x * kBandGradWaves;
+  int64_t it = (int64_t)blockIdx.x * kBandGradWaves + wave;  // (k * bands + band) * gpr + xb, as k_adjoint_rows
+  int xb = (int)(it % gpr), band = (int)((it / gpr) % bands), k = (int)(it / gpr / bands);
+  const int sx = (int)(stride % gpr), sj = (int)((stride / gpr) % bands), sk = (int)(stride / gpr / bands);
+  for (; it < items; it += stride) {
+    const int lane = lane_of(c);
+    const int j = band * R, rows = min(R, g.n[1] - j);
+    const int64_t row0 = ((int64_t)k * g.n[1] + j) * g.n[0];
+    const int i = xb * 64 + lane;
+    const bool valid = i < g.n[0];
+    const int ic = min(i, g.n[0] - 1);
+    const float x = node_coord(g.o[0], g.s[0], ic);
+    const float yl = node_coord(g.o[1], g.s[1], j + min(lane & (R - 1), rows - 1));
+    const float z = node_coord(g.o[2], g.s[2], k);
+    float w[R], f[R], gr[R][3];
+#pragma unroll
+    for (int r = 0; r < R; r++) w[r] = THETA && valid && r < rows ? dLdf[row0 + (int64_t)r * g.n[0] + ic] : 0.0f;
+    band_field_grad<R, THETA, WIDE>(c, s, x, yl, z, w, f, gr, acc);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int64_t node = row0 + (int64_t)r * g.n[0] + xb * 64 + lane_of(c);
+      if (r < rows && xb * 64 + lane_of(c) < g.n[0]) {
+        if (fout) fout[node] = f[r];
+        if (dfdx) { dfdx[3 * node] = gr[r][0]; dfdx[3 * node + 1] = gr[r][1]; dfdx[3 * node + 2] = gr[r][2]; }
+      }
+    }
+    xb += sx;
+    const int cx = xb >= gpr;
+    xb -= cx ? gpr : 0;
+    band += sj + cx;
+    const int cj = band >= bands;
+    band -= cj ? bands : 0;
+    k += sk + cj;
+  }
+  if (THETA) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < UPF_THETA_COUNT; t += 64 * kBandGradWaves) {
+      float v = 0.0f;
+      for (int q = 0; q < kBandGradWaves; q++) v = v + th[q][t];
+      if (v != 0.0f) atomicAdd(dLdtheta + t, v);
+    }
+  }
+}
+
 namespace {
 int adjoint_blocks(int64_t n) {
   // enough workgroups to fill 256 CUs several times; capped so the per-block θ
@@ -357,7 +425,8 @@ int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int varian
   } else if (band_items(g) >= kBandItems && band_fits(s, g)) {
     constexpr int rows_per_block = kBandRows * kRowWaves;
     const dim3 blocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + rows_per_block - 1) / rows_per_block, g.n[2]);
-    const auto kernel = spec_composed(s) ? k_eval_grid_band<true> : k_eval_grid_band<false>;
+    const auto kernel = band_wide(s, g, kRowSlice2) ? (spec_composed(s) ? k_eval_grid_band<true, true> : k_eval_grid_band<false, true>)
+                                                    : (spec_composed(s) ? k_eval_grid_band<true, false> : k_eval_grid_band<false, false>);
     hipLaunchKernelGGL(kernel, blocks, dim3(kGridBX, kRowWaves, 1), 0, stream, s, g, d_field, S, iso);
   } else {
     constexpr int rows_per_block = kRowsPerWave * kRowWaves;
@@ -459,16 +528,16 @@ int upf_field_adjoint_grid(const upf_field_spec* spec, const upf_grid* grid, con
     UPF_LAUNCH_CHECK();
     return UPF_OK;
   }
-  const int64_t items = (int64_t)((g.n[0] + 63) / 64) * g.n[1] * g.n[2];
-  const void* kern = d_dLdtheta ? reinterpret_cast<const void*>(&k_adjoint_rows<true>)
-                                : reinterpret_cast<const void*>(&k_adjoint_rows<false>);
-  const int nb = (int)std::min<int64_t>((items + 3) / 4, (int64_t)resident_blocks(kern, 256));
-  if (d_dLdtheta)
-    hipLaunchKernelGGL((k_adjoint_rows<true>), dim3(nb), dim3(256), 0, as_stream(stream), s, g, items, d_dLdf, d_f,
-                       d_dfdx, d_dLdtheta);
-  else
-    hipLaunchKernelGGL((k_adjoint_rows<false>), dim3(nb), dim3(256), 0, as_stream(stream), s, g, items, d_dLdf,
-                       d_f, d_dfdx, d_dLdtheta);
+  const bool bands = band_grad_items(g) >= kBandItems && band_grad_fits(s, g);
+  const int64_t items = bands ? band_grad_items(g) : (int64_t)((g.n[0] + 63) / 64) * g.n[1] * g.n[2];
+  const bool wide = bands && band_wide(s, g, kRowSlice);
+  auto kernel = d_dLdtheta ? k_adjoint_rows<true> : k_adjoint_rows<false>;
+  if (wide) kernel = d_dLdtheta ? k_adjoint_bands<true, true> : k_adjoint_bands<false, true>;
+  else if (bands) kernel = d_dLdtheta ? k_adjoint_bands<true, false> : k_adjoint_bands<false, false>;
+  const int waves = bands ? kBandGradWaves : 4;
+  const int nb = (int)std::min<int64_t>((items + waves - 1) / waves,
+                                        (int64_t)resident_blocks(reinterpret_cast<const void*>(kernel), 64 * waves));
+  hipLaunchKernelGGL(kernel, dim3(nb), dim3(64 * waves), 0, as_stream(stream), s, g, items, d_dLdf, d_f, d_dfdx, d_dLdtheta);
   UPF_LAUNCH_CHECK();
   return UPF_OK;
 }
