@@ -309,6 +309,9 @@ __global__ __launch_bounds__(256) void k_bake(const DBake b, const float* __rest
                                               const float* __restrict__ uv, const int32_t* __restrict__ tri, int w,
                                               int h, float* __restrict__ albedo, float* __restrict__ bump,
                                               float* __restrict__ rough) {
+  __shared__ float4 s_gtab[16];
+  if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+  __syncthreads();
   const int x = blockIdx.x * 64 + (threadIdx.x & 63);
   const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
   if (x >= w || y >= h) return;
@@ -350,7 +353,7 @@ __global__ __launch_bounds__(256) void k_bake(const DBake b, const float* __rest
   // the shape and the detail noise round like the CPU restatement (X = true): the bands'
   // smoothsteps would amplify a few ulps of elevation by up to 150x
   const float elev = shape_eval<EXT, true, true>(b.field, p[0], p[1], p[2]) / b.field.escale;
-  const float d = b.detail.weight * layer_value<true>(b.detail, p[0], p[1], p[2]);
+  const float d = b.detail.weight * layer_value<true>(b.detail, p[0], p[1], p[2], GradTable{s_gtab});
   const float s1 = smoothstep_(b.bands[0] - b.band_width, b.bands[0] + b.band_width, elev);
   const float s2 = smoothstep_(b.bands[1] - b.band_width, b.bands[1] + b.band_width, elev);
   const float s3 = smoothstep_(b.bands[2] - b.band_width, b.bands[2] + b.band_width, elev);

@@ -124,6 +124,33 @@ __device__ __forceinline__ void gvec(uint32_t h, float& gx, float& gy, float& gz
   gz = vz ? sv : 0.0f;
 }
 
+// Where a noise takes its gradients from: computed by selects, or from a table of the 16 in
+// LDS, the same values (the components are -1, 0 and 1, two of them not 0, so the table's
+// products are exact and its sum rounds once, as the selects' +-u +- v does) in 5
+// instructions a corner instead of 14.  Kernels that fill the machine take the table (texel
+// bake 185 -> 160 us at 4096^2, narrow-band coarse pass 44 -> 34 us and normals 68 -> 45 us at
+// 1025^3); those of a few points keep the selects, which need no fill and no barrier.
+struct GradSelect {
+  __device__ __forceinline__ float dot(uint32_t h, float x, float y, float z) const { return gdot(h, x, y, z); }
+  __device__ __forceinline__ void vec(uint32_t h, float& gx, float& gy, float& gz) const { gvec(h, gx, gy, gz); }
+};
+struct GradTable {
+  const float4* t;
+  __device__ __forceinline__ float dot(uint32_t h, float x, float y, float z) const {
+    const float4 g = t[h >> 28];
+    return fmaf(g.z, z, fmaf(g.y, y, g.x * x));
+  }
+  __device__ __forceinline__ void vec(uint32_t h, float& gx, float& gy, float& gz) const {
+    const float4 g = t[h >> 28];
+    gx = g.x; gy = g.y; gz = g.z;
+  }
+};
+__device__ __forceinline__ float4 gradient_entry(int g) {
+  float gx, gy, gz;
+  gvec((uint32_t)g << 28, gx, gy, gz);
+  return make_float4(gx, gy, gz, 0.0f);
+}
+
 // Corner hashes of the lattice cell (ix, iy, iz): h[c] for c = x + 2y + 4z.
 __device__ __forceinline__ void cell_hashes(uint32_t seed, int ix, int iy, int iz, uint32_t h[8]) {
   const uint32_t x0 = (uint32_t)ix * kPX, x1 = x0 + kPX;
@@ -138,18 +165,18 @@ __device__ __forceinline__ void cell_hashes(uint32_t seed, int ix, int iy, int i
 }
 
 // ------------------------------------------------------------------ noise (values)
-template <bool X = false>
-__device__ __forceinline__ float noise_gradient(uint32_t seed, float qx, float qy, float qz) {
+template <bool X = false, class G = GradSelect>
+__device__ __forceinline__ float noise_gradient(uint32_t seed, float qx, float qy, float qz, const G& grad = G()) {
   const float fx = floorf(qx), fy = floorf(qy), fz = floorf(qz);
   uint32_t h[8];
   cell_hashes(seed, (int)fx, (int)fy, (int)fz, h);
   const float tx = qx - fx, ty = qy - fy, tz = qz - fz;
   const float sx = tx - 1.0f, sy = ty - 1.0f, sz = tz - 1.0f;
   const float ux = fade<X>(tx), uy = fade<X>(ty), uz = fade<X>(tz);
-  const float x00 = lerpf<X>(gdot(h[0], tx, ty, tz), gdot(h[1], sx, ty, tz), ux);
-  const float x10 = lerpf<X>(gdot(h[2], tx, sy, tz), gdot(h[3], sx, sy, tz), ux);
-  const float x01 = lerpf<X>(gdot(h[4], tx, ty, sz), gdot(h[5], sx, ty, sz), ux);
-  const float x11 = lerpf<X>(gdot(h[6], tx, sy, sz), gdot(h[7], sx, sy, sz), ux);
+  const float x00 = lerpf<X>(grad.dot(h[0], tx, ty, tz), grad.dot(h[1], sx, ty, tz), ux);
+  const float x10 = lerpf<X>(grad.dot(h[2], tx, sy, tz), grad.dot(h[3], sx, sy, tz), ux);
+  const float x01 = lerpf<X>(grad.dot(h[4], tx, ty, sz), grad.dot(h[5], sx, ty, sz), ux);
+  const float x11 = lerpf<X>(grad.dot(h[6], tx, sy, sz), grad.dot(h[7], sx, sy, sz), ux);
   return lerpf<X>(lerpf<X>(x00, x10, uy), lerpf<X>(x01, x11, uy), uz);
 }
 
@@ -319,28 +346,28 @@ __device__ __forceinline__ float shape_eval(const DSpec& s, float x, float y, fl
 }
 
 // ------------------------------------------------------------------ layers
-template <bool X = false>
-__device__ __forceinline__ float octave_noise(const DLayer& L, int k, float x, float y, float z) {
+template <bool X = false, class G = GradSelect>
+__device__ __forceinline__ float octave_noise(const DLayer& L, int k, float x, float y, float z, const G& grad = G()) {
   const float f = L.freq[k];
   const float qx = x * f, qy = y * f, qz = z * f;
   const uint32_t seed = L.seed + (uint32_t)k;
-  if (L.noise == UPF_NOISE_GRADIENT) return noise_gradient<X>(seed, qx, qy, qz);
+  if (L.noise == UPF_NOISE_GRADIENT) return noise_gradient<X>(seed, qx, qy, qz, grad);
   if (L.noise == UPF_NOISE_VALUE) return noise_value<X>(seed, qx, qy, qz);
   if (L.noise == UPF_NOISE_SIMPLEX) return noise_simplex(seed, qx, qy, qz);
   return noise_cellular<X>(seed, qx, qy, qz, L.js, L.j0);
 }
 
-template <bool X = false>
-__device__ __forceinline__ float layer_value(const DLayer& L, float x, float y, float z) {
-  if (L.fractal == UPF_FRACTAL_NONE) return octave_noise<X>(L, 0, x, y, z);
+template <bool X = false, class G = GradSelect>
+__device__ __forceinline__ float layer_value(const DLayer& L, float x, float y, float z, const G& grad = G()) {
+  if (L.fractal == UPF_FRACTAL_NONE) return octave_noise<X>(L, 0, x, y, z, grad);
   float acc = 0.0f;
   if (L.fractal == UPF_FRACTAL_RIDGED) {
     for (int k = 0; k < L.octaves; k++) {
-      const float n = octave_noise<X>(L, k, x, y, z);
+      const float n = octave_noise<X>(L, k, x, y, z, grad);
       acc = mad_x<X>(L.amp[k], mad_x<X>(-2.0f, fabsf(n), 1.0f), acc);
     }
   } else {
-    for (int k = 0; k < L.octaves; k++) acc = mad_x<X>(L.amp[k], octave_noise<X>(L, k, x, y, z), acc);
+    for (int k = 0; k < L.octaves; k++) acc = mad_x<X>(L.amp[k], octave_noise<X>(L, k, x, y, z, grad), acc);
   }
   return acc;
 }
@@ -350,8 +377,8 @@ __device__ __forceinline__ float layer_value(const DLayer& L, float x, float y, 
 // Voronoi parameters (seed, points per cell in octaves, cell size in freq[0]).
 // EXT = false compiles the modes and the further shapes out (the kernels' common
 // instantiation); specs with either run the EXT = true instantiations.
-template <bool EXT = true, bool X = false>
-__device__ __forceinline__ float elevation_eval(const DSpec& s, float x, float y, float z) {
+template <bool EXT = true, bool X = false, class G = GradSelect>
+__device__ __forceinline__ float elevation_eval(const DSpec& s, float x, float y, float z, const G& grad = G()) {
   const int mode = EXT ? s.mode : UPF_ELEV_LAYERS;
   ModeState<float> st;
   if (mode != UPF_ELEV_LAYERS) mode_begin(mode, s.L[0].seed, s.L[0].octaves, s.L[0].freq[0], x, y, z, 0.0f, st);
@@ -360,7 +387,7 @@ __device__ __forceinline__ float elevation_eval(const DSpec& s, float x, float y
     const DLayer& L = s.L[l];
     float px = x, py = y, pz = z;
     if (mode != UPF_ELEV_LAYERS) mode_position(mode, l, st, x, y, z, 0.0f, px, py, pz);
-    const float raw = layer_value<X>(L, px, py, pz);
+    const float raw = layer_value<X>(L, px, py, pz, grad);
     if (mode != UPF_ELEV_LAYERS) {
       if (mode_after(mode, l, raw, 0.0f, st)) break;
       continue;
@@ -377,12 +404,12 @@ __device__ __forceinline__ float elevation_eval(const DSpec& s, float x, float y
 // X = EXT by default: the per-lane kernels of the elevation modes and the further shapes
 // round like the CPU restatement (the modes' pow is upf_math.hpp's on both sides), so
 // their fields equal it bit for bit; the common kernels keep the fused form.
-template <bool EXT = true, bool X = EXT>
-__device__ __forceinline__ float field_eval(const DSpec& s, float x, float y, float z) {
+template <bool EXT = true, bool X = EXT, class G = GradSelect>
+__device__ __forceinline__ float field_eval(const DSpec& s, float x, float y, float z, const G& grad = G()) {
   const bool need_elev = s.compose == UPF_COMPOSE_LAND || s.compose == UPF_COMPOSE_NAVIGATION ||
                          s.compose == UPF_COMPOSE_ELEVATION_RAW;
   const float shape = s.compose == UPF_COMPOSE_ELEVATION_RAW ? 0.0f : shape_eval<EXT, true, X>(s, x, y, z);
-  const float elev = need_elev ? elevation_eval<EXT, X>(s, x, y, z) : 0.0f;
+  const float elev = need_elev ? elevation_eval<EXT, X>(s, x, y, z, grad) : 0.0f;
   switch (s.compose) {
     case UPF_COMPOSE_LAND: return shape - s.escale * elev;
     case UPF_COMPOSE_WATER: return shape;

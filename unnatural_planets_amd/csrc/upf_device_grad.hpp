@@ -17,8 +17,9 @@ namespace upf {
 
 // ------------------------------------------------------------------ noise + gradient
 // Returns n(q) and dn/dq.
+template <class G>
 __device__ __forceinline__ float noise_gradient_d(uint32_t seed, float qx, float qy, float qz,
-                                                  float& dx, float& dy, float& dz) {
+                                                  float& dx, float& dy, float& dz, const G& grad) {
   const float fx = floorf(qx), fy = floorf(qy), fz = floorf(qz);
   uint32_t h[8];
   cell_hashes(seed, (int)fx, (int)fy, (int)fz, h);
@@ -27,7 +28,7 @@ __device__ __forceinline__ float noise_gradient_d(uint32_t seed, float qx, float
   const float ux = fade(tx), uy = fade(ty), uz = fade(tz);
   float g[8][3];
 #pragma unroll
-  for (int c = 0; c < 8; c++) gvec(h[c], g[c][0], g[c][1], g[c][2]);
+  for (int c = 0; c < 8; c++) grad.vec(h[c], g[c][0], g[c][1], g[c][2]);
   float d[8];
 #pragma unroll
   for (int c = 0; c < 8; c++) {
@@ -111,12 +112,13 @@ __device__ __forceinline__ float noise_simplex_d(uint32_t seed, float qx, float 
   return 72.0f * n;
 }
 
+template <class G>
 __device__ __forceinline__ float octave_noise_d(const DLayer& L, int k, float x, float y, float z,
-                                                float& dx, float& dy, float& dz) {
+                                                float& dx, float& dy, float& dz, const G& grad) {
   const float f = L.freq[k];
   const float qx = x * f, qy = y * f, qz = z * f;
   const uint32_t seed = L.seed + (uint32_t)k;
-  if (L.noise == UPF_NOISE_GRADIENT) return noise_gradient_d(seed, qx, qy, qz, dx, dy, dz);
+  if (L.noise == UPF_NOISE_GRADIENT) return noise_gradient_d(seed, qx, qy, qz, dx, dy, dz, grad);
   if (L.noise == UPF_NOISE_VALUE) return noise_value_d(seed, qx, qy, qz, dx, dy, dz);
   if (L.noise == UPF_NOISE_SIMPLEX) return noise_simplex_d(seed, qx, qy, qz, dx, dy, dz);
   return noise_cellular_d(seed, qx, qy, qz, L.js, L.j0, dx, dy, dz);
@@ -267,14 +269,14 @@ __device__ __forceinline__ int shape_param_count(int shape) {
 
 // Layer contribution with gradient: adds coeff * dv/dp into g, and (THETA) the
 // per-octave dθ terms scaled by coeff_theta = dLdf * d f / d v.  Returns v (unweighted).
-template <bool THETA>
+template <bool THETA, class G = GradSelect>
 __device__ __forceinline__ float layer_grad(const DLayer& L, int l, float x, float y, float z, float coeff,
-                                            float coeff_theta, float g[3], ThetaAcc& acc) {
+                                            float coeff_theta, float g[3], ThetaAcc& acc, const G& grad = G()) {
   const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
   float v = 0.0f;
   for (int k = 0; k < oct; k++) {
     float nx, ny, nz;
-    const float n = octave_noise_d(L, k, x, y, z, nx, ny, nz);
+    const float n = octave_noise_d(L, k, x, y, z, nx, ny, nz, grad);
     float term, dterm;  // term(n) and d term / d n
     if (L.fractal == UPF_FRACTAL_NONE) { term = n; dterm = 1.0f; }
     else if (L.fractal == UPF_FRACTAL_RIDGED) {
@@ -298,7 +300,8 @@ __device__ __forceinline__ float layer_grad(const DLayer& L, int l, float x, flo
 // Elevation of a fixed mode with its position gradient (forward mode).  A layer sampled
 // at a position that is itself a function of the sample (the legacy mode's p * scale)
 // chains its lattice gradient through that position's derivatives.
-__device__ __forceinline__ Grad elevation_mode_grad(const DSpec& s, float x, float y, float z) {
+template <class G>
+__device__ __forceinline__ Grad elevation_mode_grad(const DSpec& s, float x, float y, float z, const G& grad) {
   const int mode = s.mode;
   const Grad gx = gvar(x, 0), gy = gvar(y, 1), gz = gvar(z, 2), zero = gc(0.0f);
   ModeState<Grad> st;
@@ -308,7 +311,7 @@ __device__ __forceinline__ Grad elevation_mode_grad(const DSpec& s, float x, flo
     mode_position(mode, l, st, gx, gy, gz, zero, px, py, pz);
     float g[3] = {0.0f, 0.0f, 0.0f};
     ThetaAcc none{nullptr};
-    const float v = layer_grad<false>(s.L[l], l, px.v, py.v, pz.v, 1.0f, 0.0f, g, none);
+    const float v = layer_grad<false>(s.L[l], l, px.v, py.v, pz.v, 1.0f, 0.0f, g, none, grad);
     const Grad lv = {v, g[0] * px.dx + g[1] * py.dx + g[2] * pz.dx, g[0] * px.dy + g[1] * py.dy + g[2] * pz.dy,
                      g[0] * px.dz + g[1] * py.dz + g[2] * pz.dz};
     if (mode_after(mode, l, lv, zero, st)) break;
@@ -319,9 +322,9 @@ __device__ __forceinline__ Grad elevation_mode_grad(const DSpec& s, float x, flo
 // f, df/dp and (THETA) dLdf * df/dθ for one sample.  EXT compiles in the modes and the
 // further shapes; with an elevation mode only the position gradient is formed (the
 // parameter gradient is defined for the layer stack).
-template <bool THETA, bool EXT = false>
+template <bool THETA, bool EXT = false, class G = GradSelect>
 __device__ __forceinline__ float field_grad(const DSpec& s, float x, float y, float z, float dLdf, float g[3],
-                                            ThetaAcc& acc) {
+                                            ThetaAcc& acc, const G& grad = G()) {
   float gs[3], dps[4];
   const bool need_shape = s.compose != UPF_COMPOSE_ELEVATION_RAW;
   const bool need_elev = s.compose == UPF_COMPOSE_LAND || s.compose == UPF_COMPOSE_NAVIGATION ||
@@ -341,7 +344,7 @@ __device__ __forceinline__ float field_grad(const DSpec& s, float x, float y, fl
     for (int i = 0; i < np; i++) acc.add(kThShape + i, dLdf * dshape * dps[i]);
   }
   if (EXT && !THETA && need_elev && s.mode != UPF_ELEV_LAYERS) {
-    const Grad e = elevation_mode_grad(s, x, y, z);
+    const Grad e = elevation_mode_grad(s, x, y, z, grad);
     if (s.compose == UPF_COMPOSE_ELEVATION_RAW) {
       g[0] = e.dx; g[1] = e.dy; g[2] = e.dz;
       return e.v;
@@ -368,7 +371,7 @@ __device__ __forceinline__ float field_grad(const DSpec& s, float x, float y, fl
     float acc0 = 0.0f, m = 0.0f;
     for (int l = 0; l < s.n_layers; l++) {
       const DLayer& L = s.L[l];
-      const float v = L.weight * layer_value(L, x, y, z);
+      const float v = L.weight * layer_value(L, x, y, z, grad);
       vv[l] = v; accin[l] = acc0; min_[l] = m;
       if (L.blend == UPF_BLEND_ADD) acc0 = acc0 + v;
       else if (L.blend == UPF_BLEND_MASK) m = __builtin_amdgcn_fmed3f(v + 0.5f, 0.0f, 1.0f);
@@ -405,7 +408,7 @@ __device__ __forceinline__ float field_grad(const DSpec& s, float x, float y, fl
   for (int l = 0; l < s.n_layers; l++) {
     const DLayer& L = s.L[l];
     const float k = fe * c[l];
-    const float v = layer_grad<THETA>(L, l, x, y, z, k, dLdf * k, g, acc);
+    const float v = layer_grad<THETA>(L, l, x, y, z, k, dLdf * k, g, acc, grad);
     elev2 = fmaf(L.weight, v, elev2);
     if (THETA) acc.add(kThWeight + l, dLdf * fe * cw[l] * v);
   }

@@ -20,13 +20,6 @@ namespace upf {
 constexpr int kRowSlice = 256;  // float4 entries of LDS per wave
 constexpr int kRowSlice2 = 2 * kRowSlice;  // the same slice as float2 entries
 
-// Gradient vectors of Perlin's 16-entry set, indexed by h >> 28 (see gdot()).
-__device__ __forceinline__ float4 gradient_entry(int g) {
-  float gx, gy, gz;
-  gvec((uint32_t)g << 28, gx, gy, gz);
-  return make_float4(gx, gy, gz, 0.0f);
-}
-
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();

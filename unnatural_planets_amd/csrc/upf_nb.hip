@@ -119,6 +119,9 @@ __device__ __forceinline__ int wg_exclusive_sum(int v, int* total) {
 template <bool EXT>
 __global__ __launch_bounds__(256) void k_nb_coarse(const DSpec s, const DGrid g, const NbDims d,
                                                    float* __restrict__ coarse) {
+  __shared__ float4 s_gtab[16];
+  if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+  __syncthreads();
   const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int cx = d.bx + 1, cy = d.by + 1;
   const int64_t n = (int64_t)cx * cy * (d.bz + 1);
@@ -127,7 +130,7 @@ __global__ __launch_bounds__(256) void k_nb_coarse(const DSpec s, const DGrid g,
   const int64_t r = c / cx;
   const int J = (int)(r % cy), K = (int)(r / cy);
   coarse[c] = field_eval<EXT>(s, node_coord(g.o[0], g.s[0], I * kB), node_coord(g.o[1], g.s[1], J * kB),
-                         node_coord(g.o[2], g.s[2], K * kB));
+                              node_coord(g.o[2], g.s[2], K * kB), GradTable{s_gtab});
 }
 
 __global__ __launch_bounds__(256) void k_nb_activity(const float* __restrict__ coarse, const NbDims d, float iso,
@@ -423,11 +426,14 @@ __global__ __launch_bounds__(kNbThreads) __attribute__((amdgpu_waves_per_eu(8)))
 template <bool EXT>
 __global__ __launch_bounds__(256) void k_nb_normals(const DSpec s, const float* __restrict__ pos, int64_t n,
                                                     float* __restrict__ nrm) {
+  __shared__ float4 s_gtab[16];
+  if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+  __syncthreads();
   const int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (v >= n) return;
   ThetaAcc none{nullptr};
   float gr[3];
-  (void)field_grad<false, EXT>(s, pos[3 * v], pos[3 * v + 1], pos[3 * v + 2], 0.0f, gr, none);
+  (void)field_grad<false, EXT>(s, pos[3 * v], pos[3 * v + 1], pos[3 * v + 2], 0.0f, gr, none, GradTable{s_gtab});
   const float len = __builtin_sqrtf(gr[0] * gr[0] + gr[1] * gr[1] + gr[2] * gr[2]);
   const float inv = len > 0.0f ? 1.0f / len : 0.0f;
   nrm[3 * v + 0] = gr[0] * inv;
