@@ -465,10 +465,15 @@ NbLayout nb_layout(const NbDims& d, int64_t max_active) {
   L.off_act = o; o = al256(o + sizeof(uint2) * (size_t)d.blocks);
   L.off_map = o; o = al256(o + 4 * (size_t)d.blocks);
   L.off_bricks = o; o = al256(o + 4 * (size_t)kBrick * max_active);
-  L.off_recs = o; o = al256(o + sizeof(uint2) * (size_t)kRows * max_active);
-  L.off_list = o; o = al256(o + sizeof(uint2) * (size_t)max_active);
+  // the blocks' records, then their list, in the room of a two-byte table of a brick's nodes;
+  // and a spare word per block: workspaces keep the sizes that callers have been given
+  static_assert(sizeof(uint2) * (kRows + 1) <= 2 * (size_t)kBrick, "records and list fit");
+  L.off_recs = o;
+  L.off_list = o + sizeof(uint2) * (size_t)kRows * max_active;
+  o = al256(o + 2 * (size_t)kBrick * max_active);
   L.off_bcounts = o; o = al256(o + 4 * (size_t)max_active);
   L.off_voff = o; o = al256(o + 4 * (size_t)max_active);
+  o = al256(o + 4 * (size_t)max_active);
   L.off_total_b = o; o = al256(o + 2 * sizeof(uint4));  // totals + unresolved counter
   L.bytes = o;
   return L;
@@ -504,7 +509,7 @@ struct NbWs {
 int nb_workspace(const NbDims& d, void* d_ws, size_t ws_bytes, NbWs* o) {
   const NbLayout L0 = nb_layout(d, 0);
   if (!d_ws || ws_bytes < L0.bytes) return UPF_ERR_WORKSPACE;
-  const size_t per = 4 * (size_t)kBrick + sizeof(uint2) * (kRows + 1) + 8;
+  const size_t per = 6 * (size_t)kBrick + 12;
   int64_t cap = std::min<int64_t>(d.blocks, (int64_t)((ws_bytes - L0.bytes) / per));
   while (cap > 0 && nb_layout(d, cap).bytes > ws_bytes) cap--;
   const NbLayout L = nb_layout(d, cap);
