@@ -33,13 +33,13 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_TFLOPS = 157.3   # MI355X FP32 vector, vendor figure (packed FP32)
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
-# HBM bytes per launch of k_eval_grid_row on the 512^3 workload as timed for `roofline`
-# (upf_field_eval_grid_ex, no sign words), from rocprofv3 --pmc: FETCH_SIZE 302 KiB (x 2.0
-# by the 1 GiB copy calibration: the kernel reads only its arguments) and WRITE_SIZE
-# 524288 KiB (x 1.0: each node written once, 512 MiB).  Launches that also store the
-# sign words read 576 MiB of writes: 16 MiB of 8-byte words counted as 64 MiB, each word
-# a partial line written by another workgroup (profiles/field_torus_ridged_voronoi_512.txt).
-FIELD_TRAFFIC_512 = 2 * 302 * 1024 + 524288 * 1024
+# HBM bytes per launch of k_eval_grid_band on the 512^3 workload as timed for `roofline`
+# (upf_field_eval_grid_ex, no sign words), from rocprofv3 --pmc: FETCH_SIZE 5,638 KiB (x 2.0
+# by the 1 GiB copy calibration) and WRITE_SIZE 912,800 KiB (x 1.0: each node written once,
+# 512 MiB, and the registers that seven waves per SIMD spill).  Launches that also store the
+# sign words read 1,064,900 KiB: 16 MiB of 8-byte words, each a partial line written by another
+# workgroup (profiles/field_torus_ridged_voronoi_512.txt).
+FIELD_TRAFFIC_512 = 2 * 5638 * 1024 + 912800 * 1024
 
 
 def cpu_model() -> str:
@@ -472,15 +472,15 @@ def bench_nb(upf, S, torch, reps: int, n: int = 1025, tex: int = 4096):
     #         at the spec's flops per sample (the vertex normals' gradient work is not
     #         counted);
     #   HBM:  the coarse corner field (written and read), the dense block -> rank map (4 B
-    #         per block, written and read), each active block's 9^3 brick (4 B per node)
-    #         and node table (2 B per node), each written once and read once, and the mesh
-    #         (24 B per vertex, 12 B per triangle) written.
+    #         per block, written and read) and the mesh (24 B per vertex, 12 B per triangle)
+    #         written; the bricks and row records of the crossed blocks, whose number stays
+    #         on the device, are not counted.
     nb_per_axis = (n - 1) // S.NB_BLOCK
     corners = (nb_per_axis + 1) ** 3
     mean_flops = float(np.mean([float(L.upf_flops_per_sample(ctypes.byref(sp_))) * (corners + a * 729)
                                 for (_, sp_), a in zip(planets, act)]))
-    mean_bytes = float(np.mean([2 * 4 * corners + 2 * 4 * blocks + a * 729 * (4 + 2) * 2 + 24 * int(st.n_vertices) +
-                                12 * int(st.n_triangles) for a, st in zip(act, stats)]))
+    mean_bytes = float(np.mean([2 * 4 * corners + 2 * 4 * blocks + 24 * int(st.n_vertices) +
+                                12 * int(st.n_triangles) for st in stats]))
     mesh_tflops = mean_flops / t_mesh / 1e12
     mesh_gbs = mean_bytes / t_mesh / 1e9
     # the bake: triangle id in + 20 B out per texel, UV and indices per triangle, position
@@ -708,7 +708,7 @@ def main() -> int:
         "mc_count_emit_ms": round(t_mc_sync * 1e3, 4),
         "field_plus_classify_ms": round(t_fused * 1e3, 4),
         "step_two_calls_ms": round(t_step_two * 1e3, 4),
-        "roofline": {"bound": "valu", "kernel": "k_eval_grid_row", "achieved": round(field_tflops, 3),
+        "roofline": {"bound": "valu", "kernel": "k_eval_grid_band", "achieved": round(field_tflops, 3),
                      "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": round(field_tflops / PEAK_FP32_TFLOPS, 4),
                      "traffic": FIELD_TRAFFIC_512 if nx == ny == nz == 512 else None},
         "roofline_mc": {"bound": "hbm", "kernel": "marching cubes (signs+classify+scan+emit, upf_mc_extract_async)", "achieved": round(mc_gbs, 1),
