@@ -181,6 +181,7 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
   __shared__ float s_fe[EXT ? kBrick : 1];
   __shared__ float4 s_slice[4][EXT ? 1 : kRowSlice];
   __shared__ float4 s_gtab[16];
+  __shared__ float2 s_yz[EXT ? 1 : 4 * kBrickRows * kBrickGroups];
   __shared__ uint64_t s_bits[EXT ? 1 : 4 * kBrickGroups];  // signs of the groups of rows
   __shared__ uint32_t s_row[kRows];                        // and of each row
   __shared__ int s_crossed;
@@ -216,21 +217,23 @@ __global__ __launch_bounds__(kNbThreads) void k_nb_fine(const DSpec s, const DGr
     // lane 7 * 9 = 63 stands in for node 8 of row 6
     static_assert(kBrickRows * kBrickGroups * 4 >= kBN * kBN, "four waves cover the brick's rows");
     if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
+    // the rows' coordinates, once a brick: the divisions by 9 took 50 of 877 vector
+    // instructions a wave
+    if (t < kBrickRows * kBrickGroups * 4) {
+      const int row = min(t, kRows - 1), k = row / kBN, j = row - k * kBN;
+      s_yz[t] = make_float2(node_coord(g.o[1], g.s[1], gj0 + j), node_coord(g.o[2], g.s[2], gk0 + k));
+    }
     __syncthreads();
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int wave = uniform((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     const RowCtx ctx = make_row_ctx(s_slice[wave], s_gtab, nullptr, lane);
     const bool node_lane = lane < kBrickRows * kBN;
     const int rl = node_lane ? lane / kBN : kBrickRows - 1;
     const int i = node_lane ? lane - rl * kBN : kBN - 1;
     const float x = node_coord(g.o[0], g.s[0], gi0 + i);
-    auto brick_row = [&](int rho) {
-      const int m = rho / kBrickRows;
-      return min(kBrickRows * (wave + 4 * m) + (rho - m * kBrickRows), kBN * kBN - 1);
-    };
-    auto yz = [&](int rho, float& yy, float& zz) {
-      const int br = brick_row(rho), kk = br / kBN, jj = br - kk * kBN;
-      yy = node_coord(g.o[1], g.s[1], gj0 + jj);
-      zz = node_coord(g.o[2], g.s[2], gk0 + kk);
+    auto yz = [&](int rho, float& yy, float& zz) {  // row rho = 7 m + r of the wave's: 7 (wave + 4 m) + r of the brick
+      const float2 c = s_yz[kBrickRows * wave + rho + 3 * kBrickRows * (rho / kBrickRows)];
+      yy = c.x;
+      zz = c.y;
     };
     float y[kBrickGroups], z[kBrickGroups];
 #pragma unroll
