@@ -1,4 +1,4 @@
-"""Grids of many rows are evaluated in bands of eight rows, smaller ones two rows at a time:
+"""Grids of many rows are evaluated in bands of eight or four rows, small ones two rows at a time:
 the same values.  A large grid is compared with its planes evaluated a few at a time, over
 ragged sides, all layer kinds and blends, spacings at which a wave spans few cells, more
 columns than a band's share and more than fit at all, bands over several cells and cells
@@ -9,8 +9,9 @@ from unnatural_planets_amd import spec as S
 
 pytestmark = pytest.mark.gpu
 
-# the fewest bands, ragged rows and row ends, one band a plane, too few rows for bands
-DIMS = [(64, 32, 1024), (65, 37, 300), (3, 9, 1030), (130, 5, 700), (130, 4, 700), (257, 66, 90)]
+# the fewest bands of eight, one fewer plane, the fewest of four, ragged rows and row ends, one
+# band a plane, too few rows for eight
+DIMS = [(64, 64, 1024), (64, 32, 1023), (64, 16, 512), (65, 37, 300), (3, 9, 1030), (130, 5, 700), (130, 4, 700), (257, 66, 90)]
 
 
 def _layers(kind):
@@ -79,7 +80,7 @@ def test_bands_are_rows(upf, shape, params, compose, kind, spacing, dims):
     s = S.field_spec(shape, params, _layers(kind), compose, 0.1)
     whole = upf.field_eval_grid(s, _grid(dims, spacing))
     assert torch.isfinite(whole).all()
-    for k in range(0, dims[2], 30):
+    for k in range(0, dims[2], 30):  # planes too few for bands
         k = min(k, dims[2] - 30)
         part = upf.field_eval_grid(s, _grid(dims, spacing, k, 30))
         assert torch.equal(whole[k:k + 30], part)

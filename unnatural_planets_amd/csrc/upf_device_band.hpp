@@ -33,8 +33,8 @@ constexpr int kWideCells = kWidePoints / 9;     // cells that 64 nodes may reach
 // (no simplex, and the octaves' spans over 64 nodes fit).  The bound covers the rounding of
 // the nodes' coordinates, so no wave needs more; near it the two-row form decides per wave.
 // A grid of four rows or fewer has no use for eight.
-inline bool band_fits(const DSpec& s, const DGrid& g) {
-  if (g.n[1] <= kBandRows / 2) return false;
+inline bool band_fits(const DSpec& s, const DGrid& g, int rows = kBandRows) {
+  if (g.n[1] <= rows / 2) return false;
   if (s.compose != UPF_COMPOSE_LAND && s.compose != UPF_COMPOSE_NAVIGATION && s.compose != UPF_COMPOSE_ELEVATION_RAW)
     return true;  // no layer is read
   const double step = std::fabs((double)g.s[0]);
@@ -72,13 +72,12 @@ inline bool band_wide(const DSpec& s, const DGrid& g, int slice) {
   return false;
 }
 
-// Bands of eight rows take a quarter of the two-row form's waves, and need 16 to a CU (four
-// workgroups).  5 octaves on a torus, two rows against eight: 64^3 (512 bands) 10.0 / 12.2
-// us, 96^3 14.1 / 16.8, 110^3 (3520) 17.2 / 16.7, 128^3 19.5 / 15.3, 256^3 99 / 55.
+// Bands that a batch (of eight rows) or a grid's adjoint (of four) needs for its waves to
+// fill the machine better than the row forms': 16 to a CU.
 constexpr int64_t kBandItems = 4096;
 
-inline int64_t band_items(const DGrid& g) {
-  return (int64_t)((g.n[0] + 63) / 64) * ((g.n[1] + kBandRows - 1) / kBandRows) * g.n[2];
+inline int64_t band_items(const DGrid& g, int rows = kBandRows) {
+  return (int64_t)((g.n[0] + 63) / 64) * ((g.n[1] + rows - 1) / rows) * g.n[2];
 }
 
 // Value v of row r's lane.
@@ -215,7 +214,7 @@ __device__ __forceinline__ void wide_points(const RowCtx& c, const DLayer& L, ui
 // One octave of a cellular layer whose lanes span more cells than the two-row form takes:
 // the distances in the order of the per-lane form, which that form then runs, the points
 // hashed once a wave.  Torus with six octaves and a cellular layer at 6 per unit, 240^3: 269
-// us with the layer per lane, 149 here.
+// us with the layer per lane, 143 here.
 template <int R>
 __device__ __forceinline__ void band_cellular_wide(const RowCtx& c, const DLayer& L, float f, uint32_t sk, float x, float yl,
                                                    float z, float* n) {

@@ -109,12 +109,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
   }
 }
 
-// Bands of kBandRows rows (upf_device_band.hpp), the same values as k_eval_grid_row.  512^3
+// Bands of R rows (upf_device_band.hpp), the same values as k_eval_grid_row.  512^3
 // torus at 7 waves a SIMD 863 us, at 6 909, at 8 (64 registers, spills) 928.
-template <bool COMPOSED, bool WIDE>
+template <int R, bool COMPOSED, bool WIDE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_eval_grid_band(
     const DSpec s, const DGrid g, float* __restrict__ out, uint64_t* __restrict__ S, float iso) {
-  constexpr int R = kBandRows;
   __shared__ float4 s_slice[kRowWaves][kRowSlice];
   __shared__ float4 s_gtab[16];
   if (threadIdx.y == 0 && threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
@@ -415,6 +414,26 @@ void exact_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, f
   else tilex_launch<1>(s, g, d_field, S, iso, stream);
 }
 
+// The rows of a band by the number of bands: eight from 8,192 on, which fill the machine about
+// four times, four below, two rows (k_eval_grid_row) where even those are few.  5 octaves on
+// a torus, eight / four: 128^3 (4,096 bands of eight) 16.2 / 15.7 us, 144^3 22.3 / 22.1, 160^3
+// (9,600) 24.7 / 25.0, 256^3 55 / 63; four / two: 64^3 (1,024 of four) 10.3 / 10.0, 72^3 10.6 /
+// 11.8, 127^3 14.8 / 19.7.  Layers of band_cellular_wide in bands of four only, which hold its
+// distances without spilling (4 octaves of cells at 400^3 1,592 / 1,211 us, a torus with one
+// such layer at 310^3 225 / 231).
+constexpr int64_t kBandGridItems = 8192;
+constexpr int kHalfBandRows = 4;
+constexpr int64_t kHalfBandItems = 2048;
+
+template <int R>
+void band_launch(const DSpec& s, const DGrid& g, bool wide, float* d_field, uint64_t* S, float iso, hipStream_t stream) {
+  const dim3 blocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + R * kRowWaves - 1) / (R * kRowWaves), g.n[2]);
+  constexpr bool W = R == kHalfBandRows;
+  const auto kernel = W && wide ? (spec_composed(s) ? k_eval_grid_band<R, true, W> : k_eval_grid_band<R, false, W>)
+                                : (spec_composed(s) ? k_eval_grid_band<R, true, false> : k_eval_grid_band<R, false, false>);
+  hipLaunchKernelGGL(kernel, blocks, dim3(kGridBX, kRowWaves, 1), 0, stream, s, g, d_field, S, iso);
+}
+
 int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int variant, uint64_t* S, float iso,
                       hipStream_t stream) {
   if (variant < 0 || variant > UPF_EVAL_PER_LANE) return UPF_ERR_BAD_SPEC;
@@ -422,12 +441,10 @@ int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int varian
     lanes_launch(s, g, d_field, S, iso, stream);
   } else if (spec_ext(s)) {  // the row form covers the layer stack and the common shapes
     exact_launch(s, g, d_field, S, iso, stream);
-  } else if (band_items(g) >= kBandItems && band_fits(s, g)) {
-    constexpr int rows_per_block = kBandRows * kRowWaves;
-    const dim3 blocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + rows_per_block - 1) / rows_per_block, g.n[2]);
-    const auto kernel = band_wide(s, g, kRowSlice2) ? (spec_composed(s) ? k_eval_grid_band<true, true> : k_eval_grid_band<false, true>)
-                                                    : (spec_composed(s) ? k_eval_grid_band<true, false> : k_eval_grid_band<false, false>);
-    hipLaunchKernelGGL(kernel, blocks, dim3(kGridBX, kRowWaves, 1), 0, stream, s, g, d_field, S, iso);
+  } else if (band_items(g) >= kBandGridItems && band_fits(s, g) && !band_wide(s, g, kRowSlice2)) {
+    band_launch<kBandRows>(s, g, false, d_field, S, iso, stream);
+  } else if (band_items(g, kHalfBandRows) >= kHalfBandItems && band_fits(s, g, kHalfBandRows)) {
+    band_launch<kHalfBandRows>(s, g, band_wide(s, g, kRowSlice2), d_field, S, iso, stream);
   } else {
     constexpr int rows_per_block = kRowsPerWave * kRowWaves;
     const dim3 rblocks((g.n[0] + kGridBX - 1) / kGridBX, (g.n[1] + rows_per_block - 1) / rows_per_block, g.n[2]);
