@@ -519,23 +519,32 @@ struct BrickLane {
   float y, z;
 };
 
+// Whether the columns of a layer's octaves are at most `most` for certain, for rows from x0
+// to x1; sum: of the octaves' frequencies.  An octave has floor(x1 f) - floor(x0 f) + 2
+// columns, at most |x1 - x0| f + 3 and what the products round, f (|x0| + |x1|) 2^-24: far
+// from the origin whole cells.  The margins cover this sum's own roundings; infinities and
+// NaN are not certain.
+__host__ __device__ __forceinline__ bool brick_columns_fit(float sum, int oct, float x0, float x1, int most) {
+  const float reach = 1.01f * fabsf(x1 - x0) + 0x1p-21f * fmaxf(fabsf(x0), fabsf(x1));
+  return 4.0f * (float)oct + reach * sum <= (float)most;
+}
+
 // Whether a layer's columns over all octaves, times the rows of M groups, exceed the slice.
 template <int M>
 __device__ __forceinline__ bool brick_per_lane(const DLayer& L, int oct, float x) {
   constexpr int most = kRowSlice2 / (kBrickRows * M);
-  // columns <= 3 + |x span| f, roundings included, unless the spans are huge
   float sum = 0.0f;
   for (int k = 0; k < oct; k++) sum = sum + fabsf(L.freq[k]);
   const float x0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 0));
   const float x1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
-  if (4.0f * (float)oct + 1.01f * fabsf(x1 - x0) * sum <= (float)most) return false;
-  int total = 0;
+  if (brick_columns_fit(sum, oct, x0, x1, most)) return false;
+  uint32_t total = 0;
   for (int k = 0; k < oct; k++) {
     int lo, hi;
     lane_range((int)floorf(x * L.freq[k]), lo, hi);
-    total += hi - lo + 2;
+    total += min((uint32_t)hi - (uint32_t)lo, (uint32_t)most) + 2u;  // a span of 2^31 cells does not wrap
   }
-  return total > most;
+  return total > (uint32_t)most;
 }
 
 // One gradient / value layer at this lane's M nodes (x, y[m], z[m]) of rows
