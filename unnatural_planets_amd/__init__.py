@@ -642,7 +642,8 @@ def texture_post(tex: Textures, rounds: int = 7, stream=None):
     if rounds > spec_mod.POST_MAX_ROUNDS or r.dim() != 2:
         special = torch.stack([r, torch.where(torch.isnan(r), r, torch.zeros_like(r))], dim=2).contiguous()
         return texture_post_images(tex.albedo, special, tex.bump, rounds, stream)
-    return _images_post((tex.albedo, r, tex.bump), (None, 2, None), rounds, stream)
+    # the special map is made from the roughness, whose strides are free; the others are the caller's images
+    return _images_post((tex.albedo, r.contiguous(), tex.bump), (None, 2, None), rounds, stream)
 
 
 def _images_post(images, out_channels, rounds, stream):
