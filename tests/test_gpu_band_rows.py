@@ -1,7 +1,8 @@
 """The band kernels (eight rows a wave, four, and the adjoint's four) against the row pairs, whose
 values they share: each grid's planes evaluated again in parts of too few bands.  The counts
 that the dispatch goes by are asserted, so that a moved bound cannot turn a comparison into one
-of a kernel with itself.  Ragged rows, row ends and last bands."""
+of a kernel with itself.  Ragged rows, row ends and last bands; planes of few rows, on both
+sides of the bounds; cells whose rows are too far apart to share their points."""
 import pytest
 
 from unnatural_planets_amd import spec as S
@@ -61,11 +62,33 @@ def _check_field(upf, kind, compose, dims, spacing):
 
 
 @pytest.mark.parametrize("dims,eight", [((64, 64, 1024), True), ((64, 64, 1023), False), ((65, 37, 820), True), ((130, 17, 911), True),
-                                        ((257, 66, 184), True), ((3, 13, 4100), True), ((3, 5, 8200), True), ((193, 39, 1050), True)])
+                                        ((257, 66, 184), True), ((3, 13, 4100), True), ((3, 12, 4100), False), ((193, 39, 1050), True)])
 @pytest.mark.parametrize("kind,step", [("blends", 0.5), ("blends", 8.0), ("columns", 0.5), ("columns", 2.0), ("cells", 1.0)])
 def test_eight_rows(upf, kind, step, dims, eight):
-    assert (_bands(dims, 8) >= FIELD8 and dims[1] >= 5) == eight and _bands(dims, 4) >= FIELD4
+    assert (_bands(dims, 8) >= FIELD8 and dims[1] >= 13) == eight and _bands(dims, 4) >= FIELD4
     _check_field(upf, kind, "land", dims, (step, 1.5 * step, 0.5 * step))
+
+
+@pytest.mark.parametrize("rows", [2, 3, 4, 5, 6, 7, 8, 12, 13, 14])
+@pytest.mark.parametrize("kind,compose", [("blends", "land"), ("cells", "elevation_raw"), ("none", "land"), ("blends", "water")])
+def test_planes_of_few_rows(upf, rows, kind, compose):
+    dims = (70, rows, 4200)
+    assert _bands(dims, 8) >= FIELD8
+    _check_field(upf, kind, compose, dims, (1.0, 1.0, 1.0))
+
+
+# rows 0.1 to 6 cells apart, over few cells along x or many
+@pytest.mark.parametrize("apart", [4.0, 24.0, 26.0, 33.0, 34.0, 52.0, 53.0, 256.0])
+@pytest.mark.parametrize("step", [0.5, 8.0])
+def test_rows_far_apart(upf, step, apart):
+    import torch
+    dims = (130, 17, 911)
+    _check_field(upf, "cells", "land", dims, (step, apart, 1.0))
+    s = S.field_spec("none", (), _layers("cells"), "elevation_raw")
+    f, dfdx, _ = upf.field_adjoint_grid(s, _grid(dims, (step, apart, 1.0)), None)
+    for k, n in _parts(dims, 4, GRAD4):
+        pf, pd, _ = upf.field_adjoint_grid(s, _grid(dims, (step, apart, 1.0), k, n), None)
+        assert torch.equal(f[k:k + n], pf) and torch.equal(dfdx[k:k + n], pd)
 
 
 def test_signs_and_mesh(upf):

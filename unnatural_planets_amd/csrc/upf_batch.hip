@@ -412,11 +412,13 @@ int upf_batch_create(const upf_chunk* chunks, int32_t n_chunks, const upf_batch_
   }
   // bands for the chunks that fit them, if there are enough bands to fill the machine (and
   // no chunk makes the whole batch run per lane)
+  // (a grid of four rows or fewer has no use for eight)
+  const auto fits = [](const BChunk& C) { return C.grid.n[1] > kBandRows / 2 && band_fits(C.spec, C.grid); };
   int64_t bands = 0;
   for (const BChunk& C : b->host)
-    if (band_fits(C.spec, C.grid)) bands += band_items(C.grid);
+    if (fits(C)) bands += band_items(C.grid);
   for (BChunk& C : b->host) {
-    const int list = !b->any_ext && bands >= kBandItems && band_fits(C.spec, C.grid);
+    const int list = !b->any_ext && bands >= kBandItems && fits(C);
     if (list && band_wide(C.spec, C.grid, kRowSlice2)) b->any_wide = true;
     for (int l = 0; l < 2; l++) C.item_off[l] = b->items[l];
     b->items[list] += (int64_t)C.gx * item_rows(C.grid, list) * C.grid.n[2];

@@ -29,14 +29,26 @@ static_assert(kBandRows * kBandStride <= kRowSlice2 && UPF_MAX_OCTAVES * kBandSt
 constexpr int kWidePoints = 4 * kRowSlice / 3;  // feature points in the slice: x, y, z
 constexpr int kWideCells = kWidePoints / 9;     // cells that 64 nodes may reach along x
 
+inline bool reads_layers(const DSpec& s) {
+  return s.n_layers > 0 && (s.compose == UPF_COMPOSE_LAND || s.compose == UPF_COMPOSE_NAVIGATION || s.compose == UPF_COMPOSE_ELEVATION_RAW);
+}
+
+// A band hashes a cellular octave's points once a row of cells, so rows far apart make them
+// anew, for lanes that hold no more nodes.  512 x 64 x 300 nodes 8 m apart along x, with two
+// cellular octaves, the rows `pitch` of the finer one's cells apart, row pairs / bands of four
+// / of eight: at most 4 cells spanned, pitch 0.5 75 / 58 / 60 us, 1.2 75 / 72 / 75, 3 75 / 77 /
+// 82 (with four octaves of gradient noise 84 / 66 / 65); 12 cells (band_cellular_wide), 0.7
+// 219 / 183 / -, 0.9 219 / 214 / -, 1.2 219 / 236 / -, and with the gradient noise 0.7 146 /
+// 138 / -, 0.9 147 / 154 / -; their adjoint (48 rows of 150 planes) 0.5 140 / 145 and 133 /
+// 120, 0.7 140 / 153.
+constexpr double kNearCells = 3.9;       // spanned by 64 nodes: the two-row form's reach (cells_in_slice)
+constexpr double kNearPitch = 1.25, kWidePitch = 0.8, kWideGradPitch = 0.6;
+
 // Whether every wave of a grid evaluates every layer of the spec in LDS, as columns or cells
 // (no simplex, and the octaves' spans over 64 nodes fit).  The bound covers the rounding of
 // the nodes' coordinates, so no wave needs more; near it the two-row form decides per wave.
-// A grid of four rows or fewer has no use for eight.
-inline bool band_fits(const DSpec& s, const DGrid& g, int rows = kBandRows) {
-  if (g.n[1] <= rows / 2) return false;
-  if (s.compose != UPF_COMPOSE_LAND && s.compose != UPF_COMPOSE_NAVIGATION && s.compose != UPF_COMPOSE_ELEVATION_RAW)
-    return true;  // no layer is read
+inline bool band_fits(const DSpec& s, const DGrid& g) {
+  if (!reads_layers(s)) return true;
   const double step = std::fabs((double)g.s[0]);
   const double reach = std::fabs((double)g.o[0]) + step * g.n[0];
   for (int l = 0; l < s.n_layers; l++) {
@@ -47,7 +59,7 @@ inline bool band_fits(const DSpec& s, const DGrid& g, int rows = kBandRows) {
     for (int k = 0; k < oct; k++) {
       const double f = std::fabs((double)L.freq[k]);
       const double span = f * (63.0 * step + reach * 0x1p-21);  // cells from end to end
-      if (L.noise == UPF_NOISE_CELLULAR && !(span <= kWideCells - 3.1)) return false;
+      if (L.noise == UPF_NOISE_CELLULAR && !(span <= kWideCells - 3.1 && (span <= kNearCells || f * g.s[1] <= kWidePitch))) return false;
       columns += span + 3.0;
     }
     if (L.noise != UPF_NOISE_CELLULAR && !(columns <= kRowSlice2)) return false;
@@ -67,7 +79,19 @@ inline bool band_wide(const DSpec& s, const DGrid& g, int slice) {
     const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
     if (72 * oct > slice) return true;
     for (int k = 0; k < oct; k++)
-      if (!(std::fabs((double)L.freq[k]) * (63.0 * step + reach * 0x1p-21) <= 3.9)) return true;
+      if (!(std::fabs((double)L.freq[k]) * (63.0 * step + reach * 0x1p-21) <= kNearCells)) return true;
+  }
+  return false;
+}
+
+// Whether a cellular octave's rows lie too far apart for bands of eight.
+inline bool band_far(const DSpec& s, const DGrid& g) {
+  if (!reads_layers(s)) return false;
+  for (int l = 0; l < s.n_layers; l++) {
+    const DLayer& L = s.L[l];
+    if (L.noise != UPF_NOISE_CELLULAR) continue;
+    for (int k = 0; k < (L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves); k++)
+      if (std::fabs((double)L.freq[k]) * g.s[1] > kNearPitch) return true;
   }
   return false;
 }

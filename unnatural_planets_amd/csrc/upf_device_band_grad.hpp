@@ -36,8 +36,10 @@ inline bool band_grad_fits(const DSpec& s, const DGrid& g) {
     const int oct = L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
     double columns = 0.0;
     for (int k = 0; k < oct; k++) {
-      const double span = std::fabs((double)L.freq[k]) * (63.0 * step + reach * 0x1p-21);
+      const double f = std::fabs((double)L.freq[k]);
+      const double span = f * (63.0 * step + reach * 0x1p-21);
       if (!(span <= (cell ? kWideCells - 3.1 : kBandGradStride - 2.1))) return false;
+      if (cell && span > kNearCells && f * g.s[1] > kWideGradPitch) return false;
       columns += span + 3.0;
     }
     if (!cell && !(3.0 * columns <= kRowSlice2)) return false;

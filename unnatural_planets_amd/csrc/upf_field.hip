@@ -414,16 +414,29 @@ void exact_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, f
   else tilex_launch<1>(s, g, d_field, S, iso, stream);
 }
 
-// The rows of a band by the number of bands: eight from 8,192 on, which fill the machine about
-// four times, four below, two rows (k_eval_grid_row) where even those are few.  5 octaves on
-// a torus, eight / four: 128^3 (4,096 bands of eight) 16.2 / 15.7 us, 144^3 22.3 / 22.1, 160^3
-// (9,600) 24.7 / 25.0, 256^3 55 / 63; four / two: 64^3 (1,024 of four) 10.3 / 10.0, 72^3 10.6 /
-// 11.8, 127^3 14.8 / 19.7.  Layers of band_cellular_wide in bands of four only, which hold its
-// distances without spilling (4 octaves of cells at 400^3 1,592 / 1,211 us, a torus with one
-// such layer at 310^3 225 / 231).
+// The rows of a band by the number of bands: eight from 8,192 on (a little more than the
+// machine's 7,168 waves of seven a SIMD), four below, two rows (k_eval_grid_row) where even
+// those are few.  5 octaves on a torus, eight / four: 128^3 (4,096 bands of eight) 16.2 / 15.7
+// us, 144^3 22.3 / 22.1, 160^3 (9,600) 24.7 / 25.0, 256^3 55 / 63; four / two: 64^3 (1,024 of
+// four) 10.3 / 10.0, 72^3 10.6 / 11.8, 127^3 14.8 / 19.7.  Layers of band_cellular_wide in bands
+// of four only, which hold its distances without spilling (4 octaves of cells at 400^3 1,592 /
+// 1,211 us, a torus with one such layer at 310^3 225 / 231).
+// And by the rows of a plane, whose last band stands for rows that are not there and whose
+// workgroup, of four bands, for bands that are not: 512 x 60,000 nodes in planes of 3 to
+// 13 rows, the same octaves, eight / four / two: 4 rows - / 238 / 251, 5 rows 258 / 228 / 233, 9
+// rows 177 / 155 / 305, 12 rows 135 / 119 / 232, 13 rows 125 / 132 / 213 (64 x 5 x 20000 nodes
+// with more than 64 columns an octave 137 / 116 / 108); the shape alone: 3 rows - / 85 / 81, 6
+// rows 72 / 52 / 49, 7 rows 63 / 45 / 49.
 constexpr int64_t kBandGridItems = 8192;
+constexpr int kBandGridRows = 13;
 constexpr int kHalfBandRows = 4;
 constexpr int64_t kHalfBandItems = 2048;
+
+bool half_band_rows(const DSpec& s, const DGrid& g) {
+  const int rows = g.n[1];
+  if (rows >= kBandGridRows) return true;
+  return (rows > 6 || (reads_layers(s) && rows > 2 && rows <= kHalfBandRows)) && !band_far(s, g);
+}
 
 template <int R>
 void band_launch(const DSpec& s, const DGrid& g, bool wide, float* d_field, uint64_t* S, float iso, hipStream_t stream) {
@@ -441,9 +454,9 @@ int field_grid_launch(const DSpec& s, const DGrid& g, float* d_field, int varian
     lanes_launch(s, g, d_field, S, iso, stream);
   } else if (spec_ext(s)) {  // the row form covers the layer stack and the common shapes
     exact_launch(s, g, d_field, S, iso, stream);
-  } else if (band_items(g) >= kBandGridItems && band_fits(s, g) && !band_wide(s, g, kRowSlice2)) {
+  } else if (band_items(g) >= kBandGridItems && g.n[1] >= kBandGridRows && band_fits(s, g) && !band_wide(s, g, kRowSlice2) && !band_far(s, g)) {
     band_launch<kBandRows>(s, g, false, d_field, S, iso, stream);
-  } else if (band_items(g, kHalfBandRows) >= kHalfBandItems && band_fits(s, g, kHalfBandRows)) {
+  } else if (band_items(g, kHalfBandRows) >= kHalfBandItems && half_band_rows(s, g) && band_fits(s, g)) {
     band_launch<kHalfBandRows>(s, g, band_wide(s, g, kRowSlice2), d_field, S, iso, stream);
   } else {
     constexpr int rows_per_block = kRowsPerWave * kRowWaves;
