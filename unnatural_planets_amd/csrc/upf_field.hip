@@ -400,18 +400,60 @@ void tilex_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, f
   hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, stream, s, g, d_field, reinterpret_cast<uint16_t*>(S), iso);
 }
 
-// The exact form's kernel by the number of nodes.  From 128^3 nodes four planes a wave share
-// its lattice work (400^3: lakes 2,805 us per lane, 1,185 in tiles; craters 11,142 and 1,523;
-// legacy 1,483 and 1,043).  Below, four planes leave too few waves (48^3 lakes: 14.8 us per
-// lane, 28 with four planes, 15.2 with one): one plane a wave, but per lane for the legacy
-// mode and the layer stack, most of whose layers the tiles evaluate per lane anyway (110^3
-// legacy: 39.4 us per lane, 43.7 in one-plane tiles).
-constexpr int64_t kTileNodes = (int64_t)1 << 21;
+// The exact form's kernel.  From 2^21 nodes on (128^3) four planes a wave share its lattice work
+// (400^3: lakes 2,805 us per lane, 1,185 in tiles; craters 11,142 and 1,523; legacy 1,483 and
+// 1,043).  Below, four planes leave too few waves (48^3 lakes: 14.8 us per lane, 28 with four
+// planes, 15.2 with one): one plane a wave, but per lane for the legacy mode and the layer
+// stack, most of whose layers the tiles evaluate per lane anyway (110^3 legacy: 39.4 us per
+// lane, 43.7 in one-plane tiles).
+// What four planes save depends on the layers, and it has to pay for the nodes that a tile's
+// 4 rows and 4 planes stand for beyond the grid (`py` and `pz` times the grid's).  Microseconds
+// per lane / one plane / four, for 2048 x 2048 nodes of 2 planes, then for 2048 x 2 x 2048:
+//   masked (lakes, islands) or shared (craters) work: lakes 327 / 227 / 322, 363 / 468 / 327
+//     (3 planes 488 / 336 / 322); craters 1,308 / 232 / 371
+//   gradient and value layers alone: 5 octaves on the gear 183 / 160 / 210, 207 / 315 / 212 (5
+//     planes 450 / 393 / 412)
+//   these among others: legacy 157 / 184 / 252, 180 / 364 / 253 (5 planes 382 / 452 / 492, 5 rows
+//     423 / 722 / 494); 11 octaves of all kinds 484 / 535 / 906, 636 / 1,061 / 909 (9
+//     rows at 1024 567 / 797 / 687; 700 x 5 x 700 167 / - / 234, but 1024 x 5 x 1024 482 / 534 /
+//     461)
+//   none: simple 181 / 165 / 308, 209 / 325 / 310 (5 planes 444 / 404 / 607, 5 rows 477 / 645 /
+//     607); cells on the gear 372 / 365 / 714, 452 / 722 / 717 (at 1024 9 rows 441 / 546 /
+//     541); these from 2^16 tiles of a plane on, 2^22 nodes (mandelbulb 128^3 332 / 293 / 387,
+//     256^3 2,013 / 1,908 / 2,126; simple 128^3 50 / 45 / 49, 200^3 225 / 201 / 195; 2 x 1024 x
+//     1024 1,463 / 580 / 512).
+constexpr int64_t kTileNodes = (int64_t)1 << 21, kLaneTiles = (int64_t)1 << 16;
+
+// Octaves of the layers read whose lattices a tile's planes share, and the others.
+void tile_octaves(const DSpec& s, int* shared, int* other) {
+  *shared = *other = 0;
+  for (int l = 0; reads_layers(s) && l < s.n_layers; l++) {
+    const DLayer& L = s.L[l];
+    const bool lattice = (L.noise == UPF_NOISE_GRADIENT || L.noise == UPF_NOISE_VALUE) && !(s.mode == UPF_ELEV_LEGACY && l == 1);
+    (lattice ? *shared : *other) += L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves;
+  }
+}
 
 void exact_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, float iso, hipStream_t stream) {
-  if ((int64_t)g.n[0] * g.n[1] * g.n[2] >= kTileNodes) tilex_launch<4>(s, g, d_field, S, iso, stream);
-  else if (s.mode == UPF_ELEV_LEGACY || s.mode == UPF_ELEV_LAYERS) lanes_launch(s, g, d_field, S, iso, stream);
-  else tilex_launch<1>(s, g, d_field, S, iso, stream);
+  const bool hills = reads_layers(s) && (s.mode == UPF_ELEV_LAKES || s.mode == UPF_ELEV_ISLANDS);
+  const bool craters = reads_layers(s) && s.mode == UPF_ELEV_CRATERS, stack = s.mode == UPF_ELEV_LAYERS;
+  int shared, other;
+  tile_octaves(s, &shared, &other);
+  const auto padded = [](int n) { return (double)((n + 3) / 4 * 4) / n; };
+  const double py = padded(g.n[1]), pz = padded(g.n[2]);
+  const bool lattices = shared && !other;
+  const bool rows_fit = hills || craters || py <= (stack ? (lattices ? 1.7 : 1.15) : 1.5);
+  const bool planes_fit = pz <= (hills || craters || lattices ? 1.7 : 1.15);
+  const int64_t nodes = (int64_t)g.n[0] * g.n[1] * g.n[2];
+  const int64_t tiles = (int64_t)((g.n[0] + kTX - 1) / kTX) * ((g.n[1] + kTY - 1) / kTY) * g.n[2];  // of a plane each
+  if (rows_fit && planes_fit && nodes >= kTileNodes && (hills || craters || shared || tiles >= kLaneTiles)) {
+    tilex_launch<4>(s, g, d_field, S, iso, stream);
+  } else if (!craters && (g.n[1] == 2 || (nodes >= kTileNodes && !rows_fit) ||
+                          ((stack || s.mode == UPF_ELEV_LEGACY) && (shared || nodes < kTileNodes)))) {
+    lanes_launch(s, g, d_field, S, iso, stream);
+  } else {
+    tilex_launch<1>(s, g, d_field, S, iso, stream);
+  }
 }
 
 // The rows of a band by the number of bands: eight from 8,192 on (a little more than the
