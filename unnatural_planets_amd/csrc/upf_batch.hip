@@ -3,8 +3,9 @@
 // sources/generator.cpp:159).
 //
 // Work items, enumerated chunk after chunk:
-//   field     64 x nodes of a band of eight grid rows or of a pair (chunk, xb, band, k),
-//             which also stores the rows' sign words: one item per wave over all chunks'
+//   field     64 x nodes of a pair of grid rows or of a band of eight or four (chunk, xb,
+//             band, k), which also stores the rows' sign words: one item per wave over all
+//             chunks', a list of items per kind
 //   classify  one marching-cubes group per lane, from the sign words alone
 //   emit      packed passes over the active groups of the concatenated scan, on a
 //             fixed grid
@@ -27,6 +28,12 @@ namespace upf {
 
 #include "upf_mc_device.hpp"
 
+// The lists of items: row pairs, bands, and bands of four for cellular layers past the pairs'
+// reach (band_wide), whose distances do not fit the registers for eight rows, or whose rows
+// lie too far apart for eight (band_far).  And the rows of their items.
+enum { kPairList = 0, kBandList = 1, kWideList = 2, kLists = 3 };
+constexpr int kItemRows[kLists] = {2, kBandRows, 4};
+
 struct BChunk {
   DSpec spec;
   DGrid grid;
@@ -35,7 +42,7 @@ struct BChunk {
   int32_t gx;          // 64-node row segments per row
   int64_t node_off;    // first field value of the chunk
   int64_t group_off;   // first marching-cubes group of the chunk
-  int64_t item_off[2]; // first field item of the pairs, of the bands: a chunk has one kind
+  int64_t item_off[kLists];  // first field item of each list: a chunk has one kind
 };
 
 // chunk holding marching-cubes group r
@@ -49,9 +56,7 @@ __device__ __forceinline__ int find_chunk(const BChunk* __restrict__ ch, int n, 
   return lo;
 }
 
-// Rows of an item of either list, and its item's rows of a grid.
-constexpr int kItemRows[2] = {2, kBandRows};
-
+// Items of a list over the rows of a grid.
 __host__ __device__ __forceinline__ int item_rows(const DGrid& g, int list) {
   return (g.n[1] + kItemRows[list] - 1) / kItemRows[list];
 }
@@ -100,12 +105,10 @@ __device__ __forceinline__ void batch_field_pair(const RowCtx& ctx, const BChunk
   }
 }
 
-// A band (upf_device_band.hpp): the same of kBandRows rows from row j on, as
-// k_eval_grid_band's waves.
-template <bool COMPOSED, bool WIDE>
+// A band (upf_device_band.hpp): the same of R rows from row j on, as k_eval_grid_band's waves.
+template <int R, bool COMPOSED, bool WIDE>
 __device__ __forceinline__ void batch_field_band(const RowCtx& ctx, const BChunk& C, int xb, int j, int k,
                                                  float* __restrict__ field, uint64_t* __restrict__ S) {
-  constexpr int R = kBandRows;
   const int lane = threadIdx.x & 63;
   const int rows = min(R, C.grid.n[1] - j);
   const int ic = min(xb * 64 + lane, C.grid.n[0] - 1);
@@ -170,7 +173,7 @@ __device__ __forceinline__ BItem batch_item(const BChunk* __restrict__ ch, int n
 // of items ran the row form at 1.06-1.08 ms on the 17 192^3 chunks of the 64-chunk batch
 // against 0.83 ms for the single-grid kernel over the same chunks one by one (20 B per
 // lane spilled in the loop).  Seven waves per SIMD as the single-grid row kernel, six for
-// the per-lane elevation modes and further shapes.  The per-lane form also takes the list
+// the per-lane elevation modes and further shapes.  The per-lane form also takes the lists
 // of bands, a row pair of each band per plane of workgroups.
 template <int VARIANT, bool EXT, bool COMPOSED, int LIST>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 7))) void k_batch_field_pairs(
@@ -191,12 +194,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EXT ? 6 : 7
   batch_field_pair<VARIANT, EXT, COMPOSED>(ctx, ch[it.c], it.xb, j, it.k, field, S);
 }
 
-// The list of bands.  64-chunk batch (32^3 to 192^3, 152 M nodes) as a whole, row pairs
+// The lists of bands.  64-chunk batch (32^3 to 192^3, 152 M nodes) as a whole, row pairs
 // against bands: 1.33 / 0.84 ms.
-template <bool COMPOSED, bool WIDE>
+template <int LIST, bool COMPOSED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_batch_field_bands(
     const BChunk* __restrict__ ch, int n_chunks, const uint64_t* __restrict__ blk_start, int64_t n_items,
     float* __restrict__ field, uint64_t* __restrict__ S) {
+  constexpr int R = kItemRows[LIST];
   __shared__ float4 s_slice[4][kRowSlice];
   __shared__ float4 s_gtab[16];
   if (threadIdx.x < 16) s_gtab[threadIdx.x] = gradient_entry(threadIdx.x);
@@ -204,9 +208,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k
   const int wave = uniform(threadIdx.x >> 6);
   const int64_t r = (int64_t)blockIdx.x * 4 + wave;
   if (r >= n_items) return;  // whole waves
-  const BItem it = batch_item<1>(ch, n_chunks, blk_start[blockIdx.x], r, wave);
+  const BItem it = batch_item<LIST>(ch, n_chunks, blk_start[blockIdx.x], r, wave);
   const RowCtx ctx = make_row_ctx(s_slice[wave], s_gtab, nullptr, threadIdx.x & 63);
-  batch_field_band<COMPOSED, WIDE>(ctx, ch[it.c], it.xb, kBandRows * it.row, it.k, field, S);
+  batch_field_band<R, COMPOSED, LIST == kWideList>(ctx, ch[it.c], it.xb, R * it.row, it.k, field, S);
 }
 
 // Counts of every group of every chunk (global id g: chunk, then its local group) from
@@ -290,17 +294,16 @@ size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
 struct upf_batch {
   std::vector<upf::BChunk> host;
   upf::BChunk* dev = nullptr;
-  // first field item of each workgroup of 4, of the pairs, then of the bands: chunk | xb << 16 | row << 32 | k << 48
+  // first field item of each workgroup of 4, list after list: chunk | xb << 16 | row << 32 | k << 48
   uint64_t* blk_start = nullptr;
-  int64_t item_blocks[2] = {0, 0};
+  int64_t item_blocks[upf::kLists] = {};
   int device = 0;
   int n = 0;
   int cus = 256;
   int emit_blocks = 256 * 32;  // k_batch_emit's grid
-  int64_t nodes = 0, groups = 0, items[2] = {0, 0};
+  int64_t nodes = 0, groups = 0, items[upf::kLists] = {};
   bool any_ext = false;  // a chunk with an elevation mode or a further shape: the field runs per lane
   bool any_composed = false;  // a chunk whose shape is a composition (spec_composed)
-  bool any_wide = false;  // a chunk in bands with a cellular layer past the pairs' reach (band_wide)
   upf_batch_opts opts{};
   size_t off_S = 0, off_counts = 0, off_voff = 0, off_toff = 0, off_act = 0, off_tiles = 0, off_total = 0,
          ws_bytes = 0;
@@ -331,12 +334,15 @@ int upload(upf_batch* b) {
 
 using FieldKernel = void (*)(const BChunk*, int, const uint64_t*, int64_t, float*, uint64_t*);
 
-FieldKernel field_kernel(int list, bool lanes, bool ext, bool composed, bool wide) {
-  if (ext) return k_batch_field_pairs<UPF_EVAL_PER_LANE, true, true, 0>;  // no bands then
-  if (lanes) return list ? k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, 1> : k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, 0>;
-  if (list && wide) return composed ? k_batch_field_bands<true, true> : k_batch_field_bands<false, true>;
-  if (list) return composed ? k_batch_field_bands<true, false> : k_batch_field_bands<false, false>;
-  return composed ? k_batch_field_pairs<UPF_EVAL_ROWS, false, true, 0> : k_batch_field_pairs<UPF_EVAL_ROWS, false, false, 0>;
+FieldKernel field_kernel(int list, bool lanes, bool ext, bool composed) {
+  if (ext) return k_batch_field_pairs<UPF_EVAL_PER_LANE, true, true, kPairList>;  // no bands then
+  if (lanes)
+    return list == kPairList ? k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, kPairList>
+                             : (list == kBandList ? k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, kBandList>
+                                                  : k_batch_field_pairs<UPF_EVAL_PER_LANE, false, true, kWideList>);
+  if (list == kBandList) return composed ? k_batch_field_bands<kBandList, true> : k_batch_field_bands<kBandList, false>;
+  if (list == kWideList) return composed ? k_batch_field_bands<kWideList, true> : k_batch_field_bands<kWideList, false>;
+  return composed ? k_batch_field_pairs<UPF_EVAL_ROWS, false, true, kPairList> : k_batch_field_pairs<UPF_EVAL_ROWS, false, false, kPairList>;
 }
 
 int run(upf_batch* b, float* field, void* ws, size_t ws_bytes, float* pos, float* nrm, uint32_t* idx, int64_t cap_v,
@@ -351,13 +357,13 @@ int run(upf_batch* b, float* field, void* ws, size_t ws_bytes, float* pos, float
   uint2* act = reinterpret_cast<uint2*>(w + b->off_act);
   uint4* tiles = reinterpret_cast<uint4*>(w + b->off_tiles);
   uint4* total = reinterpret_cast<uint4*>(w + b->off_total);
-  for (int list = 0; list < 2; list++) {
+  const bool lanes = b->any_ext || b->opts.field_variant == UPF_EVAL_PER_LANE;
+  const uint64_t* start = b->blk_start;
+  for (int list = 0; list < kLists; start += b->item_blocks[list++]) {
     if (!b->items[list]) continue;
-    const bool lanes = b->any_ext || b->opts.field_variant == UPF_EVAL_PER_LANE;
-    const auto kernel = field_kernel(list, lanes, b->any_ext, b->any_composed, b->any_wide);
+    const auto kernel = field_kernel(list, lanes, b->any_ext, b->any_composed);
     const dim3 blocks((unsigned)b->item_blocks[list], lanes ? kItemRows[list] / 2 : 1);
-    hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, s, b->dev, b->n, b->blk_start + (list ? b->item_blocks[0] : 0),
-                       b->items[list], field, S);
+    hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, s, b->dev, b->n, start, b->items[list], field, S);
   }
   hipLaunchKernelGGL(k_batch_classify, dim3((unsigned)((b->groups + 255) / 256)), dim3(256), 0, s, b->dev, b->n,
                      b->groups, S, counts);
@@ -410,17 +416,17 @@ int upf_batch_create(const upf_chunk* chunks, int32_t n_chunks, const upf_batch_
     b->nodes += (int64_t)C.grid.n[0] * C.grid.n[1] * C.grid.n[2];
     b->groups += C.md.groups;
   }
-  // bands for the chunks that fit them, if there are enough bands to fill the machine (and
-  // no chunk makes the whole batch run per lane)
-  // (a grid of four rows or fewer has no use for eight)
+  // bands for the chunks that fit them, if there are enough bands of eight to fill the machine
+  // (and no chunk makes the whole batch run per lane)
   const auto fits = [](const BChunk& C) { return C.grid.n[1] > kBandRows / 2 && band_fits(C.spec, C.grid); };
   int64_t bands = 0;
   for (const BChunk& C : b->host)
-    if (fits(C)) bands += band_items(C.grid);
+    if (!b->any_ext && fits(C)) bands += band_items(C.grid);
   for (BChunk& C : b->host) {
-    const int list = !b->any_ext && bands >= kBandItems && fits(C);
-    if (list && band_wide(C.spec, C.grid, kRowSlice2)) b->any_wide = true;
-    for (int l = 0; l < 2; l++) C.item_off[l] = b->items[l];
+    int list = kPairList;
+    if (bands >= kBandItems && fits(C))
+      list = band_wide(C.spec, C.grid, kRowSlice2) || band_far(C.spec, C.grid) ? kWideList : kBandList;
+    for (int l = 0; l < kLists; l++) C.item_off[l] = b->items[l];
     b->items[list] += (int64_t)C.gx * item_rows(C.grid, list) * C.grid.n[2];
   }
   if (b->groups >= ((int64_t)1 << 31)) { delete b; return UPF_ERR_BAD_GRID; }
@@ -442,18 +448,21 @@ int upf_batch_create(const upf_chunk* chunks, int32_t n_chunks, const upf_batch_
   {
     // each workgroup's first field item (chunk, segment, row, plane; all < 2^16: at most
     // 65536 chunks of at most 65535 nodes per axis), for the field kernels
-    for (int l = 0; l < 2; l++) {
+    int64_t item_blocks = 0;
+    for (int l = 0; l < kLists; l++) {
       b->item_blocks[l] = (b->items[l] + 3) / 4;
       if (b->item_blocks[l] >= ((int64_t)1 << 31)) { upf_batch_destroy(b); return UPF_ERR_BAD_GRID; }
+      item_blocks += b->item_blocks[l];
     }
-    std::vector<uint64_t> tab((size_t)(b->item_blocks[0] + b->item_blocks[1]));
-    for (int l = 0, c = 0; l < 2; l++, c = 0)
+    std::vector<uint64_t> tab;
+    tab.reserve((size_t)item_blocks);
+    for (int l = 0, c = 0; l < kLists; l++, c = 0)
       for (int64_t q = 0; q < b->item_blocks[l]; q++) {
         while (c + 1 < n_chunks && b->host[c + 1].item_off[l] <= 4 * q) c++;
         const BChunk& C = b->host[c];
         const int64_t local = 4 * q - C.item_off[l], rows = item_rows(C.grid, l);
         const uint64_t xb = (uint64_t)(local % C.gx), rest = (uint64_t)(local / C.gx);
-        tab[(size_t)(l ? b->item_blocks[0] + q : q)] = (uint64_t)c | xb << 16 | (rest % rows) << 32 | (rest / rows) << 48;
+        tab.push_back((uint64_t)c | xb << 16 | (rest % rows) << 32 | (rest / rows) << 48);
       }
     if (hipMalloc(&b->blk_start, sizeof(uint64_t) * tab.size()) != hipSuccess ||
         hipMemcpy(b->blk_start, tab.data(), sizeof(uint64_t) * tab.size(), hipMemcpyHostToDevice) != hipSuccess) {
