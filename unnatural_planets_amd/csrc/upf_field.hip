@@ -434,8 +434,30 @@ void tile_octaves(const DSpec& s, int* shared, int* other) {
   }
 }
 
+// Whether every layer is certain to be finite, and its powers: the tiles of the lakes and
+// islands modes leave out layers whose mask is 0, which an infinite one would turn into NaN.
+bool layers_finite(const DSpec& s, const DGrid& g) {
+  double reach = 0.0;
+  for (int a = 0; a < 3; a++) reach = std::max(reach, std::fabs((double)g.o[a]) + (double)g.s[a] * g.n[a]);
+  for (int l = 0; l < s.n_layers; l++) {
+    const DLayer& L = s.L[l];
+    const double noise = L.noise == UPF_NOISE_CELLULAR ? 1.0 + std::fabs((double)L.jitter) : 1.0;
+    double amps = 1.0;
+    for (int k = 0; k < (L.fractal == UPF_FRACTAL_NONE ? 1 : L.octaves); k++) {
+      if (std::fabs((double)L.freq[k]) * reach > 0x1p30) return false;
+      amps += std::fabs((double)L.amp[k]);
+    }
+    if (noise * amps > 0x1p40) return false;
+  }
+  return true;
+}
+
 void exact_launch(const DSpec& s, const DGrid& g, float* d_field, uint64_t* S, float iso, hipStream_t stream) {
   const bool hills = reads_layers(s) && (s.mode == UPF_ELEV_LAKES || s.mode == UPF_ELEV_ISLANDS);
+  if (hills && !layers_finite(s, g)) {
+    lanes_launch(s, g, d_field, S, iso, stream);
+    return;
+  }
   const bool craters = reads_layers(s) && s.mode == UPF_ELEV_CRATERS, stack = s.mode == UPF_ELEV_LAYERS;
   int shared, other;
   tile_octaves(s, &shared, &other);
