@@ -497,10 +497,10 @@ int upf_nb_extract(const upf_field_spec* spec, const upf_grid* fine, float iso, 
 /* The mesh of the last upf_nb_extract on this workspace, which returned UPF_ERR_CAPACITY
  * (the same spec, grid, iso, workspace and its stats; nothing else may have used the
  * workspace since): emitted from the blocks it evaluated, without evaluating them again.
- * Errors as upf_nb_extract's; does not synchronise. */
+ * Errors as upf_nb_extract's, and UPF_ERR_INVALID_VALUE for counts that no extraction of
+ * so many active blocks gives; does not synchronise. */
 int upf_nb_emit(const upf_field_spec* spec, const upf_grid* fine, float iso, upf_mesh_buffers* out,
                 uint64_t* d_vertex_keys, void* d_ws, size_t ws_bytes, const upf_nb_stats* stats, void* stream);
-
 
 /* ---- texel bake ---------------------------------------------------------------------
  * Replaces meshGenerateTexture(mesh, {w, h, generator = Generator::pixel})

@@ -632,6 +632,10 @@ int upf_nb_emit(const upf_field_spec* spec, const upf_grid* grid, float iso, upf
   if ((st = nb_workspace(d, d_ws, ws_bytes, &W))) return st;
   if (stats->active_blocks < 0 || stats->active_blocks > W.cap) return UPF_ERR_WORKSPACE;
   if (stats->unresolved) return UPF_ERR_BAND;
+  // counts that no extraction gives: a mesh of no blocks, or more than its blocks' edges and cells
+  if (stats->n_vertices < 0 || stats->n_vertices > 3 * kBrick * stats->active_blocks || stats->n_triangles < 0 ||
+      stats->n_triangles > UPF_MC_MAX_TRIS * kCells * stats->active_blocks)
+    return UPF_ERR_INVALID_VALUE;
   out->n_vertices = stats->n_vertices;
   out->n_triangles = stats->n_triangles;
   return nb_emit(s, g, d, W, iso, stats->active_blocks, out, d_keys, as_stream(stream));
