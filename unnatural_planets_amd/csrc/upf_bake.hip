@@ -392,20 +392,23 @@ struct DilTile {
   float* v;       // [C][kDilS * kDilS]
   uint8_t* tag;   // [kDilS * kDilS]
   uint16_t* nan;  // [kDilS * kDilS]: the loaded texels that are NaN (only they can change)
-  int* nnan;
+  int* n;         // [2]: how many; the last round that filled one
 };
 
 // Loads the tile whose loaded corner is (x0, y0) and runs the rounds on it, by a workgroup
 // of kDilThreads; false (in every thread) when nothing changed, because no loaded texel or
-// none but NaN is valid.  Rounds end early once one fills nothing.
+// none but NaN is valid.  Rounds end early once one fills nothing; a round says so in LDS
+// under its one barrier (a workgroup-wide or of a lane flag took image_dilate of 4096^2 images,
+// 30% uncovered in blocks, 259 / 287 / 321 us at 1 / 2 / 3 channels; rounds without an early
+// end 215 / 248 / 290, so 222 / 254 / 292, and 2% uncovered texels 122 / 142 / 165 and 111 / 134
+// / 154).
 template <int C>
 __device__ __forceinline__ bool dilate_tile(const DilTile T, const float* __restrict__ in, int w, int h, int x0, int y0,
                                             int rounds) {
   constexpr int N = kDilS * kDilS;
-  if (threadIdx.x == 0) *T.nnan = 0;
+  if (threadIdx.x < 2) T.n[threadIdx.x] = 0;
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  bool valid_here = false;
   for (int t0 = 0; t0 < N; t0 += kDilThreads) {  // uniform trip count: whole waves ballot
     const int t = t0 + (int)threadIdx.x;
     bool nan_here = false;
@@ -419,21 +422,21 @@ __device__ __forceinline__ bool dilate_tile(const DilTile T, const float* __rest
         for (int ch = 0; ch < C; ch++) T.v[ch * N + t] = in[o + ch];
         nan_here = isnan(T.v[t]);
         tag = nan_here ? kTagNone : 0;
-        valid_here = valid_here || !nan_here;
       }
       T.tag[t] = tag;
     }
     const uint64_t m = __ballot(nan_here);
     int base = 0;
-    if (lane == 0 && m) base = atomicAdd(T.nnan, __popcll(m));
+    if (lane == 0 && m) base = atomicAdd(T.n, __popcll(m));
     base = __shfl(base, 0, 64);
     if (nan_here) T.nan[base + __popcll(m & ((1ull << lane) - 1))] = (uint16_t)t;
   }
-  const bool any_valid = __syncthreads_or(valid_here);
-  const int nnan = *T.nnan;
-  if (!any_valid || nnan == 0) return false;
+  __syncthreads();
+  const int nnan = T.n[0];
+  const int loaded = (min(x0 + kDilS, w) - max(x0, 0)) * (min(y0 + kDilS, h) - max(y0, 0));
+  if (nnan == loaded || nnan == 0) return false;
   for (int k = 1; k <= rounds; k++) {
-    bool filled = false;
+    int filled = 0;  // a count: a flag is a lane mask, merged at each of the loop's exits
     for (int e = threadIdx.x; e < nnan; e += kDilThreads) {
       const int idx = T.nan[e];
       const int ly = idx / kDilS, lx = idx - ly * kDilS;  // constant divisor
@@ -457,10 +460,12 @@ __device__ __forceinline__ bool dilate_tile(const DilTile T, const float* __rest
 #pragma unroll
         for (int ch = 0; ch < C; ch++) T.v[ch * N + idx] = sum[ch] / (float)cnt;
         T.tag[idx] = (uint8_t)k;
-        filled = true;
+        filled++;
       }
     }
-    if (!__syncthreads_or(filled)) break;
+    if (filled) T.n[1] = k;
+    __syncthreads();
+    if (T.n[1] < k) break;  // (a faster wave may have written the next round's number)
   }
   return true;
 }
@@ -473,9 +478,9 @@ __global__ __launch_bounds__(kDilThreads) void k_dilate(const float* __restrict_
   __shared__ float s_v[C * kDilS * kDilS];
   __shared__ uint8_t s_tag[kDilS * kDilS];
   __shared__ uint16_t s_nan[kDilS * kDilS];
-  __shared__ int s_nnan;
+  __shared__ int s_n[2];
   const int x0 = (int)blockIdx.x * kDilT - kDilR, y0 = (int)blockIdx.y * kDilT - kDilR;
-  (void)dilate_tile<C>({s_v, s_tag, s_nan, &s_nnan}, in, w, h, x0, y0, rounds);
+  (void)dilate_tile<C>({s_v, s_tag, s_nan, s_n}, in, w, h, x0, y0, rounds);
   for (int t = threadIdx.x; t < kDilT * kDilT; t += kDilThreads) {
     const int ly = kDilR + t / kDilT, lx = kDilR + t % kDilT;
     const int x = x0 + lx, y = y0 + ly;
@@ -644,9 +649,9 @@ __global__ __launch_bounds__(256) void k_to_u8_x4(const float4* __restrict__ in,
 // filled: no copy of the image, no float result, no merge.  HBM-bound where most tiles
 // are covered: 24 B read and 6 B written per texel of a chunk's three images.  The U8
 // values are image_to_u8's of image_dilate's result, bit for bit.  Three images (3 + 2 + 1
-// channels), copies + dilations + merges + conversions against one pass: 4096^2 covered 500
-// and 104 us (4.8 TB/s), 30% uncovered in 8 x 8 blocks 966 and 745, three quarters covered
-// 746 and 146; 500^2 90 and 21 us.  Measured and not kept: four tiles per workgroup, all
+// channels), copies + dilations + merges + conversions against one pass: 4096^2 covered 610
+// and 104 us (4.8 TB/s), 30% uncovered in 8 x 8 blocks 1,087 and 629, half covered 1,098 and
+// 176; 500 x 375 105 and 19 us.  Measured and not kept: four tiles per workgroup, all
 // streamed before the first one's rounds (89, 880 and 204 us at 4096^2); a streaming kernel
 // and one that fills the tiles its flags name (101, 982 and 132: the second reads the tiles
 // again); leaving the tiles of nothing but NaN to a second launch (135, 768 and 163).
@@ -656,7 +661,7 @@ struct PostArgs {
 };
 
 template <int C>
-__device__ __forceinline__ void post_tile(const upf_post_image& im, int rounds, char* lds, int* nnan) {
+__device__ __forceinline__ void post_tile(const upf_post_image& im, int rounds, char* lds, int* n) {
   const float* __restrict__ in = im.d_in;
   uint8_t* __restrict__ out = im.d_out;
   const int w = im.width, h = im.height, oc = im.out_channels;
@@ -715,7 +720,7 @@ __device__ __forceinline__ void post_tile(const upf_post_image& im, int rounds, 
   float* v = reinterpret_cast<float*>(lds);
   uint16_t* list = reinterpret_cast<uint16_t*>(v + C * N);
   uint8_t* tag = reinterpret_cast<uint8_t*>(list + N);
-  if (!dilate_tile<C>({v, tag, list, nnan}, in, w, h, x0 - kDilR, y0 - kDilR, rounds)) return;
+  if (!dilate_tile<C>({v, tag, list, n}, in, w, h, x0 - kDilR, y0 - kDilR, rounds)) return;
   for (int t = threadIdx.x; t < kDilT * kDilT; t += kDilThreads) {
     const int q = (kDilR + t / kDilT) * kDilS + kDilR + t % kDilT;
     if (tag[q] == 0 || tag[q] > kDilR) continue;  // valid from the start, still NaN, or outside
@@ -727,13 +732,13 @@ __device__ __forceinline__ void post_tile(const upf_post_image& im, int rounds, 
 
 __global__ __launch_bounds__(kDilThreads) void k_images_post(const PostArgs a, int rounds) {
   extern __shared__ __attribute__((aligned(16))) char s_post[];
-  __shared__ int s_nnan;
+  __shared__ int s_n[2];
   const upf_post_image& im = a.im[blockIdx.z];
   switch (im.channels) {
-    case 1: post_tile<1>(im, rounds, s_post, &s_nnan); break;
-    case 2: post_tile<2>(im, rounds, s_post, &s_nnan); break;
-    case 3: post_tile<3>(im, rounds, s_post, &s_nnan); break;
-    default: post_tile<4>(im, rounds, s_post, &s_nnan); break;
+    case 1: post_tile<1>(im, rounds, s_post, s_n); break;
+    case 2: post_tile<2>(im, rounds, s_post, s_n); break;
+    case 3: post_tile<3>(im, rounds, s_post, s_n); break;
+    default: post_tile<4>(im, rounds, s_post, s_n); break;
   }
 }
 
