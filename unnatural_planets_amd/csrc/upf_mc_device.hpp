@@ -139,8 +139,9 @@ __device__ __forceinline__ uint4 tile_sum(uint4 v) {
 // ------------------------------------------------------------------ classify
 // One workgroup classifies a scan tile of kScanTile groups, a group per thread.  With 256
 // threads of eight groups each (the next group's words loaded ahead) the chip was idle at
-// all but the largest grids and the kernel no faster there: marching cubes of a stored
-// field took 51 us at 48^3, 74 at 110^3, 91 at 256^3 and 197 at 512^3; 25, 38, 69 and 193 so.
+// all but the largest grids and the kernel hardly faster there: marching cubes of a stored
+// field took 51 us at 48^3, 74 at 110^3, 91 at 256^3, 115 at 384^3, 191 at 512^3 and 538 at
+// 700^3; 25, 38, 69, 105, 195 and 541 so.
 // (The batched kernel keeps 256 threads and a separate tile pass: its workgroups' 1024 groups
 // would cross chunks, and it measured 0.6% slower per batch.)
 // Packed counts of a group from the sign words alone (written by the field kernel or
